@@ -6,7 +6,7 @@
 // browind[k] of C.  Each C element is the sum of its products in that scan
 // order; in the sparse result the columns of a row appear in the order of
 // their first product.  A row's products are numbered t = 0, 1, ... in that
-// scan order.  Rows take one of two paths:
+// scan order.  Rows take one of three paths:
 //
 // Short rows (at most 64 products from at most 64 entries of A): one
 // wavefront per row, lane t holding product t.  The lanes enter their
@@ -16,6 +16,11 @@
 // the mask, added in lane (= t) order.  The heads in lane order are the
 // columns in first-appearance order (a ballot gives each head its rank).
 //
+// Medium rows (at most 4096 distinct columns, by the lesser of the row's
+// products and C's columns): one wavefront per row again, 64 products a step
+// in t order, the columns found so far in an LDS hash table with each
+// column's rank (the order of its first product) and running sum.
+//
 // Other rows: every product is materialised at its position t (numbered
 // over these rows, row-major), then
 //   1. stable radix sort of t by column, then by row: (row, col, t) order
@@ -23,21 +28,36 @@
 //   3. the runs sorted by their first t (unique, row-major), so each row
 //      lists its columns by first appearance.
 //
-// Both paths add a column's products one after another in t order: the
+// All paths add a column's products one after another in t order: the
 // first product, then += the others (the dense variant starts from +0.0 as
 // the reference's zeroed row does, so a lone -0.0 becomes +0.0).  The sparse
 // result needs each row's entry count before the rows can be placed: the
-// short rows write their entries in first-appearance order to a staging
-// area at the row's first product position, with their counts; the scan of
-// the counts gives the row pointers and a copy puts the staged rows in
-// place.  (When the staging area would pass its limit, 8 GiB unless
-// GOOSEBERRY_SPGEMM_STAGE_MAX says otherwise, the short rows are counted in
+// short and medium rows write their entries in first-appearance order to a
+// staging area at the row's first product position, with their counts; the
+// scan of the counts gives the row pointers and a copy puts the staged rows
+// in place.  (When the staging area would pass its limit, 8 GiB unless
+// GOOSEBERRY_SPGEMM_STAGE_MAX says otherwise, these rows are counted in
 // one pass and written in another instead.)
 #include <stdlib.h>
 
 #include "gb_common.h"
 
-#define GB_SG_SHORT 64  // products (and A entries) of a wavefront row
+#define GB_SG_SHORT 64  // products (and A entries) of a short row
+
+// Row classes: short rows, six classes of medium rows by the distinct
+// columns their hash table must hold, and the rows of the sort path.  On
+// random matrices of 29 entries a row (841 products, 60,000 rows) three
+// classes (256, 1024, 4096) took 1.20 ms, these six 0.88 ms: a row in the
+// smallest table that fits leaves LDS for more wavefronts.
+#define GB_SG_NHASH 6
+enum { GB_SG_CSHORT = 0, GB_SG_CHASH = 1, GB_SG_CSORT = GB_SG_CHASH + GB_SG_NHASH,
+       GB_SG_NCLASS };
+constexpr uint32_t gb_sg_cap[GB_SG_NHASH] = {256, 512, 1024, 1536, 2560, 4096};
+constexpr uint32_t gb_sg_slots(uint32_t cap) { return cap * 3 / 2; }
+// products and A entries of a medium row at most: one wavefront walks them
+// alone, 64 in about half a microsecond, so a longer row would hold up the
+// launch for more than half a millisecond
+#define GB_SG_HASH_MAXP 65536u
 
 enum { GB_SG_COUNT = 0, GB_SG_FILL = 1, GB_SG_DENSE = 2, GB_SG_STAGE = 3 };
 #define GB_SG_STAGE_MAX (8ull << 30)  // bytes of staged short-row entries
@@ -54,50 +74,61 @@ static uint64_t gb_sg_stage_max() {
   return GB_SG_STAGE_MAX;
 }
 
-// products per A entry: the length of the B row it selects
+// products per A entry (the length of the B row it selects) and their total
 __global__ void __launch_bounds__(GB_BLOCK)
 gb_sg_len(uint64_t annz, const uint32_t *__restrict__ arowind,
-          const uint32_t *__restrict__ browptr, uint32_t *__restrict__ len) {
+          const uint32_t *__restrict__ browptr, uint32_t *__restrict__ len,
+          unsigned long long *__restrict__ total) {
+  __shared__ unsigned long long lds[GB_WAVES_PER_BLOCK];
+  unsigned long long v = 0;
+#pragma unroll 4
   for (uint64_t j = (uint64_t)blockIdx.x * GB_BLOCK + threadIdx.x; j < annz;
        j += (uint64_t)gridDim.x * GB_BLOCK) {
     const uint32_t l = arowind[j];
-    len[j] = browptr[l + 1] - browptr[l];
+    const uint32_t n = browptr[l + 1] - browptr[l];
+    len[j] = n;
+    v += n;
   }
-}
-
-__global__ void __launch_bounds__(GB_BLOCK)
-gb_sg_sum64(const uint32_t *__restrict__ a, uint64_t n, unsigned long long *__restrict__ total) {
-  __shared__ unsigned long long lds[GB_WAVES_PER_BLOCK];
-  unsigned long long v = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * GB_BLOCK + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * GB_BLOCK)
-    v += a[i];
   v = gb_block_sum(v, lds);
   if (threadIdx.x == 0) atomicAdd(total, v);
 }
 
-// row classes: isshort[i] = 1 for a wavefront row, islong[i] = 1 for a row
-// of the sort path (off = exclusive scan of the products per A entry)
+// the class of every row and the rows in each class (off = exclusive scan
+// of the products per A entry)
 __global__ void __launch_bounds__(GB_BLOCK)
-gb_sg_classify(uint32_t anrows, const uint32_t *__restrict__ arowptr,
-               const uint32_t *__restrict__ off, uint32_t *__restrict__ isshort,
-               uint32_t *__restrict__ islong) {
+gb_sg_classify(uint32_t anrows, uint32_t bncols, const uint32_t *__restrict__ arowptr,
+               const uint32_t *__restrict__ off, uint32_t *__restrict__ cls,
+               uint32_t *__restrict__ count) {
+  __shared__ uint32_t h[GB_SG_NCLASS];
+  if (threadIdx.x < GB_SG_NCLASS) h[threadIdx.x] = 0;
+  __syncthreads();
   for (uint32_t i = blockIdx.x * GB_BLOCK + threadIdx.x; i < anrows;
        i += gridDim.x * GB_BLOCK) {
-    const uint32_t j0 = arowptr[i], j1 = arowptr[i + 1];
+    const uint32_t j0 = arowptr[i], j1 = arowptr[i + 1], m = j1 - j0;
     const uint32_t p = off[j1] - off[j0];
-    const bool s = p <= GB_SG_SHORT && j1 - j0 <= GB_SG_SHORT;
-    isshort[i] = s ? 1u : 0u;
-    islong[i] = s ? 0u : 1u;
+    const uint32_t d = p < bncols ? p : bncols;  // distinct columns at most
+    uint32_t c;
+    if (p <= GB_SG_SHORT && m <= GB_SG_SHORT) c = GB_SG_CSHORT;
+    else if (p > GB_SG_HASH_MAXP || m > GB_SG_HASH_MAXP) c = GB_SG_CSORT;
+    else {
+      c = GB_SG_CSORT;
+#pragma unroll
+      for (int k = GB_SG_NHASH - 1; k >= 0; --k)
+        if (d <= gb_sg_cap[k]) c = GB_SG_CHASH + k;
+    }
+    cls[i] = c;
+    // one count per class and wavefront: by the lanes' masks
+    for (uint64_t todo = __ballot(true); todo;) {
+      const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)c, __builtin_ctzll(todo));
+      const uint64_t same = __ballot(c == k);
+      if ((threadIdx.x & (GB_WAVE - 1)) == (uint32_t)__builtin_ctzll(same))
+        atomicAdd(&h[k], (uint32_t)__popcll(same));
+      todo &= ~same;
+    }
   }
-}
-
-// list[pos[i]] = i for flagged rows (pos = exclusive scan of the flags)
-__global__ void __launch_bounds__(GB_BLOCK)
-gb_sg_compact(uint32_t n, const uint32_t *__restrict__ flag, const uint32_t *__restrict__ pos,
-              uint32_t *__restrict__ list) {
-  for (uint32_t i = blockIdx.x * GB_BLOCK + threadIdx.x; i < n; i += gridDim.x * GB_BLOCK)
-    if (flag[i]) list[pos[i]] = i;
+  __syncthreads();
+  if (threadIdx.x < GB_SG_NCLASS && h[threadIdx.x])
+    atomicAdd(&count[threadIdx.x], h[threadIdx.x]);
 }
 
 #define GB_SG_HASH_BITS 7
@@ -130,7 +161,7 @@ gb_sg_wave(uint32_t nlist, const uint32_t *__restrict__ list,
   const uint32_t lane = threadIdx.x & (GB_WAVE - 1);
   if (w >= nlist) return;  // the whole wavefront
   // one row per wavefront: its scalars live in scalar registers
-  const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)list[w]);
+  const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)(list ? list[w] : w));
   const uint32_t j0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)arowptr[i]);
   const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)arowptr[i + 1]) - j0;
   // lane a < m: A entry j0 + a and the B row it selects
@@ -218,6 +249,181 @@ gb_sg_wave(uint32_t nlist, const uint32_t *__restrict__ list,
   }
 }
 
+// One wavefront (and workgroup) per medium row of at most CAP distinct
+// columns.  A entries are taken 64 at a time: a scan of their B rows' lengths
+// numbers the products, and 64 consecutive products at a time are formed,
+// one per lane, the next 64 loaded while these are added.  A lane finds its
+// column's slot in the hash table (linear probing, compare-and-swap); new
+// columns take ranks in lane order.  When every lane holds a column of its
+// own (each lane writes its number into its slot and reads it back), one
+// read, add and write of the sums does; otherwise the lowest lane of each
+// shared column adds the others' products in lane order.  LDS operations of
+// a wavefront complete in order, so the steps' additions to a column keep
+// t order.
+//
+// Bound: a chain of about a dozen dependent LDS operations per 64 products;
+// the table's size decides how many wavefronts a CU holds to overlap them,
+// hence the classes and the load of two thirds.  The sort path, which took
+// these rows before, moves each product through global memory about 20 times:
+// a product of random matrices of 29 entries a row (60,000 rows, 50 million
+// products) and its first SpMV took 10.6 ms, and take 2.04 ms.
+template <uint32_t CAP, uint32_t SLOTS, int MODE>
+__global__ void __launch_bounds__(GB_WAVE)
+gb_sg_hash(const uint32_t *__restrict__ list, const uint32_t *__restrict__ arowptr,
+           const uint32_t *__restrict__ arowind, const double *__restrict__ arowval,
+           const uint32_t *__restrict__ browptr, const uint32_t *__restrict__ browind,
+           const double *__restrict__ browval, const uint32_t *__restrict__ crowptr,
+           uint32_t *__restrict__ cnt, uint32_t *__restrict__ crowind,
+           double *__restrict__ crowval, double *__restrict__ cdense, uint32_t bncols,
+           const uint32_t *__restrict__ pbase) {
+  static_assert(CAP <= 65536 && SLOTS > CAP, "16-bit ranks, and a free slot always");
+  __shared__ uint32_t key[SLOTS];
+  __shared__ double sum[MODE == GB_SG_COUNT ? 1 : CAP];
+  __shared__ double bx[GB_WAVE];      // A entry: its value
+  __shared__ uint32_t boff[GB_WAVE];  // A entry: B position of product t, less t
+  __shared__ uint32_t mark[GB_WAVE];
+  __shared__ uint16_t rnk[SLOTS];
+  __shared__ uint8_t tag[SLOTS];
+  const uint32_t lane = threadIdx.x;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const uint32_t i =
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)(list ? list[blockIdx.x] : blockIdx.x));
+  const uint32_t j0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)arowptr[i]);
+  const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)arowptr[i + 1]) - j0;
+  uint32_t o = 0;  // the row's place in crowind and crowval
+  if (MODE == GB_SG_FILL) o = (uint32_t)__builtin_amdgcn_readfirstlane((int)crowptr[i]);
+  if (MODE == GB_SG_STAGE) o = (uint32_t)__builtin_amdgcn_readfirstlane((int)pbase[j0]);
+  for (uint32_t q = lane; q < SLOTS; q += GB_WAVE) key[q] = GB_SG_EMPTY;
+  uint32_t ndist = 0;
+  for (uint32_t jb = 0; jb < m; jb += GB_WAVE) {
+    uint32_t bstart = 0, blen = 0;
+    double x = 0.0;
+    if (jb + lane < m) {
+      const uint32_t l = arowind[j0 + jb + lane];
+      x = arowval[j0 + jb + lane];
+      bstart = browptr[l];
+      blen = browptr[l + 1] - bstart;
+    }
+    const uint32_t incl = gb_wave_scan_incl(blen);
+    const uint32_t excl = incl - blen;
+    const uint32_t P = (uint32_t)__builtin_amdgcn_readlane((int)incl, GB_WAVE - 1);
+    gb_sg_wave_sync();
+    boff[lane] = bstart - excl;
+    bx[lane] = x;
+    uint32_t acarry = 0;  // the A entry of the product before this step's first
+    // the column and factors of product t = c0 + lane (loads only)
+    auto fetch = [&](uint32_t c0, uint32_t &col, double &xa, double &bv) {
+      gb_sg_wave_sync();
+      mark[lane] = GB_SG_EMPTY;
+      gb_sg_wave_sync();
+      if (blen && excl - c0 < GB_WAVE) mark[excl - c0] = lane;
+      gb_sg_wave_sync();
+      const uint32_t mk = mark[lane];
+      const unsigned long long at = __ballot(mk != GB_SG_EMPTY) & (below | (1ull << lane));
+      const uint32_t from = (uint32_t)__shfl((int)mk, at ? 63 - __clzll(at) : 0, GB_WAVE);
+      const uint32_t a = at ? from : acarry;
+      acarry = (uint32_t)__builtin_amdgcn_readlane((int)a, GB_WAVE - 1);
+      col = 0;
+      xa = bv = 0.0;
+      if (c0 + lane < P) {
+        const uint32_t k = boff[a] + c0 + lane;
+        col = browind[k];
+        if (MODE != GB_SG_COUNT) {
+          bv = browval[k];
+          xa = bx[a];
+        }
+      }
+    };
+    uint32_t col = 0, ncol = 0;
+    double xa = 0.0, bv = 0.0, nxa = 0.0, nbv = 0.0;
+    if (P) fetch(0, ncol, nxa, nbv);
+    for (uint32_t c0 = 0; c0 < P; c0 += GB_WAVE) {
+      col = ncol;
+      xa = nxa;
+      bv = nbv;
+      if (c0 + GB_WAVE < P) fetch(c0 + GB_WAVE, ncol, nxa, nbv);
+      const bool live = c0 + lane < P;
+      const double val = xa * bv;
+      uint32_t slot = 0;
+      bool won = false;
+      if (live) {
+        uint32_t h = __umulhi(col * 2654435761u, SLOTS);
+        for (;;) {  // at most CAP < SLOTS columns: a free or equal slot exists
+          const uint32_t prev = atomicCAS(&key[h], GB_SG_EMPTY, col);
+          won = prev == GB_SG_EMPTY;
+          if (won || prev == col) break;
+          if (++h == SLOTS) h = 0;
+        }
+        slot = h;
+        tag[slot] = (uint8_t)lane;
+      }
+      gb_sg_wave_sync();
+      const unsigned long long dup = __ballot(live && tag[slot] != lane);
+      unsigned long long newm = __ballot(won);    // lanes whose column is new
+      unsigned long long lead = __ballot(live);   // lanes that write their column's sum
+      for (unsigned long long todo = dup; todo;) {
+        const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)slot, __ffsll(todo) - 1);
+        const unsigned long long grp = __ballot(live && slot == s);
+        const unsigned long long first = grp & (0ull - grp);
+        if (newm & grp) newm = (newm & ~grp) | first;
+        lead = (lead & ~grp) | first;
+        todo &= ~grp;
+      }
+      const bool isnew = (newm >> lane) & 1ull, leads = (lead >> lane) & 1ull;
+      uint32_t r = 0;
+      if (isnew) {
+        r = ndist + (uint32_t)__popcll(newm & below);
+        rnk[slot] = (uint16_t)r;
+        if (MODE == GB_SG_FILL || MODE == GB_SG_STAGE) crowind[o + r] = col;
+      } else if (leads) {
+        r = rnk[slot];
+      }
+      ndist += (uint32_t)__popcll(newm);
+      if (MODE != GB_SG_COUNT) {
+        double acc = 0.0;
+        if (isnew) acc = MODE == GB_SG_DENSE ? 0.0 + val : val;
+        else if (leads) acc = sum[r] + val;
+        for (unsigned long long todo = dup; todo;) {
+          const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)slot, __ffsll(todo) - 1);
+          const unsigned long long grp = __ballot(live && slot == s);
+          const uint32_t first = (uint32_t)__ffsll(grp) - 1;
+          for (unsigned long long rest = grp & (grp - 1ull); rest; rest &= rest - 1ull) {
+            const double v = gb_readlane(val, (uint32_t)__ffsll(rest) - 1);
+            if (lane == first) acc += v;
+          }
+          todo &= ~grp;
+        }
+        if (leads) sum[r] = acc;
+      }
+      gb_sg_wave_sync();
+    }
+  }
+  gb_sg_wave_sync();
+  if ((MODE == GB_SG_COUNT || MODE == GB_SG_STAGE) && lane == 0) cnt[i] = ndist;
+  if (MODE == GB_SG_FILL || MODE == GB_SG_STAGE)
+    for (uint32_t q = lane; q < ndist; q += GB_WAVE) crowval[o + q] = sum[q];
+  if (MODE == GB_SG_DENSE)
+    for (uint32_t q = lane; q < SLOTS; q += GB_WAVE)
+      if (key[q] != GB_SG_EMPTY) cdense[(size_t)i * bncols + key[q]] = sum[rnk[q]];
+}
+
+// the staged medium rows to their places, one wavefront per row
+__global__ void __launch_bounds__(GB_BLOCK)
+gb_sg_unstage_wave(uint32_t nlist, const uint32_t *__restrict__ list,
+                   const uint32_t *__restrict__ arowptr, const uint32_t *__restrict__ pbase,
+                   const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ sind,
+                   const double *__restrict__ sval, const uint32_t *__restrict__ crowptr,
+                   uint32_t *__restrict__ crowind, double *__restrict__ crowval) {
+  const uint32_t w = blockIdx.x * GB_WAVES_PER_BLOCK + threadIdx.x / GB_WAVE;
+  if (w >= nlist) return;
+  const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)(list ? list[w] : w));
+  const uint32_t c = cnt[i], src = pbase[arowptr[i]], dst = crowptr[i];
+  for (uint32_t q = threadIdx.x & (GB_WAVE - 1); q < c; q += GB_WAVE) {
+    crowind[dst + q] = sind[src + q];
+    crowval[dst + q] = sval[src + q];
+  }
+}
+
 // the staged short rows to their places, GB_BLOCK list rows per workgroup:
 // row i's cnt[i] entries from its staging slots (pbase[arowptr[i]] on) to
 // crowptr[i] on.  The workgroup numbers its rows' entries k = 0, 1, ...
@@ -236,7 +442,7 @@ gb_sg_unstage(uint32_t nlist, const uint32_t *__restrict__ list,
   const uint32_t w = blockIdx.x * GB_BLOCK + threadIdx.x;
   uint32_t c = 0;
   if (w < nlist) {
-    const uint32_t i = list[w];
+    const uint32_t i = list ? list[w] : w;
     c = cnt[i];
     src[threadIdx.x] = pbase[arowptr[i]];
     dst[threadIdx.x] = crowptr[i];
@@ -272,15 +478,15 @@ __device__ __forceinline__ uint32_t gb_sg_row_of(const uint32_t *arowptr, uint32
   return lo;
 }
 
-// products per A entry of the sort path's rows (0 for short rows)
+// products per A entry of the sort path's rows (0 for other rows)
 __global__ void __launch_bounds__(GB_BLOCK)
 gb_sg_len_long(uint32_t anrows, uint64_t annz, const uint32_t *__restrict__ arowptr,
-               const uint32_t *__restrict__ islong, const uint32_t *__restrict__ len,
+               const uint32_t *__restrict__ cls, const uint32_t *__restrict__ len,
                uint32_t *__restrict__ len2) {
   for (uint64_t j = (uint64_t)blockIdx.x * GB_BLOCK + threadIdx.x; j < annz;
        j += (uint64_t)gridDim.x * GB_BLOCK) {
     const uint32_t i = gb_sg_row_of(arowptr, anrows, (uint32_t)j);
-    len2[j] = islong[i] ? len[j] : 0u;
+    len2[j] = cls[i] == GB_SG_CSORT ? len[j] : 0u;
   }
 }
 
@@ -417,6 +623,38 @@ static uint32_t gb_sg_grid(uint64_t n) {
   return g ? (uint32_t)g : 1u;
 }
 
+// the medium rows of one class in one mode (dense and the staged or final
+// arrays as the short rows' kernel takes them)
+template <int MODE>
+static hipError_t gb_sg_medium(const uint32_t *count, const uint32_t *list,
+                               const uint32_t *arowptr, const uint32_t *arowind,
+                               const double *arowval, const uint32_t *browptr,
+                               const uint32_t *browind, const double *browval,
+                               const uint32_t *crowptr, uint32_t *cnt, uint32_t *crowind,
+                               double *crowval, double *cdense, uint32_t bncols,
+                               const uint32_t *pbase) {
+  uint32_t first = count[GB_SG_CSHORT];
+  for (int c = 0; c < GB_SG_NHASH; ++c) {
+    const uint32_t n = count[GB_SG_CHASH + c];
+    if (!n) continue;
+    auto *k = gb_sg_hash<gb_sg_cap[0], gb_sg_slots(gb_sg_cap[0]), MODE>;
+    switch (c) {
+      case 1: k = gb_sg_hash<gb_sg_cap[1], gb_sg_slots(gb_sg_cap[1]), MODE>; break;
+      case 2: k = gb_sg_hash<gb_sg_cap[2], gb_sg_slots(gb_sg_cap[2]), MODE>; break;
+      case 3: k = gb_sg_hash<gb_sg_cap[3], gb_sg_slots(gb_sg_cap[3]), MODE>; break;
+      case 4: k = gb_sg_hash<gb_sg_cap[4], gb_sg_slots(gb_sg_cap[4]), MODE>; break;
+      case 5: k = gb_sg_hash<gb_sg_cap[5], gb_sg_slots(gb_sg_cap[5]), MODE>; break;
+    }
+    k<<<n, GB_WAVE, 0, gb_stream()>>>(list ? list + first : nullptr, arowptr, arowind, arowval,
+                                      browptr, browind, browval, crowptr, cnt, crowind,
+                                      crowval, cdense, bncols, pbase);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    first += n;
+  }
+  return hipSuccess;
+}
+
 extern "C" {
 
 int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
@@ -431,16 +669,17 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
   if (!dense && (!d_crowptr || !d_crowind || !d_crowval || !r_cnnz))
     return GOOSEBERRY_ERROR_INVALIDINPUT;
   hipStream_t s = gb_stream();
-  uint32_t annz = 0, E = 0, nruns = 0, nshort = 0, nlong = 0, cnnz = 0;
-  uint32_t *len = nullptr, *off = nullptr, *isshort = nullptr, *islong = nullptr,
-           *slist = nullptr, *len2 = nullptr, *off2 = nullptr, *erow = nullptr,
+  uint32_t annz = 0, E = 0, nruns = 0, nshort = 0, nmed = 0, nlong = 0, cnnz = 0;
+  uint32_t hcount[GB_SG_NCLASS] = {0};
+  uint32_t *len = nullptr, *off = nullptr, *cls = nullptr, *count = nullptr,
+           *list = nullptr, *mlist = nullptr, *len2 = nullptr, *off2 = nullptr, *erow = nullptr,
            *ecol = nullptr, *perm1 = nullptr, *row1 = nullptr, *ord = nullptr,
            *flag = nullptr, *rid = nullptr, *runstart = nullptr, *rrow = nullptr,
            *rcol = nullptr, *rfirst = nullptr, *ordr = nullptr, *rbeg = nullptr,
            *cnt = nullptr, *crowptr = nullptr, *crowind = nullptr, *sind = nullptr;
   double *eval = nullptr, *rval = nullptr, *crowval = nullptr, *sval = nullptr;
   unsigned long long e64 = 0, *tot = nullptr;
-  bool staged = false;
+  bool staged = false, one_class = false;
   hipError_t he = hipSuccess;
 #define GB_SG_TRY(call)                                         \
   do {                                                          \
@@ -466,16 +705,12 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
   GB_SG_TRY(hipStreamSynchronize(s));
   GB_SG_TRY(gb_dev_alloc((void **)&len, ((size_t)annz + 1) * 4));
   GB_SG_TRY(gb_dev_alloc((void **)&off, ((size_t)annz + 1) * 4));
-  if (annz) {
-    gb_sg_len<<<gb_sg_grid(annz), GB_BLOCK, 0, s>>>(annz, d_arowind, d_browptr, len);
-    GB_SG_TRY(hipGetLastError());
-  }
   // every product position must fit 32 bits: the total in 64 bits first
   GB_SG_TRY(gb_dev_alloc((void **)&tot, 8));
   GB_SG_RV(gbd_zero(tot, 8));
   if (annz) {
-    gb_sg_sum64<<<gb_sg_grid(annz) > 1024u ? 1024u : gb_sg_grid(annz), GB_BLOCK, 0, s>>>(
-        len, annz, tot);
+    const uint32_t g = gb_sg_grid(annz);
+    gb_sg_len<<<g > 1024u ? 1024u : g, GB_BLOCK, 0, s>>>(annz, d_arowind, d_browptr, len, tot);
     GB_SG_TRY(hipGetLastError());
   }
   GB_SG_TRY(hipMemcpyAsync(&e64, tot, 8, hipMemcpyDeviceToHost, s));
@@ -485,52 +720,73 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
     goto done;
   }
   GB_SG_RV(gbd_scan_u32(len, off, annz, off + annz));
-  // row classes and the list of wavefront rows
-  GB_SG_TRY(gb_dev_alloc((void **)&isshort, ((size_t)anrows + 1) * 4));
-  GB_SG_TRY(gb_dev_alloc((void **)&islong, ((size_t)anrows + 1) * 4));
-  GB_SG_TRY(gb_dev_alloc((void **)&slist, ((size_t)anrows + 1) * 4));
+  // row classes, and the rows in class order unless they are all of one
+  GB_SG_TRY(gb_dev_alloc((void **)&cls, ((size_t)anrows + 1) * 4));
+  GB_SG_TRY(gb_dev_alloc((void **)&count, GB_SG_NCLASS * 4));
   GB_SG_TRY(gb_dev_alloc((void **)&cnt, ((size_t)anrows + 1) * 4));
+  GB_SG_RV(gbd_zero(count, GB_SG_NCLASS * 4));
   if (anrows) {
-    gb_sg_classify<<<gb_sg_grid(anrows), GB_BLOCK, 0, s>>>(anrows, d_arowptr, off, isshort,
-                                                          islong);
+    // few workgroups: each adds its counts to the same words (2,848 of them
+    // took 37 us for 729,000 rows)
+    const uint32_t g = gb_sg_grid(anrows);
+    gb_sg_classify<<<g > 512u ? 512u : g, GB_BLOCK, 0, s>>>(anrows, bncols, d_arowptr, off,
+                                                            cls, count);
     GB_SG_TRY(hipGetLastError());
   }
-  // cnt holds the list positions until the counts replace them
-  GB_SG_RV(gbd_scan_u32(isshort, cnt, anrows, cnt + anrows));
-  GB_SG_TRY(hipMemcpyAsync(&nshort, cnt + anrows, 4, hipMemcpyDeviceToHost, s));
+  GB_SG_TRY(hipMemcpyAsync(hcount, count, GB_SG_NCLASS * 4, hipMemcpyDeviceToHost, s));
   GB_SG_TRY(hipStreamSynchronize(s));
-  nlong = anrows - nshort;
-  if (nshort) {
-    gb_sg_compact<<<gb_sg_grid(anrows), GB_BLOCK, 0, s>>>(anrows, isshort, cnt, slist);
-    GB_SG_TRY(hipGetLastError());
+  nshort = hcount[GB_SG_CSHORT];
+  nlong = hcount[GB_SG_CSORT];
+  nmed = anrows - nshort - nlong;
+  for (int c = 0; c < GB_SG_NCLASS; ++c) one_class |= hcount[c] == anrows;
+  if (!one_class) {
+    GB_SG_TRY(gb_dev_alloc((void **)&list, (size_t)anrows * 4));
+    GB_SG_RV(gbd_countingsort_kv_unchecked(cls, nullptr, 0, GB_SG_NCLASS - 1, anrows, list,
+                                           nullptr));
   }
   if (!dense) {
-    GB_SG_RV(gbd_zero(cnt, ((size_t)anrows + 1) * 4));
+    if (nlong) GB_SG_RV(gbd_zero(cnt, ((size_t)anrows + 1) * 4));
     staged = e64 * 12 <= gb_sg_stage_max();
-    if (nshort && staged) {
+    if ((nshort || nmed) && staged) {
       GB_SG_TRY(gb_dev_alloc((void **)&sind, (size_t)e64 * 4));
       GB_SG_TRY(gb_dev_alloc((void **)&sval, (size_t)e64 * 8));
+    }
+    if (nshort && staged) {
       gb_sg_wave<GB_SG_STAGE><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, slist, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
+          nshort, list, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
           nullptr, cnt, sind, sval, nullptr, 0, off);
       GB_SG_TRY(hipGetLastError());
     } else if (nshort) {
       gb_sg_wave<GB_SG_COUNT><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, slist, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
+          nshort, list, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
           nullptr, cnt, nullptr, nullptr, nullptr, 0, nullptr);
       GB_SG_TRY(hipGetLastError());
     }
-  } else if (nshort) {
-    gb_sg_wave<GB_SG_DENSE><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
-        nshort, slist, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
-        nullptr, nullptr, nullptr, nullptr, d_cdense, bncols, nullptr);
-    GB_SG_TRY(hipGetLastError());
+    if (nmed && staged)
+      GB_SG_TRY(gb_sg_medium<GB_SG_STAGE>(hcount, list, d_arowptr, d_arowind, d_arowval,
+                                          d_browptr, d_browind, d_browval, nullptr, cnt, sind,
+                                          sval, nullptr, 0, off));
+    else if (nmed)
+      GB_SG_TRY(gb_sg_medium<GB_SG_COUNT>(hcount, list, d_arowptr, d_arowind, d_arowval,
+                                          d_browptr, d_browind, d_browval, nullptr, cnt,
+                                          nullptr, nullptr, nullptr, 0, nullptr));
+  } else {
+    if (nshort) {
+      gb_sg_wave<GB_SG_DENSE><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
+          nshort, list, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
+          nullptr, nullptr, nullptr, nullptr, d_cdense, bncols, nullptr);
+      GB_SG_TRY(hipGetLastError());
+    }
+    if (nmed)
+      GB_SG_TRY(gb_sg_medium<GB_SG_DENSE>(hcount, list, d_arowptr, d_arowind, d_arowval,
+                                          d_browptr, d_browind, d_browval, nullptr, nullptr,
+                                          nullptr, nullptr, d_cdense, bncols, nullptr));
   }
   // the sort path's products, numbered over its rows
   if (nlong && annz) {
     GB_SG_TRY(gb_dev_alloc((void **)&len2, ((size_t)annz + 1) * 4));
     GB_SG_TRY(gb_dev_alloc((void **)&off2, ((size_t)annz + 1) * 4));
-    gb_sg_len_long<<<gb_sg_grid(annz), GB_BLOCK, 0, s>>>(anrows, annz, d_arowptr, islong, len,
+    gb_sg_len_long<<<gb_sg_grid(annz), GB_BLOCK, 0, s>>>(anrows, annz, d_arowptr, cls, len,
                                                         len2);
     GB_SG_TRY(hipGetLastError());
     GB_SG_RV(gbd_scan_u32(len2, off2, annz, off2 + annz));
@@ -599,13 +855,23 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
     GB_SG_TRY(gb_dev_alloc((void **)&crowval, ((size_t)cnnz + 1) * 8));
     if (nshort && staged) {
       gb_sg_unstage<<<gb_div_up(nshort, GB_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, slist, d_arowptr, off, cnt, sind, sval, crowptr, crowind, crowval);
+          nshort, list, d_arowptr, off, cnt, sind, sval, crowptr, crowind, crowval);
       GB_SG_TRY(hipGetLastError());
     } else if (nshort) {
       gb_sg_wave<GB_SG_FILL><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, slist, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
+          nshort, list, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
           crowptr, nullptr, crowind, crowval, nullptr, 0, nullptr);
       GB_SG_TRY(hipGetLastError());
+    }
+    if (nmed && staged) {
+      mlist = list ? list + nshort : nullptr;
+      gb_sg_unstage_wave<<<gb_div_up(nmed, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
+          nmed, mlist, d_arowptr, off, cnt, sind, sval, crowptr, crowind, crowval);
+      GB_SG_TRY(hipGetLastError());
+    } else if (nmed) {
+      GB_SG_TRY(gb_sg_medium<GB_SG_FILL>(hcount, list, d_arowptr, d_arowind, d_arowval,
+                                         d_browptr, d_browind, d_browval, crowptr, nullptr,
+                                         crowind, crowval, nullptr, 0, nullptr));
     }
     if (nruns) {
       gb_sg_out<<<gb_sg_grid(nruns), GB_BLOCK, 0, s>>>(nruns, ordr, rrow, rcol, rval, rbeg,
@@ -623,7 +889,7 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
   rv = GOOSEBERRY_SUCCESS;
 done:
   {
-    void *tmp[] = {len, off, isshort, islong, slist, len2, off2, erow, ecol, eval,
+    void *tmp[] = {len, off, cls, count, list, len2, off2, erow, ecol, eval,
                    perm1, row1, ord, flag, rid, runstart, rrow, rcol, rfirst, rval,
                    ordr, rbeg, cnt, crowptr, crowind, crowval, tot, sind, sval};
     for (void *q : tmp) (void)gb_dev_free(q);

@@ -48,6 +48,70 @@ def test_spgemm_bitwise_with_oracle(gb, oracle, case, stage, monkeypatch):
         assert np.array_equal(bits(dense), bits(oracle.spmultsp(a, b, bnc)))
 
 
+def rows_of_products(targets, bncols, seed):
+    """A, B where A's row r has exactly targets[r] products: rows of B of 0 to
+    90 entries (repeated columns among them), filled up with single entries;
+    the last row of A selects 100 empty rows of B first."""
+    rng = np.random.default_rng(seed)
+    blen = np.concatenate([np.zeros(40, int), np.ones(60, int), rng.integers(2, 91, 300)])
+    brp = np.concatenate([[0], np.cumsum(blen)]).astype(np.uint32)
+    b = (brp, rng.integers(0, bncols, brp[-1]).astype(np.uint32),
+         rng.uniform(-1, 1, brp[-1]))
+    rows = []
+    for r, t in enumerate(targets):
+        row, left = [], t
+        if r == len(targets) - 1:
+            row += list(rng.integers(0, 40, 100))
+        while left:
+            l = int(rng.integers(0, 400))
+            if blen[l] > left:
+                l = int(rng.integers(40, 100))
+            row.append(l)
+            left -= int(blen[l])
+        rows.append(row)
+    arp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.uint32)
+    a = (arp, np.concatenate(rows).astype(np.uint32), rng.uniform(-1, 1, arp[-1]))
+    return a, b
+
+
+# products per row around the limits of the row classes (64 products; hash
+# tables of 256 to 4096 columns; 65536 products), for few columns (every step
+# of 64 products shares columns) and for many
+TARGETS = [0, 1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 512, 513, 1000, 1023, 1024, 1025,
+           1536, 1537, 2560, 2561, 4095, 4096, 4097, 9000, 65536, 65537, 7]
+
+
+@pytest.mark.parametrize("stage", ["staged", "two_pass"])
+@pytest.mark.parametrize("bncols", [1, 30, 256, 257, 4096, 4097, 1 << 30])
+def test_spgemm_row_classes(gb, oracle, bncols, stage, monkeypatch):
+    if stage == "two_pass":
+        monkeypatch.setenv("GOOSEBERRY_SPGEMM_STAGE_MAX", "0")
+    print("spgemm row classes", bncols, stage, flush=True)
+    a, b = rows_of_products(TARGETS, bncols, bncols % 1000)
+    n, k = len(TARGETS), 400
+    rp, ri, rv = gb.spmultsp_sp(n, k, bncols, a, b)
+    orp, ori, orv = oracle.spmultsp_sp(a, b, bncols)
+    assert np.array_equal(rp, orp) and np.array_equal(ri, ori)
+    assert np.array_equal(bits(rv), bits(orv))
+    if bncols < 1 << 20:
+        dense = gb.spmultsp(n, k, bncols, a, b)
+        assert np.array_equal(bits(dense), bits(oracle.spmultsp(a, b, bncols)))
+
+
+def test_spgemm_one_medium_class(gb, oracle):
+    # every row in one class of medium rows (no list of rows is made), with
+    # a negative zero that a lone product keeps and the dense result turns
+    rng = np.random.default_rng(8)
+    a, b = rows_of_products([70, 200, 90], 5000, 8)
+    a[2][:] = np.where(rng.random(a[2].size) < 0.5, 0.0, -1.0)
+    rp, ri, rv = gb.spmultsp_sp(3, 400, 5000, a, b)
+    orp, ori, orv = oracle.spmultsp_sp(a, b, 5000)
+    assert np.array_equal(rp, orp) and np.array_equal(ri, ori)
+    assert np.array_equal(bits(rv), bits(orv))
+    assert np.array_equal(bits(gb.spmultsp(3, 400, 5000, a, b)),
+                          bits(oracle.spmultsp(a, b, 5000)))
+
+
 def test_spgemm_signed_zero_empty_and_identity(gb, oracle):
     a = (np.array([0, 1, 1], np.uint32), np.array([0], np.uint32), np.array([-1.0]))
     b = (np.array([0, 1], np.uint32), np.array([1], np.uint32), np.array([0.0]))
