@@ -75,7 +75,9 @@ GB_HD inline uint64_t gbt_strtoull(const char *s, uint64_t n, uint64_t p, int ba
     c = gbt_at(s, n, q);
     int d = base == 16 ? gbt_hexval(c) : (gbt_digit(c) ? (int)(c - '0') : -1);
     if (d < 0) break;
-    if (!ovf) {
+    if (q - d0 < 16) {  // 16 digits fit 64 bits in either base
+      v = v * (uint64_t)base + (uint64_t)d;
+    } else if (!ovf) {
       if (v > (~0ull - (uint64_t)d) / (uint64_t)base) ovf = true;
       else v = v * (uint64_t)base + (uint64_t)d;
     }

@@ -7,6 +7,7 @@ final newline, odd token counts, malformed tokens, signs, hexadecimal and
 special values, long digit strings (settled by the exact fallback, more of
 them than its first list holds), embedded NUL bytes, 0-based and huge
 columns."""
+import ctypes
 import os
 import random
 import struct
@@ -74,6 +75,74 @@ def test_edge_lines(gb, oracle, tmp_path):
                          ids=["empty", "nl", "blank3", "comments", "one", "zero", "wrap"])
 def test_tiny_texts(gb, oracle, tmp_path, text):
     check_text(gb, oracle, tmp_path, text)
+
+
+def line_of(length, rng):
+    """A row line of exactly `length` bytes (at least 12)."""
+    out = b""
+    while length - len(out) > 24:
+        out += b"%d %.6f " % (rng.integers(1, 100000), rng.uniform(-9, 9))
+    return out + b"7 " + b"1" * (length - len(out) - 2)
+
+
+@pytest.mark.parametrize("offset", [0, 1, 8, 15])
+@pytest.mark.parametrize("fill", [0, 9, 300])
+def test_line_lengths_and_text_alignment(gb, oracle, tmp_path, fill, offset):
+    # lines around the sizes of the LDS tile that a wavefront parses from (8
+    # and 16 KiB, by the mean length: `fill` bytes in most lines), at every
+    # alignment of the text in device memory
+    print("ingest lines", fill, offset, flush=True)
+    rng = np.random.default_rng(fill + offset)
+    lengths = [8175, 8176, 8177, 8190, 8191, 8192, 8193, 8208, 16367, 16368, 16383, 16384,
+               16385, 40000, 12, 0]
+    lines = []
+    for n in lengths:
+        lines += [line_of(fill, rng) if fill > 12 else b"3 2.25"[:fill]] * 67
+        lines.append(line_of(n, rng) if n else b"")
+    text = b"\n".join(lines)
+    path = os.path.join(str(tmp_path), "t.csr")
+    with open(path, "wb") as f:
+        f.write(text)
+    d = gb.DeviceArray(len(text) + 16, np.uint8)
+    d.upload(np.frombuffer(b"9" * offset + text + b"9" * (16 - offset), dtype=np.uint8))
+    nr, nc = ctypes.c_uint32(), ctypes.c_uint32()
+    p = [ctypes.c_void_p() for _ in range(3)]
+    gb.check(gb.lib().gooseberry_parse_csr_device(
+        d.ptr + offset, len(text), ctypes.byref(nr), ctypes.byref(nc),
+        *[ctypes.byref(q) for q in p]), "parse")
+    same((nr.value, nc.value) + gb._take_device(nr.value, *[q.value for q in p]),
+         oracle.read_sparse(path))
+
+
+@pytest.mark.parametrize("end", [b"", b"\n", b"\r\n", b" 5 1.5x 2 3", b"\n3 0." + b"7" * 700])
+@pytest.mark.parametrize("base", [0, 1])
+def test_plain_text(gb, oracle, tmp_path, base, end):
+    # entries converted pair by pair: every spacing, odd token counts, comments,
+    # blank and CRLF lines, special values, entries across the 4 KiB chunks; and
+    # (the last two ends) text that is then gone through line by line, for a
+    # token that is no number and for one that reaches too far past its chunk
+    rng = random.Random(base)
+    print("ingest plain", base, end[:8], flush=True)
+    forms = [lambda: "%g" % rng.uniform(-1, 1), lambda: "%.17g" % rng.gauss(0, 1e9),
+             lambda: "%d" % rng.randrange(-9, 9), lambda: "%.3e" % rng.uniform(-1, 1),
+             lambda: rng.choice(["inf", "-nan", "+Infinity", "0x1.8p3", "nan(12)", ".5", "-7.",
+                                 "1e400", "1e-400"]),
+             lambda: "0." + "".join(rng.choice("0123456789") for _ in range(60)),
+             lambda: "0.3000000000000000444089209850062616169452667236328125"]
+    lines = []
+    for r in range(3000):
+        if r % 97 == 5:
+            lines.append("%s 1 2 3 x" % rng.choice("#%'\"/"))
+            continue
+        toks = []
+        for _ in range(rng.randrange(0, 12)):
+            toks += ["%d" % rng.randrange(base, 70000), rng.choice(forms)()]
+        if r % 11 == 0:
+            toks.append("17")  # a column without a value
+        sep = rng.choice([" ", "\t", "  ", " \v\f "])
+        lead = rng.choice(["", "", " ", "\t "])
+        lines.append(lead + sep.join(toks) + rng.choice(["", " ", "\r", " \r"]))
+    check_text(gb, oracle, tmp_path, "\n".join(lines).encode() + end)
 
 
 def test_written_matrices(gb, oracle, tmp_path):
