@@ -869,6 +869,207 @@ static int gb_spmv_launch_t(const gbd_matrix *m, const T *val, const uint8_t *vi
   return GOOSEBERRY_SUCCESS;
 }
 
+// ---------------------------------------------------- several columns
+// C = A B for several columns at a time, A read once for up to GB_MM_COLS of
+// them.  Every column's sums are those of the one-column kernels, product by
+// product in the same order, so C is bit for bit what a column-by-column
+// loop gives.  Two forms:
+//
+// gb_spmm_band, for plans with 16-bit offsets and short rows only: one
+// thread per row gathers from B's columns where they lie.  Consecutive rows
+// of a banded matrix have consecutive columns, so a wavefront's gathers are
+// contiguous in each column of B.
+//
+// gb_spmm_rows, for other plans: B's columns are first transposed to rows of
+// G (2, 4 or 8) values, and G lanes take a row of A, one column each: a
+// scattered entry then costs one 64-byte access for eight columns instead of
+// eight accesses.
+//
+// Bound: the band form by HBM and the latency of its gathers (a million rows
+// of 7 entries, 8 columns: 65.5 us against 208 us for eight SpMVs with a
+// strided result; 152 MB once, 2.3 TB/s), the row form by the accesses to
+// B's rows (random matrices of 29 entries a row, 4 to 32 columns: 1.9 to 2.9
+// times the loop's rate).
+#define GB_MM_COLS 8
+
+// Bt[i G + j] = B[j n + i] for the cols (<= G) columns
+template <int G>
+__global__ void __launch_bounds__(GB_BLOCK)
+gb_spmm_transpose(const double *__restrict__ b, uint32_t n, uint32_t cols,
+                  double *__restrict__ bt) {
+  for (uint32_t i = blockIdx.x * GB_BLOCK + threadIdx.x; i < n; i += gridDim.x * GB_BLOCK) {
+    double v[G];
+#pragma unroll
+    for (int j = 0; j < G; ++j) v[j] = (uint32_t)j < cols ? b[(size_t)j * n + i] : 0.0;
+#pragma unroll
+    for (int j = 0; j < G; ++j) bt[(size_t)i * G + j] = v[j];
+  }
+}
+
+// the work items of gb_spmv_kernel (row blocks, four wavefront rows, one
+// long row), columns c .. c + cols of the row-major C with ldc columns
+template <int G>
+__global__ void __launch_bounds__(GB_BLOCK)
+gb_spmm_rows(const uint32_t *__restrict__ rowptr, const uint32_t *__restrict__ rowind,
+             const double *__restrict__ val, const double *__restrict__ bt,
+             double *__restrict__ c, uint32_t ldc, uint32_t cols,
+             const uint4 *__restrict__ bdesc, uint32_t nstream,
+             const uint32_t *__restrict__ wave_rows, uint32_t nwave, uint32_t nwaveblocks,
+             const uint32_t *__restrict__ block_rows) {
+  __shared__ double lv[GB_STREAM_LDS];
+  __shared__ uint32_t lc[GB_STREAM_LDS];
+  const uint32_t tid = threadIdx.x, w = blockIdx.x;
+  const uint32_t lane = tid & (GB_WAVE - 1), wave = tid / GB_WAVE;
+  if (w < nstream) {
+    const uint4 bd = bdesc[w];
+    const uint32_t k0 = bd.z, cnt = bd.w;
+#pragma unroll
+    for (int i = 0; i < GB_STREAM_ITERS; ++i) {
+      const uint32_t e = i * GB_BLOCK + tid;
+      if (e < cnt) {
+        lc[e] = __builtin_nontemporal_load(&rowind[k0 + e]);
+        lv[e] = __builtin_nontemporal_load(&val[k0 + e]);
+      }
+    }
+    __syncthreads();
+    const uint32_t j = tid % G;
+    for (uint32_t r = bd.x + tid / G; r < bd.y; r += GB_BLOCK / G) {
+      const uint32_t e1 = rowptr[r + 1] - k0;
+      double s = 0.0;
+#pragma unroll 4
+      for (uint32_t e = rowptr[r] - k0; e < e1; ++e) s += lv[e] * bt[(size_t)lc[e] * G + j];
+      if (j < cols) c[(size_t)r * ldc + j] = s;
+    }
+    return;
+  }
+  // a lane's share of a row, as gb_row_lane_sum, for every column
+  const bool is_wave = w < nstream + nwaveblocks;
+  uint32_t row;
+  if (is_wave) {
+    const uint32_t wid = (w - nstream) * GB_WAVES_PER_BLOCK + wave;
+    if (wid >= nwave) return;  // no barrier on this path
+    row = wave_rows[wid];
+  } else {
+    row = block_rows[w - nstream - nwaveblocks];
+  }
+  const uint32_t stride = is_wave ? GB_WAVE : GB_BLOCK;
+  const uint32_t k1 = rowptr[row + 1];
+  double s[G];
+#pragma unroll
+  for (int j = 0; j < G; ++j) s[j] = 0.0;
+  for (uint64_t k = (uint64_t)rowptr[row] + (is_wave ? lane : tid); k < k1; k += stride) {
+    const double *bp = bt + (size_t)__builtin_nontemporal_load(&rowind[k]) * G;
+    const double v = __builtin_nontemporal_load(&val[k]);
+#pragma unroll
+    for (int j = 0; j < G; ++j) s[j] += v * bp[j];
+  }
+#pragma unroll
+  for (int j = 0; j < G; ++j) s[j] = gb_wave_sum(s[j]);
+  if (is_wave) {
+#pragma unroll
+    for (int j = 0; j < G; ++j)
+      if (lane == (uint32_t)j && (uint32_t)j < cols) c[(size_t)row * ldc + j] = s[j];
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < G; ++j)
+    if (lane == 0) lv[wave * G + j] = s[j];
+  __syncthreads();
+  if (tid < cols) {
+    double t = lv[tid];
+#pragma unroll
+    for (int q = 1; q < GB_WAVES_PER_BLOCK; ++q) t += lv[q * G + tid];
+    c[(size_t)row * ldc + tid] = t;
+  }
+}
+
+template <int COLS, bool VD>
+__global__ void __launch_bounds__(GB_BLOCK)
+gb_spmm_band(const uint32_t *__restrict__ rowptr, const int16_t *__restrict__ dcol,
+             const double *__restrict__ val, const uint8_t *__restrict__ vidx,
+             const double *__restrict__ vtab, uint32_t nvals, const double *__restrict__ b,
+             uint32_t ldb, double *__restrict__ c, uint32_t ldc,
+             const uint4 *__restrict__ bdesc) {
+  __shared__ double ltab[VD ? GB_VDICT_MAX : 1];
+  __shared__ double lv[VD ? 1 : GB_STREAM_LDS];
+  __shared__ double out[GB_BLOCK * COLS];
+  __shared__ int16_t lc[GB_STREAM_LDS];
+  __shared__ uint8_t li[VD ? GB_STREAM_LDS : 1];
+  const uint32_t tid = threadIdx.x;
+  const uint4 bd = bdesc[blockIdx.x];
+  const uint32_t k0 = bd.z, cnt = bd.w;
+  if (VD && tid < nvals) ltab[tid] = vtab[tid];
+#pragma unroll
+  for (int i = 0; i < GB_STREAM_ITERS; ++i) {
+    const uint32_t e = i * GB_BLOCK + tid;
+    if (e < cnt) {
+      lc[e] = dcol[k0 + e];
+      if constexpr (VD) li[e] = vidx[k0 + e];
+      else lv[e] = __builtin_nontemporal_load(&val[k0 + e]);
+    }
+  }
+  __syncthreads();
+  const double *bg = b + bd.x;  // the offsets count from the block's first row
+  for (uint32_t r0 = bd.x; r0 < bd.y; r0 += GB_BLOCK) {
+    const uint32_t r = r0 + tid;
+    double s[COLS];
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) s[j] = 0.0;
+    if (r < bd.y) {
+      const uint32_t e1 = rowptr[r + 1] - k0;
+#pragma unroll 2
+      for (uint32_t e = rowptr[r] - k0; e < e1; ++e) {
+        double v;
+        if constexpr (VD) v = ltab[li[e]];
+        else v = lv[e];
+        const double *bp = bg + lc[e];
+#pragma unroll
+        for (int j = 0; j < COLS; ++j) s[j] += v * bp[(size_t)j * ldb];
+      }
+    }
+    // through LDS, so that consecutive lanes write consecutive words of C
+    if (r0 != bd.x) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) out[tid * COLS + j] = s[j];
+    __syncthreads();
+    const uint32_t n = min((uint32_t)GB_BLOCK, bd.y - r0) * COLS;
+    for (uint32_t i = tid; i < n; i += GB_BLOCK)
+      c[(size_t)(r0 + i / COLS) * ldc + i % COLS] = out[i];
+  }
+}
+
+template <int COLS>
+static void gb_spmm_band_go(const gbd_matrix *m, const double *b, double *c, uint32_t ldc) {
+  hipStream_t s = gb_stream();
+  if (m->vidx)
+    gb_spmm_band<COLS, true><<<m->nstream, GB_BLOCK, 0, s>>>(
+        m->rowptr, m->dcol, m->val, m->vidx, m->vtab, m->nvals, b, m->ncols, c, ldc, m->bdesc);
+  else
+    gb_spmm_band<COLS, false><<<m->nstream, GB_BLOCK, 0, s>>>(
+        m->rowptr, m->dcol, m->val, m->vidx, m->vtab, m->nvals, b, m->ncols, c, ldc, m->bdesc);
+}
+
+template <int G>
+static void gb_spmm_rows_go(const gbd_matrix *m, const double *b, double *bt, double *c,
+                            uint32_t ldc, uint32_t cols) {
+  hipStream_t s = gb_stream();
+  const uint32_t g = gb_div_up(m->ncols, GB_BLOCK);
+  gb_spmm_transpose<G><<<g, GB_BLOCK, 0, s>>>(b, m->ncols, cols, bt);
+  const uint32_t nw = gb_spmv_nwaveblocks(m);
+  gb_spmm_rows<G><<<gb_spmv_nwork(m), GB_BLOCK, 0, s>>>(
+      m->rowptr, m->rowind, m->val, bt, c, ldc, cols, m->bdesc, m->nstream,
+      m->rowbins + (m->nrows - m->nwave - m->nblockrows), m->nwave, nw,
+      m->rowbins + (m->nrows - m->nblockrows));
+}
+
+// Several columns at once where the row kernels of this file do the SpMV:
+// not on column splits, x tiles or row parts (kernels of their own), nor on
+// exact plans (whose longer rows are folded in another order).
+static bool gb_spmm_several(const gbd_matrix *m, uint32_t bncols) {
+  return bncols > 1 && !m->nsplit && !m->nparts && !m->xt_ptr && !m->params.exact &&
+         gb_spmv_nwork(m) > 0 && m->ncols > 0;
+}
+
 int gb_spmv_launch(const gbd_matrix *m, const double *x, double *y,
                    uint32_t ystride, double *partials, const gbd_cg_state *cg) {
   return gb_spmv_launch_t<double>(m, m->val, m->vidx, m->vtab, x, y, ystride, partials, cg);
@@ -1947,11 +2148,61 @@ int gbd_spmv(const gbd_matrix *m, const double *d_x, double *d_y) {
 
 int gbd_spmm(const gbd_matrix *m, uint32_t bncols, const double *d_b,
              double *d_c) {
-  for (uint32_t j = 0; j < bncols; ++j) {
-    int rv = gb_spmv_launch(m, d_b + (size_t)j * m->ncols, d_c + j, bncols,
-                            nullptr, nullptr);
-    if (rv != GOOSEBERRY_SUCCESS) return rv;
+  const bool several = gb_spmm_several(m, bncols);
+  const bool band = several && m->dcol && !m->nwave && !m->nblockrows && !m->cshift;
+  // bncols columns in the fewest launches of at most GB_MM_COLS, evenly
+  const uint32_t nl = gb_div_up(bncols, GB_MM_COLS);
+  double *bt = nullptr;
+  if (several && !band) {
+    const uint32_t most = gb_div_up(bncols, nl), g = most > 4 ? 8 : most > 2 ? 4 : 2;
+    if (gb_dev_alloc((void **)&bt, (size_t)m->ncols * g * sizeof(double)) != hipSuccess) {
+      bt = nullptr;  // no room for B's rows: one column at a time
+      (void)hipGetLastError();
+    }
   }
+  if (!band && !bt) {
+    for (uint32_t j = 0; j < bncols; ++j) {
+      int rv = gb_spmv_launch(m, d_b + (size_t)j * m->ncols, d_c + j, bncols,
+                              nullptr, nullptr);
+      if (rv != GOOSEBERRY_SUCCESS) return rv;
+    }
+    return GOOSEBERRY_SUCCESS;
+  }
+  for (uint32_t i = 0, j = 0; i < nl; ++i) {
+    const uint32_t cols = (bncols - j) / (nl - i);
+    const double *b = d_b + (size_t)j * m->ncols;
+    double *c = d_c + j;
+    if (cols == 1) {
+      int rv = gb_spmv_launch(m, b, c, bncols, nullptr, nullptr);
+      if (rv != GOOSEBERRY_SUCCESS) {
+        if (bt) (void)gb_dev_free(bt);
+        return rv;
+      }
+    } else if (band) {
+      switch (cols) {
+        case 2: gb_spmm_band_go<2>(m, b, c, bncols); break;
+        case 3: gb_spmm_band_go<3>(m, b, c, bncols); break;
+        case 4: gb_spmm_band_go<4>(m, b, c, bncols); break;
+        case 5: gb_spmm_band_go<5>(m, b, c, bncols); break;
+        case 6: gb_spmm_band_go<6>(m, b, c, bncols); break;
+        case 7: gb_spmm_band_go<7>(m, b, c, bncols); break;
+        default: gb_spmm_band_go<8>(m, b, c, bncols); break;
+      }
+    } else if (cols > 4) {
+      gb_spmm_rows_go<8>(m, b, bt, c, bncols, cols);
+    } else if (cols > 2) {
+      gb_spmm_rows_go<4>(m, b, bt, c, bncols, cols);
+    } else {
+      gb_spmm_rows_go<2>(m, b, bt, c, bncols, cols);
+    }
+    const hipError_t e = gb_launch_status();
+    if (e != hipSuccess) {
+      if (bt) (void)gb_dev_free(bt);
+      return gb_hip_fail(e, "gbd_spmm", __FILE__, __LINE__);
+    }
+    j += cols;
+  }
+  if (bt) GB_HIP(gb_dev_free(bt));
   return GOOSEBERRY_SUCCESS;
 }
 

@@ -209,6 +209,38 @@ def test_spmm_bncols3(gb, oracle):
     assert np.array_equal(c[short], ref[short])
 
 
+@pytest.mark.parametrize("cols", [2, 3, 4, 5, 6, 7, 8, 9, 11, 17, 32])
+@pytest.mark.parametrize("kind", ["band", "band_values", "bins", "one_row", "plans"])
+def test_spmm_bitwise_each_column(gb, kind, cols):
+    # several columns at a time give bit for bit what a column alone gives:
+    # stencils (16-bit offsets, with and without the value table), every row
+    # bin with scattered columns (row blocks, wavefront rows, long rows, empty
+    # rows, more columns than rows), and the plans that go column by column
+    if kind in ("band", "band_values"):
+        rp, ri, rv = gb.laplacian(3, 17, 13, 19)
+        nc, plans = rp.size - 1, [None, {"wide_values": True}]
+        if kind == "band_values":
+            rv = np.random.default_rng(cols).uniform(-1, 1, rv.size)
+    elif kind == "bins":
+        rp, ri, rv = irregular(3000, 13, [(4, 700), (90, 65), (91, 64), (1000, 5000), (7, 0),
+                                          (2999, 4097)], ncols=9001)
+        nc, plans = 9001, [None, {"wide_index": True}, {"short_max": 8, "wave_max": 40}]
+    elif kind == "one_row":
+        rp, ri, rv = np.array([0, 3], np.uint32), np.array([4, 0, 4], np.uint32), np.ones(3) / 3
+        nc, plans = 5, [None]
+    else:
+        rp, ri, rv = irregular(2000, 5, [(3, 300)], ncols=3000)
+        nc, plans = 3000, [{"exact": True}, {"csplit": 3}, {"xtile": 256}]
+    n = rp.size - 1
+    B = np.random.default_rng(14).uniform(-1, 1, (nc, cols))
+    for plan in plans:
+        print("spmm", kind, cols, plan, flush=True)
+        M = gb.Matrix(rp, ri, rv, ncols=nc, plan=plan)
+        c = M.spmm(np.ascontiguousarray(B.T).ravel(), cols).reshape(n, cols)
+        for j in range(cols):
+            assert np.array_equal(c[:, j], M.spmv(B[:, j])), (plan, j)
+
+
 def test_scale_dropin(gb):
     v = np.random.default_rng(15).uniform(-1, 1, 1000)
     assert np.array_equal(gb.scale(v, 0.37), v * 0.37)
