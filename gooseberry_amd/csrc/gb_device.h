@@ -210,6 +210,13 @@ int gbd_cg_start(gbd_cg *cg, const double *d_b, double *d_x, double tol,
 int gbd_cg_enqueue(gbd_cg *cg, uint32_t k);
 /* Synchronise and copy the state (and, when h_trace != NULL, the trace
  * ring) to the host. */
+/* whether the workspace's solves run whole batches of iterations in one
+ * launch (any number: the launch stops where the solve does).  Such a run whose
+ * workgroups did not get to run side by side ends with the status
+ * GBD_CG_WAITED; gbd_cg_several_launches turns to one launch per step. */
+#define GBD_CG_WAITED 4
+int gbd_cg_one_launch(const gbd_cg *cg);
+void gbd_cg_several_launches(gbd_cg *cg);
 int gbd_cg_poll(gbd_cg *cg, gbd_cg_state *st, double *h_trace);
 /* Capture k iterations into a hipGraph once and replay it for each
  * gbd_cg_enqueue_graph call. */

@@ -35,6 +35,8 @@ struct gbd_cg {
   const gbd_matrix *m;
   uint32_t n;
   double *r, *p, *ap;
+  double *p2;         // one-launch runs: the other buffer of p
+  uint64_t *slots;    // one-launch runs: the exchanges' slots
   double *partials;   // SpMV p.Ap partials (one per SpMV workgroup)
   double *partials2;  // r.r partials (one per elementwise workgroup)
   uint32_t npartials;
@@ -46,6 +48,9 @@ struct gbd_cg {
   const double *b;
   double *x;
   uint32_t grid_elem;  // workgroups of the set-up kernel
+  uint32_t grid_one;   // one-launch runs: workgroups of gb_cg_persist; else 0
+  uint32_t rows_one;   // and rows per workgroup
+  uint32_t spins;      // and reads of a slot before a wait is given up
   uint32_t grid_vec;   // workgroups of the r and x/p updates
   uint32_t chunk;      // rows per workgroup of the r and x/p updates
   hipGraph_t graph[GB_CG_NGRAPH];       // graph[i]: 2^i iterations
@@ -147,11 +152,12 @@ gb_cg_init_state(const double *__restrict__ partials, uint32_t np,
 // with all of its loads issued at once.
 #define GB_CGV_THREADS 512
 #define GB_CGV_GRID 256u
+// rows per thread and pass at most.  Smaller systems take the kernel built
+// for the rows they have (U), and for the SpMV partials per thread (R: at
+// most 32 loads in one round): the sums' order is the same for every U and R.
+// A kernel built for 32 rows a thread spends about 2 us on the 31 absent ones:
+// an iteration took 16.2 us on the 256^2 Laplacian, and takes 12.0 us.
 #define GB_CGV_U 32
-// loads per thread of the partial sums: K2 adds up to 16K SpMV partials in
-// one round, K3 the r update's (at most GB_CGV_GRID)
-#define GB_CGV_RED1 32
-#define GB_CGV_RED2 1
 
 // Fixed-order sum of n partials by a workgroup of T threads: each thread
 // issues R loads before adding (one memory round trip per T R partials);
@@ -196,7 +202,7 @@ __device__ __forceinline__ double gb_cgv_block_sum(double v, double *red) {
   return t;
 }
 
-template <int T, int U>
+template <int T, int U, int R>
 __global__ void __launch_bounds__(T)
 gb_cg_update_r(double *__restrict__ r, const double *__restrict__ ap, uint32_t n,
                uint32_t chunk, const double *__restrict__ pap_partials, uint32_t npap,
@@ -226,7 +232,7 @@ gb_cg_update_r(double *__restrict__ r, const double *__restrict__ ap, uint32_t n
     if (stop && !dn && blockIdx.x == 0) st->done = 1;
     s_stop = stop;
   }
-  const double pap = gb_cgv_sum<T, GB_CGV_RED1>(pap_partials, npap, red);  // barriers inside
+  const double pap = gb_cgv_sum<T, R>(pap_partials, npap, red);  // barriers inside
   if (s_stop) return;
   if (tid == 0) {
     const double dr = st->dr;
@@ -308,7 +314,7 @@ gb_cg_update_xp(double *__restrict__ x, const double *__restrict__ r,
   // `done` is written only by the r update and the set-up, never during
   // this kernel
   if (tid == 0) s_done = *(volatile int32_t *)&st->done;
-  const double dnr = gb_cgv_sum<T, GB_CGV_RED2>(dnr_partials, ndnr, red);  // barriers inside
+  const double dnr = gb_cgv_sum<T, 1>(dnr_partials, ndnr, red);  // barriers inside
   if (s_done) return;
   const double alpha = st->alpha;
   const double beta = dnr / st->dr_prev;
@@ -357,19 +363,351 @@ gb_cg_update_xp(double *__restrict__ x, const double *__restrict__ r,
   }
 }
 
+// A whole run of iterations in one launch, for systems small enough that the
+// matrix fits the workgroups' LDS (one workgroup per CU).  Workgroup w owns a
+// range of rows: their entries in LDS, their x, r, p and Ap in registers, one
+// thread per row.  What workgroups tell each other goes through memory with
+// relaxed agent-scope accesses, which no L1 or other XCD's L2 holds back:
+//
+//  - a sum over all rows: each workgroup stores its partial (after its other
+//    stores have completed) to a slot of its own, and every workgroup reads
+//    all slots until none holds the empty mark, and adds them in order.  The
+//    same exchange orders the data: whoever has read all partials may read
+//    what their owners stored before them.  Three rounds of slots take
+//    turns; an owner empties its slot of the round before once it has
+//    passed a round (all have then read it).
+//  - p: the products of an iteration need the new p of other workgroups'
+//    rows, p = r + (beta/alpha) (alpha p).  r was stored before the r.r
+//    exchange and the old p an iteration earlier, so each workgroup forms
+//    the new p of the columns it needs by itself, with the owner's operations
+//    and so the same bits: two exchanges an iteration, p.Ap and r.r.
+//
+// The sums of each row and the updates are those of gb_cg_update_r and
+// gb_cg_update_xp; the dot products are grouped by thread and workgroup in
+// this kernel's own fixed way.
+//
+// The grid is at most the CUs, so the workgroups run side by side; a wait
+// that does not end within `spins` reads sets the status GBD_CG_WAITED
+// and ends the launch (the host then starts again on the other kernels).
+//
+// Bound: the latency of two exchanges (1.4 us for 16 workgroups to 2.5 us for
+// 256, in a kernel of exchanges alone) and of the gathers.  Per iteration,
+// with the host's part, against three kernels replayed from a graph: 5.1 and
+// 15.3 us on the 64^2 Laplacian, 7.6 and 16.2 us at 256^2, 10.7 and 17.9 us at
+// 400^2, 16.5 and 22.1 us at 600^2, 17.5 and 22.4 us at 70^3 (those kernels
+// built for small systems, below: 11.2, 12.0, 14.0, 18.5 and 18.8 us).  With
+// 1024 threads a workgroup 256^2 takes 8.0 us, with 128 workgroups 8.8 us,
+// with 32 workgroups 8.8 us.  Tried instead, and slower at every size above
+// 65,000 rows: two kernels an iteration, the x/p update in the SpMV's (11.1 us
+// at 256^2, 22.1 us at 600^2, 43 us at 100^3).
+#define GB_CGP_THREADS 512
+#define GB_CGP_ENTRIES 12544u  // entries in a workgroup's LDS (147 KB)
+#define GB_CGP_GRID 256u
+#define GB_CGP_ROWS 4          // rows per thread at most
+#define GB_CGP_WGS 64u         // workgroups, while the rows fit them
+#define GB_CGP_SPINS (1u << 20)
+static_assert(GB_CGP_GRID <= GB_CGP_THREADS, "one slot per thread");
+#define GB_CGP_PAD 16          // slots a cache line apart
+#define GB_CGP_SLOT_BYTES (3ull * GB_CGP_GRID * GB_CGP_PAD * 8)
+#define GB_CGP_EMPTY 0x7ff8dead00000001ull
+
+__device__ __forceinline__ double gb_cgp_load(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void gb_cgp_store(double *p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct gb_cgp_lds {
+  double val[GB_CGP_ENTRIES];
+  uint32_t col[GB_CGP_ENTRIES];
+  double part[GB_CGP_GRID];
+  double red[GB_CGP_THREADS / GB_WAVE];
+  uint32_t bad;
+};
+
+// the sum of every workgroup's d, in a fixed order, on every thread; round
+// counts the exchanges of the launch.  False when a wait ran out.
+__device__ __forceinline__ bool gb_cgp_sum(double d, uint64_t *slots, uint32_t round,
+                                           uint32_t spins, gb_cgp_lds &L, double *sum) {
+  const uint32_t tid = threadIdx.x, W = gridDim.x;
+  d = gb_wave_sum(d);
+  if ((tid & (GB_WAVE - 1)) == 0) L.red[tid / GB_WAVE] = d;
+  // this wavefront's stores have completed before any partial is out
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  uint64_t *mine = slots + (size_t)(round % 3) * GB_CGP_GRID * GB_CGP_PAD;
+  if (tid == 0 && W > 1) {
+    double t = L.red[0];
+#pragma unroll
+    for (int w = 1; w < GB_CGP_THREADS / GB_WAVE; ++w) t += L.red[w];
+    uint64_t bits = (uint64_t)__double_as_longlong(t);
+    if (!(t == t)) bits = 0x7ff8000000000000ull;  // any NaN, and not the mark
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __hip_atomic_store(&mine[blockIdx.x * GB_CGP_PAD], bits, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (W == 1) {  // the workgroup's own partials are all
+    double t = L.red[0];
+#pragma unroll
+    for (int w = 1; w < GB_CGP_THREADS / GB_WAVE; ++w) t += L.red[w];
+    __syncthreads();  // red is used by the next sum
+    *sum = t;
+    return true;
+  }
+  if (tid < W) {
+    uint64_t v;
+    uint32_t n = 0;
+    while ((v = __hip_atomic_load(&mine[tid * GB_CGP_PAD], __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT)) == GB_CGP_EMPTY) {
+      if (++n > spins) {
+        L.bad = 1;
+        break;
+      }
+    }
+    L.part[tid] = __longlong_as_double((long long)v);
+  }
+  __syncthreads();
+  if (L.bad) return false;
+  if (tid == 0)  // the round before: everyone has read it
+    __hip_atomic_store(&slots[((size_t)((round + 2) % 3) * GB_CGP_GRID + blockIdx.x) *
+                              GB_CGP_PAD],
+                       GB_CGP_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  double t = 0.0;
+  for (uint32_t i = tid & (GB_WAVE - 1); i < W; i += GB_WAVE) t += L.part[i];
+  *sum = gb_wave_sum(t);
+  return true;
+}
+
+__global__ void __launch_bounds__(GB_BLOCK)
+gb_cgp_empty(uint64_t *__restrict__ slots) {
+  for (uint32_t i = threadIdx.x; i < 3 * GB_CGP_GRID; i += GB_BLOCK)
+    slots[(size_t)i * GB_CGP_PAD] = GB_CGP_EMPTY;
+}
+
+// k iterations (fewer when the solve stops); p0 holds p before and after,
+// p1 is the other buffer
+template <int R>
+__global__ void __launch_bounds__(GB_CGP_THREADS)
+gb_cg_persist(const uint32_t *__restrict__ rowptr, const uint32_t *__restrict__ rowind,
+              const double *__restrict__ val, uint32_t n, uint32_t rows, double *x, double *r,
+              double *p0, double *p1, uint64_t *slots, gbd_cg_state *st, double *trace,
+              uint32_t trace_cap, uint32_t k, uint32_t spins) {
+  constexpr uint32_t T = GB_CGP_THREADS;
+  constexpr uint32_t U = 8;  // entries of a row whose gathers are in flight
+  __shared__ gb_cgp_lds L;
+  const uint32_t tid = threadIdx.x;
+  if (st->done || st->status) return;  // every workgroup alike: nothing is written yet
+  const uint32_t row0 = blockIdx.x * rows;
+  const uint32_t end = n - row0 < rows ? n : row0 + rows;
+  const uint32_t k0 = rowptr[row0], k1 = rowptr[end];
+  if (tid == 0) L.bad = 0;
+  for (uint32_t e = tid; e < k1 - k0; e += T) {
+    L.col[e] = rowind[k0 + e];
+    L.val[e] = val[k0 + e];
+  }
+  uint32_t e0[R], e1[R];
+  double xo[R], ro[R], po[R], ao[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const uint32_t i = row0 + q * T + tid;
+    e0[q] = e1[q] = 0;
+    xo[q] = ro[q] = po[q] = ao[q] = 0.0;
+    if (i < end) {
+      e0[q] = rowptr[i] - k0;
+      e1[q] = rowptr[i + 1] - k0;
+      xo[q] = x[i];
+      ro[q] = r[i];
+      po[q] = p0[i];
+    }
+  }
+  double dr = st->dr, dr_prev = st->dr_prev, rnorm = st->rnorm, pap = st->pap;
+  double alpha = st->alpha, beta = st->beta, boa = 0.0;
+  const double tol = st->tol;
+  unsigned long long iter = st->iter;
+  const unsigned long long maxiter = st->maxiter;
+  int status = 0;
+  uint32_t round = 0;
+  double *pold = p0, *pnew = p1;
+  uint32_t ulen = 0;  // entries of the wavefront's longest row
+#pragma unroll
+  for (int q = 0; q < R; ++q) ulen = max(ulen, e1[q] - e0[q]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) ulen = max(ulen, (uint32_t)__shfl_xor((int)ulen, o, GB_WAVE));
+  ulen = (uint32_t)__builtin_amdgcn_readfirstlane((int)ulen);
+  __syncthreads();
+  for (uint32_t it = 0; it < k && !status; ++it) {
+    // Ap of the new p (the first iteration's p is complete)
+    double d = 0.0;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const uint32_t i = row0 + q * T + tid;
+      if (it && i < end) {
+        const double ps = alpha * po[q];
+        const double t = ps * boa;
+        po[q] = ro[q] + t;
+        gb_cgp_store(&pnew[i], po[q]);
+      }
+      double s = 0.0;
+      for (uint32_t e = e0[q]; e < e1[q]; e += U) {
+        uint32_t c[U];
+        double a[U], gp[U], gr[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) c[u] = L.col[min(e + u, e1[q] - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+          if (u < ulen) {
+            gp[u] = gb_cgp_load(&pold[c[u]]);
+            if (it) gr[u] = gb_cgp_load(&r[c[u]]);
+          }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) a[u] = L.val[min(e + u, e1[q] - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+          double pc = gp[u];
+          if (it) {
+            const double t = (alpha * gp[u]) * boa;
+            pc = gr[u] + t;
+          }
+          if (e + u < e1[q]) s += a[u] * pc;
+        }
+      }
+      ao[q] = s;
+      d += po[q] * s;
+    }
+    if (!gb_cgp_sum(d, slots, round++, spins, L, &pap)) break;
+    alpha = dr / pap;
+    if (!(pap != 0.0) || !isfinite(alpha)) {
+      status = 3;
+      break;
+    }
+    if (it) {  // pnew is the current p now
+      double *t = pold;
+      pold = pnew;
+      pnew = t;
+    }
+    d = 0.0;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const uint32_t i = row0 + q * T + tid;
+      if (i < end) {
+        const double aps = alpha * ao[q];
+        ro[q] = ro[q] - aps;
+        gb_cgp_store(&r[i], ro[q]);
+        d += ro[q] * ro[q];
+        const double ps = alpha * po[q];
+        xo[q] = xo[q] + ps;
+      }
+    }
+    double dnr;
+    if (!gb_cgp_sum(d, slots, round++, spins, L, &dnr)) break;
+    beta = dnr / dr;
+    dr_prev = dr;
+    dr = dnr;
+    rnorm = sqrt(dnr);
+    ++iter;
+    if (rnorm <= tol) status = 1;
+    else if (!isfinite(dnr)) status = 3;
+    else if (maxiter && iter >= maxiter) status = 2;
+    boa = beta / alpha;
+    if (trace_cap && blockIdx.x == 0 && tid == 0) trace[(iter - 1) % trace_cap] = rnorm;
+  }
+  if (L.bad) {  // set before a barrier that every thread has passed
+    if (tid == 0) st->status = GBD_CG_WAITED;
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const uint32_t i = row0 + q * T + tid;
+    if (i < end) {
+      x[i] = xo[q];
+      if (!status) {
+        const double ps = alpha * po[q];
+        const double t = ps * boa;
+        p0[i] = ro[q] + t;
+      }
+    }
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    st->pap = pap;
+    st->alpha = alpha;
+    st->beta = beta;
+    st->dr = dr;
+    st->dr_prev = dr_prev;
+    st->rnorm = rnorm;
+    st->iter = iter;
+    st->iter_next = iter;
+    if (status) {
+      st->status = status;
+      st->done = 1;
+    }
+  }
+}
+
+template <int U, int R>
+static void gb_cg_go_r(gbd_cg *cg, uint32_t npap) {
+  gb_cg_update_r<GB_CGV_THREADS, U, R><<<cg->grid_vec, GB_CGV_THREADS, 0, gb_stream()>>>(
+      cg->r, cg->ap, cg->n, cg->chunk, cg->partials, npap, cg->partials2, cg->st);
+}
+
+template <int U>
+static void gb_cg_go_r_u(gbd_cg *cg, uint32_t npap) {
+  if (npap <= 1 * GB_CGV_THREADS) gb_cg_go_r<U, 1>(cg, npap);
+  else if (npap <= 4 * GB_CGV_THREADS) gb_cg_go_r<U, 4>(cg, npap);
+  else gb_cg_go_r<U, 32>(cg, npap);
+}
+
+// the r update after npap SpMV partials
+static void gb_cg_launch_r(gbd_cg *cg, uint32_t npap) {
+  const uint32_t rows = gb_div_up(cg->chunk, GB_CGV_THREADS);
+  if (rows <= 1) gb_cg_go_r_u<1>(cg, npap);
+  else if (rows <= 4) gb_cg_go_r_u<4>(cg, npap);
+  else if (rows <= 8) gb_cg_go_r_u<8>(cg, npap);
+  else gb_cg_go_r_u<GB_CGV_U>(cg, npap);
+}
+
+template <int U>
+static void gb_cg_go_xp(gbd_cg *cg) {
+  gb_cg_update_xp<GB_CGV_THREADS, U><<<cg->grid_vec, GB_CGV_THREADS, 0, gb_stream()>>>(
+      cg->x, cg->r, cg->p, cg->n, cg->chunk, cg->partials2, cg->grid_vec, cg->st,
+      cg->trace, cg->trace_cap);
+}
+
+static void gb_cg_launch_xp(gbd_cg *cg) {
+  const uint32_t rows = gb_div_up(cg->chunk, GB_CGV_THREADS);
+  if (rows <= 1) gb_cg_go_xp<1>(cg);
+  else if (rows <= 4) gb_cg_go_xp<4>(cg);
+  else if (rows <= 8) gb_cg_go_xp<8>(cg);
+  else gb_cg_go_xp<GB_CGV_U>(cg);
+}
+
+template <int R>
+static void gb_cg_go_persist(gbd_cg *cg, uint32_t k) {
+  const gbd_matrix *m = cg->m;
+  gb_cg_persist<R><<<cg->grid_one, GB_CGP_THREADS, 0, gb_stream()>>>(
+      m->rowptr, m->rowind, m->val, cg->n, cg->rows_one, cg->x, cg->r, cg->p, cg->p2,
+      cg->slots, cg->st, cg->trace, cg->trace_cap, k, cg->spins);
+}
+
 static int gb_cg_enqueue_raw(gbd_cg *cg, uint32_t k) {
-  hipStream_t s = gb_stream();
-  const uint32_t n = cg->n;
-  const uint32_t g1 = gb_spmv_npartials(cg->m);
+  if (cg->grid_one) {
+    gb_cgp_empty<<<1, GB_BLOCK, 0, gb_stream()>>>(cg->slots);
+    GB_LAUNCH_CHECK();
+    const uint32_t per = gb_div_up(cg->rows_one, GB_CGP_THREADS);
+    if (per <= 1) gb_cg_go_persist<1>(cg, k);
+    else if (per <= 2) gb_cg_go_persist<2>(cg, k);
+    else gb_cg_go_persist<GB_CGP_ROWS>(cg, k);
+    GB_LAUNCH_CHECK();
+    return GOOSEBERRY_SUCCESS;
+  }
   for (uint32_t it = 0; it < k; ++it) {
     int rv = gb_spmv_launch(cg->m, cg->p, cg->ap, 1, cg->partials, cg->st);
     if (rv != GOOSEBERRY_SUCCESS) return rv;
-    gb_cg_update_r<GB_CGV_THREADS, GB_CGV_U><<<cg->grid_vec, GB_CGV_THREADS, 0, s>>>(
-        cg->r, cg->ap, n, cg->chunk, cg->partials, g1, cg->partials2, cg->st);
+    gb_cg_launch_r(cg, gb_spmv_npartials(cg->m));
     GB_LAUNCH_CHECK();
-    gb_cg_update_xp<GB_CGV_THREADS, GB_CGV_U><<<cg->grid_vec, GB_CGV_THREADS, 0, s>>>(
-        cg->x, cg->r, cg->p, n, cg->chunk, cg->partials2, cg->grid_vec, cg->st,
-        cg->trace, cg->trace_cap);
+    gb_cg_launch_xp(cg);
     GB_LAUNCH_CHECK();
   }
   return GOOSEBERRY_SUCCESS;
@@ -394,13 +732,55 @@ extern "C" {
 // looked up once per device with hipGetSymbolAddress; host code uses that
 // address, never the array's name.  Every such solve on a device shares the
 // array, so solves that overlap on one device would race (the library lock
-// serialises the public entry points of one process).
+// serialises the public entry points of one process).  Small systems run in
+// one launch here too, so both entry points give the same bits.
 #define GB_CG_SCRATCH_BYTES (128ull << 20)
 #define GB_CG_SCRATCH_MAXDEV 64
 static __device__ __align__(256) unsigned char scratch[GB_CG_SCRATCH_BYTES];
 static void *g_scratch_addr[GB_CG_SCRATCH_MAXDEV];
 static gbd_cg g_scratch_cg;            // host bookkeeping of the shared workspace
 static gbd_cg_state g_scratch_hst;     // its polled state (pageable host memory)
+
+// Whether the solve runs in one launch, and on which workgroups: the fewest
+// (the exchanges' time grows with them) whose rows' entries fit their LDS,
+// for matrices with short rows only.  The entries of a range of rows are read
+// from the row pointers once per matrix.
+static void gb_cg_geometry_one(gbd_cg *cg) {
+  const gbd_matrix *m = cg->m;
+  cg->grid_one = 0;
+  if (!cg->n || m->nwave || m->nblockrows || m->nsplit || m->nparts || m->xt_ptr || m->cshift)
+    return;
+  uint32_t cus = gb_num_cus();
+  if (cus > GB_CGP_GRID) cus = GB_CGP_GRID;
+  for (uint32_t W = GB_CGP_WGS; W <= cus; W *= 2) {
+    // a row per thread, or fewer rows a workgroup when they are long
+    uint32_t w = gb_div_up(cg->n, GB_CGP_THREADS);
+    const uint32_t we = gb_div_up(m->nnz, GB_CGP_ENTRIES / 8 * 7);
+    if (w < we) w = we;
+    if (w > W) w = W;
+    const uint32_t rows = gb_div_up(gb_div_up(cg->n, w), GB_WAVE) * GB_WAVE;
+    if (rows > GB_CGP_ROWS * GB_CGP_THREADS) continue;
+    w = gb_div_up(cg->n, rows);
+    uint32_t ptr[GB_CGP_GRID + 1];
+    if (hipMemcpy2DAsync(ptr, 4, m->rowptr, (size_t)rows * 4, 4, w, hipMemcpyDeviceToHost,
+                         gb_stream()) != hipSuccess ||
+        hipStreamSynchronize(gb_stream()) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    ptr[w] = (uint32_t)m->nnz;
+    uint32_t most = 0;
+    for (uint32_t i = 0; i < w; ++i)
+      if (ptr[i + 1] - ptr[i] > most) most = ptr[i + 1] - ptr[i];
+    if (most > GB_CGP_ENTRIES) continue;
+    // GOOSEBERRY_CG_SPINS: the tests' way into the end of a wait
+    const char *e = getenv("GOOSEBERRY_CG_SPINS");
+    cg->spins = e && *e ? (uint32_t)strtoul(e, nullptr, 10) : GB_CGP_SPINS;
+    cg->grid_one = w;
+    cg->rows_one = rows;
+    return;
+  }
+}
 
 // Launch geometry and partial-array sizes of a solve with m.
 static void gb_cg_geometry(gbd_cg *cg, const gbd_matrix *m) {
@@ -415,6 +795,7 @@ static void gb_cg_geometry(gbd_cg *cg, const gbd_matrix *m) {
   if (gv > GB_CGV_GRID) gv = GB_CGV_GRID;
   cg->chunk = gb_div_up(gb_div_up(nn, gv), GB_WAVE) * GB_WAVE;
   cg->grid_vec = gb_div_up(nn, cg->chunk);
+  gb_cg_geometry_one(cg);
   uint32_t gs = gb_spmv_npartials(m);
   cg->npartials = gs > cg->grid_elem ? gs : cg->grid_elem;
 }
@@ -434,6 +815,9 @@ int gbd_cg_create(const gbd_matrix *m, gbd_cg **out) {
   hipError_t e = gb_dev_alloc((void **)&cg->r, nb);
   if (e == hipSuccess) e = gb_dev_alloc((void **)&cg->p, nb);
   if (e == hipSuccess) e = gb_dev_alloc((void **)&cg->ap, nb);
+  if (e == hipSuccess && cg->grid_one) e = gb_dev_alloc((void **)&cg->p2, nb);
+  if (e == hipSuccess && cg->grid_one)
+    e = gb_dev_alloc((void **)&cg->slots, GB_CGP_SLOT_BYTES);
   if (e == hipSuccess)
     e = gb_dev_alloc((void **)&cg->partials, (size_t)cg->npartials * sizeof(double));
   if (e == hipSuccess)
@@ -457,6 +841,8 @@ void gbd_cg_destroy(gbd_cg *cg) {
   (void)gb_dev_free(cg->r);
   (void)gb_dev_free(cg->p);
   (void)gb_dev_free(cg->ap);
+  (void)gb_dev_free(cg->p2);
+  (void)gb_dev_free(cg->slots);
   (void)gb_dev_free(cg->partials);
   (void)gb_dev_free(cg->partials2);
   (void)gb_dev_free(cg->st);
@@ -499,7 +885,7 @@ int gbd_cg_enqueue(gbd_cg *cg, uint32_t k) { return gb_cg_enqueue_raw(cg, k); }
 // per power of two, captured on first use and kept while x stays the same).
 int gbd_cg_enqueue_graph(gbd_cg *cg, uint32_t k) {
   hipStream_t s = gb_stream();
-  if (!gb_graphs_enabled() || cg->noalloc) return gb_cg_enqueue_raw(cg, k);
+  if (!gb_graphs_enabled() || cg->noalloc || cg->grid_one) return gb_cg_enqueue_raw(cg, k);
   if (cg->graph_x != cg->x) {
     gb_cg_drop_graph(cg);
     cg->graph_x = cg->x;
@@ -545,6 +931,10 @@ int gbd_cg_poll(gbd_cg *cg, gbd_cg_state *st, double *h_trace) {
   return GOOSEBERRY_SUCCESS;
 }
 
+int gbd_cg_one_launch(const gbd_cg *cg) { return cg->grid_one != 0; }
+
+void gbd_cg_several_launches(gbd_cg *cg) { cg->grid_one = 0; }
+
 size_t gbd_cg_scratch_max() { return GB_CG_SCRATCH_BYTES; }
 
 int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out) {
@@ -556,7 +946,9 @@ int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out) {
   gb_cg_geometry(cg, m);
   auto al = [](uint64_t b) { return (b + 255) & ~(uint64_t)255; };
   const uint64_t nb = al((uint64_t)(cg->n ? cg->n : 1) * sizeof(double));
-  const uint64_t o_p = nb, o_ap = 2 * nb, o_pa = 3 * nb;
+  const uint64_t o_p = nb, o_ap = 2 * nb, o_p2 = 3 * nb;
+  const uint64_t o_sl = 4 * nb;
+  const uint64_t o_pa = cg->grid_one ? o_sl + GB_CGP_SLOT_BYTES : 3 * nb;
   const uint64_t o_pa2 = o_pa + al((uint64_t)cg->npartials * sizeof(double));
   const uint64_t o_st = o_pa2 + al((uint64_t)gb_cg_np2(cg) * sizeof(double));
   const uint64_t need = o_st + al(sizeof(gbd_cg_state));
@@ -582,6 +974,10 @@ int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out) {
   cg->r = (double *)base;
   cg->p = (double *)(base + o_p);
   cg->ap = (double *)(base + o_ap);
+  if (cg->grid_one) {
+    cg->p2 = (double *)(base + o_p2);
+    cg->slots = (uint64_t *)(base + o_sl);
+  }
   cg->partials = (double *)(base + o_pa);
   cg->partials2 = (double *)(base + o_pa2);
   cg->st = (gbd_cg_state *)(base + o_st);

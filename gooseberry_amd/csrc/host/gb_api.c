@@ -751,6 +751,9 @@ int gooseberry_matrix_cuthillmckee(gooseberry_matrix_t mat,
 #define GB_CG_FIRST 8
 #define GB_CG_MAXBATCH 64
 #define GB_CG_TRACE 64
+/* iterations of a one-launch run: it stops by itself, so the number only
+ * bounds a launch's time (a few milliseconds) */
+#define GB_CG_ONE 1024
 
 static uint32_t gb_cg_next_batch(uint32_t k, uint64_t it0, double r0,
     const gbd_cg_state *st)
@@ -775,15 +778,20 @@ static uint32_t gb_cg_next_batch(uint32_t k, uint64_t it0, double r0,
 static int cgd_loop(gbd_cg *cg, const real_t *d_b, real_t *d_x, real_t tol,
     int tol_mode, size_t niter, FILE *flog, gooseberry_cgd_info_t *info)
 {
+  uint64_t printed = 0;
+  int rv;
+START:
   /* the per-iteration residuals are kept on the device only for a log */
-  int rv = gbd_cg_start(cg, d_b, d_x, tol,
+  rv = gbd_cg_start(cg, d_b, d_x, tol,
       tol_mode == GOOSEBERRY_TOL_RELATIVE, niter, flog ? GB_CG_TRACE : 0);
   if (rv != GOOSEBERRY_SUCCESS) return rv;
   gbd_cg_state st;
   double trace[GB_CG_TRACE];
-  uint64_t printed = 0;
-  rv = gbd_cg_poll(cg, &st, NULL);
+  const int one = gbd_cg_one_launch(cg);
   uint32_t k = GB_CG_FIRST;
+  memset(&st, 0, sizeof(st));
+  if (one) k = flog ? GB_CG_TRACE : GB_CG_ONE;   /* it looks at the state itself */
+  else rv = gbd_cg_poll(cg, &st, NULL);
   while (rv == GOOSEBERRY_SUCCESS && !st.done) {
     const uint64_t it0 = st.iter;
     const double r0 = st.rnorm;
@@ -791,6 +799,12 @@ static int cgd_loop(gbd_cg *cg, const real_t *d_b, real_t *d_x, real_t tol,
     if (rv != GOOSEBERRY_SUCCESS) break;
     rv = gbd_cg_poll(cg, &st, flog ? trace : NULL);
     if (rv != GOOSEBERRY_SUCCESS) break;
+    if (st.status == GBD_CG_WAITED) {
+      /* the workgroups did not run side by side: again, in several launches */
+      gbd_cg_several_launches(cg);
+      if (d_b == d_x) return GOOSEBERRY_ERROR_DEVICE;
+      goto START;
+    }
     if (flog) {
       for (; printed < st.iter; ++printed) {
         /* src/cgd.c:116 */
@@ -798,7 +812,7 @@ static int cgd_loop(gbd_cg *cg, const real_t *d_b, real_t *d_x, real_t tol,
             trace[printed % GB_CG_TRACE]);
       }
     }
-    k = gb_cg_next_batch(k, it0, r0, &st);
+    if (!one) k = gb_cg_next_batch(k, it0, r0, &st);
   }
   if (rv != GOOSEBERRY_SUCCESS) return rv;
   if (info) {

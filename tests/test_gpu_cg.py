@@ -69,6 +69,102 @@ def test_first_iterations_track_oracle(gb, oracle):
         assert np.max(np.abs(x - xr)) <= 1e-12 * np.max(np.abs(xr))
 
 
+def band_spd(n, half, seed):
+    """A symmetric, strictly dominant band matrix; each row's off-diagonals at
+    distances 1 .. half, a third of them missing."""
+    rng = np.random.default_rng(seed)
+    ii, jj, vv = [], [], []
+    for d in range(1, min(half, n - 1) + 1):
+        keep = np.nonzero(rng.random(n - d) < 2 / 3)[0]
+        v = rng.uniform(-1, 0, keep.size)
+        ii += [keep, keep + d]
+        jj += [keep + d, keep]
+        vv += [v, v]
+    ii = np.concatenate(ii + [np.arange(n)]) if ii else np.arange(n)
+    off = np.bincount(ii[:ii.size - n], weights=-np.concatenate(vv) if vv else None, minlength=n)
+    jj = np.concatenate(jj + [np.arange(n)])
+    vv = np.concatenate(vv + [1.05 * off + 0.1])
+    order = np.lexsort((jj, ii))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(ii, minlength=n))]).astype(np.uint32)
+    return rp, jj[order].astype(np.uint32), vv[order]
+
+
+def solve_both(gb, monkeypatch, rp, ri, rv, b, tol, niter=0):
+    """One launch for the run of iterations, and (its waits given up at once)
+    one launch per step."""
+    x1, i1 = gb.Matrix(rp, ri, rv).cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
+    monkeypatch.setenv("GOOSEBERRY_CG_SPINS", "0")
+    M = gb.Matrix(rp, ri, rv)
+    x2, i2 = M.cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
+    x3, i3 = M.cgd(b, tol, gb.TOL_RELATIVE, niter=niter)  # stays with that
+    monkeypatch.delenv("GOOSEBERRY_CG_SPINS")
+    assert i3.niter == i2.niter and np.array_equal(x2, x3)
+    return (x1, i1), (x2, i2)
+
+
+# rows around the sizes of the one-launch solve: one workgroup (512 rows), 64
+# workgroups of 512 to 2048 rows, 128 and 256 workgroups, and past them; and
+# the entries its LDS holds (rows of about 3, 28 and 60 entries)
+@pytest.mark.parametrize("n,half", [
+    (1, 0), (2, 1), (64, 3), (511, 2), (512, 2), (513, 2), (1025, 40), (5000, 44), (32768, 2),
+    (32769, 2), (40000, 20), (65600, 2), (131072, 2), (131073, 2), (262145, 2), (524289, 2)])
+def test_small_systems_in_one_launch(gb, oracle, monkeypatch, n, half):
+    print("cg one launch", n, half, flush=True)
+    rp, ri, rv = band_spd(n, half, n)
+    b = gb.uniform(n, n)
+    (x1, i1), (x2, i2) = solve_both(gb, monkeypatch, rp, ri, rv, b, 1e-11)
+    xr, it, rmse, _ = oracle.cgd(rp, ri, rv, b, 1e-11 * np.linalg.norm(b))
+    for x, i in ((x1, i1), (x2, i2)):
+        assert i.status == 1 and abs(int(i.niter) - it) <= 2
+        # residuals of 1e-11 and a condition number below 43 (the rows'
+        # dominance): x within 43 x 2e-11 of the oracle's
+        assert np.linalg.norm(x - xr) <= 1e-9 * np.linalg.norm(xr)
+        assert true_rel(oracle, rp, ri, rv, x, b) <= 1.05e-11
+    # the first iterations differ only by the order of the dot products
+    if n > 64:
+        (y1, j1), (y2, j2) = solve_both(gb, monkeypatch, rp, ri, rv, b, 0.0, niter=3)
+        assert j1.niter == j2.niter == 3 and j1.status == j2.status == 2
+        assert np.max(np.abs(y1 - y2)) <= 1e-13 * np.max(np.abs(y2))
+
+
+def test_one_launch_scattered_columns_and_repeats(gb, oracle):
+    # random columns all over the system, rows of very different lengths; a
+    # matrix solved twice (and with another x) gives the same bits
+    M = gb.generate_sdd(20000, 7, 2, 25)
+    rp, ri, rv = M.download()
+    b = gb.uniform(2, 20000)
+    x, info = M.cgd(b, 1e-10, gb.TOL_RELATIVE)
+    x2, info2 = M.cgd(b, 1e-10, gb.TOL_RELATIVE)
+    assert info.status == 1 and info2.niter == info.niter and np.array_equal(x, x2)
+    _, it, _, _ = oracle.cgd(rp, ri, rv, b, 1e-10 * np.linalg.norm(b))
+    assert abs(int(info.niter) - it) <= 2
+    assert true_rel(oracle, rp, ri, rv, x, b) <= 1.05e-10
+
+
+@pytest.mark.parametrize("kind", ["zero_b", "nan_b", "zero_matrix", "indefinite"])
+def test_one_launch_stops_as_the_steps_do(gb, monkeypatch, kind):
+    rp, ri, rv = gb.laplacian(2, 40)
+    b = gb.uniform(4, 1600)
+    if kind == "zero_b":
+        b = np.zeros(1600)
+    elif kind == "nan_b":
+        b[700] = np.nan
+    elif kind == "zero_matrix":
+        rv = np.zeros_like(rv)
+    else:
+        rv = np.where(np.arange(rv.size) % 2 == 0, rv, -rv)
+    got = []
+    for spins in (None, "0"):
+        if spins:
+            monkeypatch.setenv("GOOSEBERRY_CG_SPINS", spins)
+        M = gb.Matrix(rp, ri, rv)
+        x, info = M.cgd(b, 1e-10, gb.TOL_RELATIVE, niter=12)
+        got.append((int(info.status), int(info.niter)))
+        if kind in ("zero_b", "zero_matrix"):
+            assert np.array_equal(x, np.zeros(1600))
+    assert got[0] == got[1], got
+
+
 def test_config2_full_size_true_residual(gb, oracle):
     rp, ri, rv = gb.laplacian(3, 160)
     n = rp.size - 1
