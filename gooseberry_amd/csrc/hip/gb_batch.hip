@@ -2,23 +2,22 @@
 //
 // A batch holds up to max_slots systems, each a resident matrix (its own CSR
 // and SpMV plan) with its own vectors, partial-sum arrays and state.  One
-// device step advances every active system by one step with four launches
+// device step advances every active system by one step with three launches
 // over work lists:
 //   K1 gb_b_spmv     (system, SpMV work item): Ap and one p.Ap partial per
 //                    item, or in a refresh step the FP64 residual b - A x and
 //                    its partials.  A column-split matrix runs over its
 //                    slices into partial vectors (FP64 ones in refresh
-//                    steps), which K3 adds; its refresh norm is tested in K4.
+//                    steps), which K2 adds; its refresh norm is tested in K3.
 //                    A matrix with an x-tile plan has no items: its SpMV is a
 //                    launch of its own (gb_b_spmv_xt, one partial per row
 //                    block) after the list's.
-//   K2 gb_b_reduce   (system): alpha, or the refreshed residual norm and the
-//                    convergence test
-//   K3 gb_b_update   (system, chunk of GB_BCHUNK rows): x/r update and r.r
-//                    partials, or the FP32 copy of a refreshed residual
-//   K4 gb_b_pupdate  (system, chunk): beta (every chunk adds the system's
-//                    partials in the same order), stopping / refresh
-//                    decision, p update
+//   K2 gb_b_update   (system, chunk of GB_BCHUNK rows): alpha, or the refreshed
+//                    residual norm and the convergence test (every chunk adds
+//                    the system's partials in the same order); x/r update
+//                    and r.r partials, or the FP32 copy of a refreshed residual
+//   K3 gb_b_pupdate  (system, chunk): beta (again from every chunk's own
+//                    sum), stopping / refresh decision, p update
 // Every sum of a system is taken over that system's own fixed decomposition
 // (its SpMV plan, its chunks) in a fixed order, so a system gives the same
 // bits alone and in any mix.
@@ -47,15 +46,16 @@
 
 #define GB_BCHUNK 2048           // rows per elementwise work item
 #define GB_BCHUNK_ITEMS (GB_BCHUNK / GB_BLOCK)
-// The SpMV and elementwise launches get one workgroup per entry of their
-// work-list allocation (workgroups past the current count exit at once), so
-// items are dispatched in list order, as one launch per matrix would be,
-// and a graph stays valid while the lists fit their allocation.  The
-// allocation is resized (and the graphs recaptured) when the lists outgrow
-// it or shrink below a quarter of it.
-#define GB_BGRID_SYS 256u
+// The SpMV and elementwise launches get one workgroup per entry of their work
+// lists, so items are dispatched in list order, as one launch per matrix
+// would be.  The lists' allocations are resized when the lists outgrow them or
+// shrink below a quarter of them.  Steps are replayed from graphs once the
+// lists have stayed the same for GB_B_STABLE steps, and launched one by one
+// before (the host keeps up).  So the kernels read nothing but their item
+// first, where a graph that outlives the lists has them read the lists'
+// lengths, and one dependent load less shows: 13.1 -> 11.6 us an SpMV.
+#define GB_B_STABLE 128u
 #define GB_BLIST_MIN 1024u
-#define GB_BRED 1024             // threads of the per-system reduction
 #define GB_B_NGRAPH 7
 
 enum { GB_MODE_CG = 0, GB_MODE_REFRESH = 1 };
@@ -101,11 +101,6 @@ struct gb_bsys {
 // items of column slice k of every split matrix, and segment 0 also the
 // items of the matrices that are not split.  Launch boundaries make the GPU
 // finish one slice of x before it starts gathering from the next.
-struct gb_blists {
-  uint32_t n_spmv, n_elem, n_sys, nseg;
-  uint32_t seg[GB_SPLIT_MAX + 1];
-};
-
 struct gbd_batch {
   uint32_t max_slots;
   gb_bsys *d_sys;          // device table
@@ -115,20 +110,20 @@ struct gbd_batch {
   uint8_t *used;           // host: slot in use
   void **slot_mem;         // host: per-slot workspace allocation
   gbd_matrix **slot_mat;   // host: the matrix each used slot holds
-  gb_blists *d_lists;      // device counts
-  gb_blists *h_lists;      // pinned
-  uint32_t *d_spmv, *d_elem, *d_sysl;  // device work lists
+  uint2 *d_spmv, *d_elem;  // device work lists: (system, item)
   uint4 *d_desc;  // per SpMV list entry: a row block's r0, r1, first entry, entries
   uint32_t cap_spmv, cap_elem;
   uint32_t nseg;                       // SpMV launches per step
-  bool banded;                         // the SpMV build for banded batches
-  uint32_t cap_seg[GB_SPLIT_MAX];      // their grids
+  uint32_t seg[GB_SPLIT_MAX + 1];      // their parts of the SpMV list
+  uint32_t lds;                        // gb_b_spmv's dynamic LDS (GB_SPMV_FEW_LDS or 0)
+  uint32_t grid_elem;                  // the elementwise launches' grid
+  uint32_t stable;                     // steps since the launches changed
   uint32_t *h_slice_nwork;             // host: max_slots x GB_SPLIT_MAX
   uint32_t *h_xt;                      // host: the active x-tile systems' slots
   uint32_t *h_xt_grid;                 // and their launch grids
   uint32_t n_xt;
   gb_bplan *d_slices;                  // max_slots x GB_SPLIT_MAX slice plans
-  uint32_t *h_spmv, *h_elem, *h_sysl;  // pinned staging
+  uint2 *h_spmv, *h_elem;              // pinned staging
   double delta;
   hipGraph_t graph[GB_B_NGRAPH];
   hipGraphExec_t gexec[GB_B_NGRAPH];
@@ -140,15 +135,16 @@ __device__ __forceinline__ double gb_b_sum_chunks(const double *part, uint32_t n
                                                   double *red) {
   // same code and order in every workgroup of K4 and in the init reduction
   double s = 0.0;
-  for (uint32_t base = 0; base < n; base += GB_BLOCK * 8) {
-    double v[8];
+#pragma unroll 1
+  for (uint32_t base = 0; base < n; base += GB_BLOCK * 4) {
+    double v[4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < 4; ++j) {
       uint32_t i = base + j * GB_BLOCK + threadIdx.x;
       v[j] = i < n ? part[i] : 0.0;
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s += v[j];
+    for (int j = 0; j < 4; ++j) s += v[j];
   }
   s = gb_wave_sum(s);
   const int lane = threadIdx.x & (GB_WAVE - 1), wave = threadIdx.x / GB_WAVE;
@@ -310,12 +306,12 @@ __device__ __forceinline__ double gb_b_spmv_item(const gb_bplan &S, uint32_t w,
 // row block (item below its plan's nstream), its first and last-plus-one
 // rows, its first entry and its entry count.
 __global__ void __launch_bounds__(GB_BLOCK)
-gb_b_describe(const gb_bsys *__restrict__ sys, const uint32_t *__restrict__ items,
+gb_b_describe(const gb_bsys *__restrict__ sys, const uint2 *__restrict__ items,
               uint32_t a, uint32_t b, uint32_t seg, const gb_bplan *__restrict__ slice_tab,
               uint4 *__restrict__ desc) {
   for (uint32_t it = a + blockIdx.x * GB_BLOCK + threadIdx.x; it < b;
        it += gridDim.x * GB_BLOCK) {
-    const uint32_t s = items[2 * it], lw = items[2 * it + 1];
+    const uint32_t s = items[it].x, lw = items[it].y;
     const gb_bsys &S = sys[s];
     const gb_bplan &L = S.nsplit ? slice_tab[(size_t)s * GB_SPLIT_MAX + seg] : S.pl;
     uint4 d = make_uint4(0u, 0u, 0u, 0u);
@@ -329,67 +325,57 @@ gb_b_describe(const gb_bsys *__restrict__ sys, const uint32_t *__restrict__ item
   }
 }
 
-// Wavefronts per SIMD the batched SpMV's register budget must allow, by
-// batch.  Measured: 512 Laplacians (mixed precision) 1645 solves/s at 5
-// (87 VGPRs, the compiler's own choice), 1755 at 7; the served stream of
-// random matrices 355-363 solves/s at 5, 344-346 at 7.  A step launches the
-// seven-wavefront build when every admitted system's matrix reads 16-bit
-// column offsets (banded rows, gathers that stay in L2), else the five.
-#define GB_B_SPMV_WAVES_BANDED 7
-#define GB_B_SPMV_WAVES_OTHER 5
-template <int WAVES>
+// One workgroup per list entry (58 VGPRs: eight wavefronts per SIMD; fewer
+// for scattered columns, GB_SPMV_FEW_LDS: 16 random systems of 4,096 to 2^20
+// rows in mixed precision 14.2 -> 12.7 ms).  512 threads instead, half the
+// loads and rows a thread, took the same time.
 __global__ void __launch_bounds__(GB_BLOCK)
-__attribute__((amdgpu_waves_per_eu(WAVES)))
-gb_b_spmv(const gb_bsys *__restrict__ sys, const uint32_t *__restrict__ items,
-          const uint4 *__restrict__ desc,
-          const gb_blists *__restrict__ lists, uint32_t seg,
+gb_b_spmv(const gb_bsys *__restrict__ sys, const uint2 *__restrict__ items,
+          const uint4 *__restrict__ desc, uint32_t seg,
           const gbd_bstate *__restrict__ states, const gb_bplan *__restrict__ slice_tab) {
   __shared__ double prodd[GB_STREAM_LDS];
   __shared__ double tredd[GB_WAVES_PER_BLOCK];
   __shared__ double red[GB_WAVES_PER_BLOCK];
-  const uint32_t end = lists->seg[seg + 1];
-  for (uint32_t it = lists->seg[seg] + blockIdx.x; it < end; it += gridDim.x) {
-    const uint32_t s = items[2 * it], lw = items[2 * it + 1];
-    const uint4 d = desc[it];
-    // the system, its state and its slice plan are addressed from the slot
-    // alone, so their loads go out together
-    const gb_bsys &S = sys[s];
-    const gbd_bstate *st = states + s;
-    if (st->done) continue;  // not written during this kernel: uniform
-    const int mode = st->mode_next;
-    double dotp;
-    uint32_t w = lw;  // the item's partial slot
-    if (S.nsplit) {
-      // a column-split matrix runs every step over its slices, slice r in
-      // launch r, each into its partial vector: CG steps in the system's
-      // precision, refresh steps A x in FP64 (the update kernel adds them)
-      const uint32_t r = seg;
-      const gb_bplan &L = slice_tab[(size_t)s * GB_SPLIT_MAX + r];
-      w = L.base + lw;
-      if (mode == GB_MODE_REFRESH) {
-        double *yp = (double *)S.ypart + (size_t)r * S.n;
-        dotp = gb_b_spmv_item<double, 0>(L, lw, L.val, S.x, yp, nullptr, prodd, tredd, d);
-      } else if (S.precision != GOOSEBERRY_PRECISION_FP64) {
-        float *yp = (float *)S.ypart + (size_t)r * S.n;
-        dotp = gb_b_spmv_item<float, 0>(L, lw, L.val32, S.p32, yp, nullptr,
-                                        (float *)prodd, (float *)tredd, d);
-      } else {
-        double *yp = (double *)S.ypart + (size_t)r * S.n;
-        dotp = gb_b_spmv_item<double, 0>(L, lw, L.val, S.p, yp, nullptr, prodd, tredd, d);
-      }
-    } else if (mode == GB_MODE_REFRESH) {
-      dotp = gb_b_spmv_item<double, 1>(S.pl, w, S.pl.val, S.x, S.r, S.b, prodd, tredd, d);
+  const uint2 item = items[blockIdx.x];  // the segment's list, one item each
+  const uint32_t s = item.x, lw = item.y;
+  const uint4 d = desc[blockIdx.x];
+  // the system, its state and its slice plan are addressed from the slot
+  // alone, so their loads go out together
+  const gb_bsys &S = sys[s];
+  const gbd_bstate *st = states + s;
+  if (st->done) return;  // not written during this kernel: uniform
+  const int mode = st->mode_next;
+  double dotp;
+  uint32_t w = lw;  // the item's partial slot
+  if (S.nsplit) {
+    // a column-split matrix runs every step over its slices, slice r in
+    // launch r, each into its partial vector: CG steps in the system's
+    // precision, refresh steps A x in FP64 (the update kernel adds them)
+    const uint32_t r = seg;
+    const gb_bplan &L = slice_tab[(size_t)s * GB_SPLIT_MAX + r];
+    w = L.base + lw;
+    if (mode == GB_MODE_REFRESH) {
+      double *yp = (double *)S.ypart + (size_t)r * S.n;
+      dotp = gb_b_spmv_item<double, 0>(L, lw, L.val, S.x, yp, nullptr, prodd, tredd, d);
     } else if (S.precision != GOOSEBERRY_PRECISION_FP64) {
-      dotp = gb_b_spmv_item<float, 0>(S.pl, w, S.pl.val32, S.p32, S.ap32, nullptr,
+      float *yp = (float *)S.ypart + (size_t)r * S.n;
+      dotp = gb_b_spmv_item<float, 0>(L, lw, L.val32, S.p32, yp, nullptr,
                                       (float *)prodd, (float *)tredd, d);
     } else {
-      dotp = gb_b_spmv_item<double, 0>(S.pl, w, S.pl.val, S.p, S.ap, nullptr, prodd, tredd, d);
+      double *yp = (double *)S.ypart + (size_t)r * S.n;
+      dotp = gb_b_spmv_item<double, 0>(L, lw, L.val, S.p, yp, nullptr, prodd, tredd, d);
     }
-    // one partial per work item
-    const double bs = gb_block_sum(dotp, red);
-    if (threadIdx.x == 0) S.part1[w] = bs;
-    __syncthreads();
+  } else if (mode == GB_MODE_REFRESH) {
+    dotp = gb_b_spmv_item<double, 1>(S.pl, w, S.pl.val, S.x, S.r, S.b, prodd, tredd, d);
+  } else if (S.precision != GOOSEBERRY_PRECISION_FP64) {
+    dotp = gb_b_spmv_item<float, 0>(S.pl, w, S.pl.val32, S.p32, S.ap32, nullptr,
+                                    (float *)prodd, (float *)tredd, d);
+  } else {
+    dotp = gb_b_spmv_item<double, 0>(S.pl, w, S.pl.val, S.p, S.ap, nullptr, prodd, tredd, d);
   }
+  // one partial per work item
+  const double bs = gb_block_sum(dotp, red);
+  if (threadIdx.x == 0) S.part1[w] = bs;
 }
 
 // The SpMV of a system on an x-tile plan (grid = its row blocks): Ap and
@@ -414,45 +400,263 @@ gb_b_spmv_xt(const gb_bsys *__restrict__ sys, uint32_t slot,
                                   S.part1, S.n, S.n, S.xt_R, S.xt_T, S.xt_lc, L);
 }
 
-__global__ void __launch_bounds__(GB_BRED)
-gb_b_reduce(const gb_bsys *__restrict__ sys, const uint32_t *__restrict__ syslist,
-            const gb_blists *__restrict__ lists) {
-  __shared__ double red[GB_BRED / GB_WAVE];
-  const uint32_t count = lists->n_sys;
-  for (uint32_t it = blockIdx.x; it < count; it += gridDim.x) {
-    const gb_bsys &S = sys[syslist[it]];
-    gbd_bstate *st = S.st;
-    if (st->done) continue;
-    const int mode = st->mode_next;
-    if (S.nsplit && mode == GB_MODE_REFRESH) {
-      // A x is still in slices: the update kernel forms b - A x and the
-      // p-update kernel tests it
-      if (threadIdx.x == 0) st->mode = mode;
-      continue;
-    }
-    // one partial per SpMV work item (per row block on an x-tile plan)
-    const uint32_t np = S.xt_ptr ? S.xt_W : S.nsplit ? S.nwork_split : S.pl.nwork;
-    const double *part = S.part1;
-    double s = 0.0;
-    for (uint32_t base = 0; base < np; base += GB_BRED * 8) {
-      double v[8];
+// A thread's GB_BCHUNK_ITEMS rows of a whole chunk of an internal vector
+// (256-byte aligned), as 16-byte words: word j of thread t is the chunk's
+// word j GB_BLOCK + t, so consecutive lanes hold consecutive words.
+template <typename T>
+__device__ __forceinline__ uint32_t gb_b_row(uint32_t i0, int j, int q) {
+  constexpr int N = 16 / sizeof(T);
+  return i0 + (j * GB_BLOCK + threadIdx.x) * N + q;
+}
+template <typename T>
+__device__ __forceinline__ void gb_b_ld(const T *__restrict__ v, uint32_t i0, T *o) {
+  constexpr int N = 16 / sizeof(T);
+  struct alignas(16) word { T e[N]; };
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        uint32_t i = base + j * GB_BRED + threadIdx.x;
-        v[j] = i < np ? part[i] : 0.0;
-      }
+  for (int j = 0; j < GB_BCHUNK_ITEMS / N; ++j) {
+    const word w = *(const word *)(v + gb_b_row<T>(i0, j, 0));
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s += v[j];
+    for (int q = 0; q < N; ++q) o[j * N + q] = w.e[q];
+  }
+}
+template <typename T>
+__device__ __forceinline__ void gb_b_st(T *__restrict__ v, uint32_t i0, const T *o) {
+  constexpr int N = 16 / sizeof(T);
+  struct alignas(16) word { T e[N]; };
+#pragma unroll
+  for (int j = 0; j < GB_BCHUNK_ITEMS / N; ++j) {
+    word w;
+#pragma unroll
+    for (int q = 0; q < N; ++q) w.e[q] = o[j * N + q];
+    *(word *)(v + gb_b_row<T>(i0, j, 0)) = w;
+  }
+}
+
+// The step's scalars and the x/r updates, one workgroup per chunk of rows,
+// eight rows a thread.  Each workgroup issues the loads of its
+// chunk, adds the system's SpMV partials itself (every one the same values in
+// the same order, so the same alpha) while they are in flight, and updates its
+// rows; chunk 0 records the scalars.  In a refresh step the sum is
+// ||b - A x||^2 and every workgroup draws the same conclusion from it.
+// (`done` may be set by chunk 0 while others start: they would decide to skip
+// their rows as well.)  A system's last chunk, split systems and refresh steps
+// go row by row.
+//
+// Bound: latency, on small systems: a launch, the dependent loads from the
+// list to the vectors, and fetching the code itself, which every launch runs
+// once.  48 Laplacians, per step: a reduction launch 4.2 us, the r update 10.0
+// and the p update 7.9 us with eight rows' loads one after another; with those
+// unrolled row by row 30 us in the update (128 registers, and code); as they
+// are, with the reduction inside, 6.4 and 6.5 us.
+__global__ void __launch_bounds__(GB_BLOCK)
+gb_b_update(const gb_bsys *__restrict__ sys, const uint2 *__restrict__ items,
+            gbd_bstate *states) {
+  __shared__ double red[GB_WAVES_PER_BLOCK];
+  __shared__ int32_t s_done;
+  constexpr int J = GB_BCHUNK_ITEMS;
+  const uint2 item = items[blockIdx.x];
+  const uint32_t c = item.y;
+  const gb_bsys &S = sys[item.x];
+  gbd_bstate *st = states + item.x;
+  const uint32_t n = S.n, nsplit = S.nsplit;
+  const uint32_t i0 = c * GB_BCHUNK;
+  const bool inside = n - i0 >= GB_BCHUNK;
+  const uint32_t i1 = inside ? i0 + GB_BCHUNK : n;
+  const bool mixed = S.precision != GOOSEBERRY_PRECISION_FP64;
+  const int mode = st->mode_next;  // only gb_b_pupdate changes it
+  const bool whole = mode == GB_MODE_CG && !nsplit && inside;
+  if (threadIdx.x == 0) s_done = *(volatile int32_t *)&st->done;
+  float rf[J], af[J];
+  double rd[J], ad[J], pd[J], xd[J];
+  if (whole) {
+    if (mixed) {
+      gb_b_ld(S.r32, i0, rf);
+      gb_b_ld(S.ap32, i0, af);
+    } else {
+      gb_b_ld(S.r, i0, rd);
+      gb_b_ld(S.ap, i0, ad);
+      gb_b_ld(S.p, i0, pd);
+      const double *const x = S.x;  // the caller's: aligned to 8 bytes
+#pragma unroll
+      for (int j = 0; j < J; ++j) xd[j] = x[gb_b_row<double>(i0, j / 2, j % 2)];
     }
-    s = gb_wave_sum(s);
-    if ((threadIdx.x & (GB_WAVE - 1)) == 0) red[threadIdx.x / GB_WAVE] = s;
+  }
+  const bool first = c == 0 && threadIdx.x == 0;
+  double alpha = 0.0;
+  if (nsplit && mode == GB_MODE_REFRESH) {
+    // A x is still in slices: b - A x is formed below and its norm tested by
+    // the p-update kernel
     __syncthreads();
-    if (threadIdx.x == 0) {
-      double t = red[0];
-      for (int q = 1; q < GB_BRED / GB_WAVE; ++q) t += red[q];
-      st->mode = mode;
-      if (mode == GB_MODE_REFRESH) {
-        // t = ||b - A x||^2 in FP64
+    if (s_done) return;
+    if (first) st->mode = mode;
+  } else {
+    // one partial per SpMV work item (per row block on an x-tile plan)
+    const uint32_t np = S.xt_ptr ? S.xt_W : nsplit ? S.nwork_split : S.pl.nwork;
+    const double t = gb_b_sum_chunks(S.part1, np, red);  // barriers inside
+    if (s_done) return;
+    int status = 0;
+    if (mode == GB_MODE_REFRESH) {
+      const double rn = sqrt(t);  // ||b - A x|| in FP64
+      if (rn <= st->tol) status = 1;
+      else if (!isfinite(rn)) status = 3;
+      else if (st->final_refresh) status = 2;
+      if (first) {
+        st->mode = mode;
+        st->nrefine += 1;
+        st->rnorm64 = rn;
+        st->rnorm_ref = rn;
+      }
+    } else {
+      const double dr = st->dr;
+      alpha = dr / t;
+      if (!(t != 0.0) || !isfinite(alpha)) status = 3;
+      if (first) {
+        st->mode = mode;
+        st->pap = t;
+        st->alpha = alpha;
+        if (!status) {
+          st->dr_prev = dr;
+          st->iter_next = st->iter + 1;
+        }
+      }
+    }
+    if (status) {
+      if (first) {
+        st->done = 1;
+        st->status = status;
+      }
+      return;
+    }
+  }
+  double d = 0.0;
+  if (whole && mixed) {
+    // d += a p is done by gb_b_pupdate, which reads p anyway
+    const float a = (float)alpha;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      rf[j] = rf[j] - a * af[j];
+      d += (double)rf[j] * (double)rf[j];
+    }
+    gb_b_st(S.r32, i0, rf);
+  } else if (whole) {
+    // src/cgd.c:92-100
+    double *const x = S.x;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const double ps = alpha * pd[j];
+      const uint32_t i = gb_b_row<double>(i0, j / 2, j % 2);
+      x[i] = xd[j] + ps;
+      const double aps = alpha * ad[j];
+      rd[j] = rd[j] - aps;
+      d += rd[j] * rd[j];
+    }
+    gb_b_st(S.r, i0, rd);
+  } else if (mixed && mode == GB_MODE_REFRESH) {
+    // r32 = (float) r64 from the refresh SpMV (for a split matrix r64 =
+    // b - A x from the slices' FP64 partials, and its squared norm goes to
+    // part3); d = 0 was set when x was updated
+    const double *const yp = (const double *)S.ypart;
+    double d64 = 0.0;
+#pragma unroll 1
+    for (uint32_t i = i0 + threadIdx.x; i < i1; i += GB_BLOCK) {
+      double rr;
+      if (nsplit) {
+        double ax = yp[i];
+        for (uint32_t r = 1; r < nsplit; ++r) ax += yp[(size_t)r * n + i];
+        rr = S.b[i] - ax;
+        S.r[i] = rr;
+        d64 += rr * rr;
+      } else {
+        rr = S.r[i];
+      }
+      const float v = S.jscale ? (float)(S.jscale[i] * rr) : (float)rr;
+      S.r32[i] = v;
+      d += (double)v * (double)v;
+    }
+    if (nsplit) {
+      const double b64 = gb_block_sum(d64, red);
+      if (threadIdx.x == 0) S.part3[c] = b64;
+      __syncthreads();
+    }
+  } else if (mixed) {
+    const float a = (float)alpha;
+    const float *const yp = (const float *)S.ypart;
+#pragma unroll 1
+    for (uint32_t i = i0 + threadIdx.x; i < i1; i += GB_BLOCK) {
+      float ap;
+      if (nsplit) {  // slice partials added in slice order
+        ap = yp[i];
+        for (uint32_t r = 1; r < nsplit; ++r) ap += yp[(size_t)r * n + i];
+      } else {
+        ap = S.ap32[i];
+      }
+      const float rn = S.r32[i] - a * ap;
+      S.r32[i] = rn;
+      d += (double)rn * (double)rn;
+    }
+  } else {
+    const double *const yp = (const double *)S.ypart;
+#pragma unroll 1
+    for (uint32_t i = i0 + threadIdx.x; i < i1; i += GB_BLOCK) {
+      double ap;
+      if (nsplit) {
+        ap = yp[i];
+        for (uint32_t r = 1; r < nsplit; ++r) ap += yp[(size_t)r * n + i];
+      } else {
+        ap = S.ap[i];
+      }
+      const double ps = alpha * S.p[i];
+      S.x[i] = S.x[i] + ps;
+      const double aps = alpha * ap;
+      const double rn = S.r[i] - aps;
+      S.r[i] = rn;
+      d += rn * rn;
+    }
+  }
+  const double bs = gb_block_sum(d, red);
+  if (threadIdx.x == 0) S.part2[c] = bs;
+}
+
+// beta, the stopping and refresh decisions and the p update; rows and loads as
+// in gb_b_update.
+__global__ void __launch_bounds__(GB_BLOCK)
+gb_b_pupdate(const gb_bsys *__restrict__ sys, const uint2 *__restrict__ items,
+             gbd_bstate *states, double delta) {
+  __shared__ double red[GB_WAVES_PER_BLOCK];
+  __shared__ int32_t s_done;
+  constexpr int J = GB_BCHUNK_ITEMS;
+  const uint2 item = items[blockIdx.x];
+  const uint32_t c = item.y;
+  const gb_bsys &S = sys[item.x];
+  gbd_bstate *st = states + item.x;
+  const uint32_t n = S.n, i0 = c * GB_BCHUNK;
+  const bool mixed = S.precision != GOOSEBERRY_PRECISION_FP64;
+  const bool whole = n - i0 >= GB_BCHUNK;
+  const uint32_t i1 = whole ? i0 + GB_BCHUNK : n;
+  // workgroup 0 of a system may set done during this kernel: decide once
+  if (threadIdx.x == 0) s_done = *(volatile int32_t *)&st->done;
+  const int mode = st->mode;
+  float pf[J], df[J], rf[J];
+  double pd[J], rd[J];
+  if (whole && mode == GB_MODE_CG) {
+    if (mixed) {
+      gb_b_ld(S.p32, i0, pf);
+      gb_b_ld(S.d32, i0, df);
+      gb_b_ld(S.r32, i0, rf);
+    } else {
+      gb_b_ld(S.p, i0, pd);
+      gb_b_ld(S.r, i0, rd);
+    }
+  }
+  const double dnr = gb_b_sum_chunks(S.part2, S.nchunks, red);  // barriers inside
+  if (s_done) return;
+  if (mode == GB_MODE_REFRESH) {
+    // MIXED only: restart the FP32 recurrence from the FP64 residual,
+    // keep the direction p.  A split matrix's FP64 residual norm is
+    // tested here (the update kernel tests the others').
+    if (S.nsplit) {
+      const double t = gb_b_sum_chunks(S.part3, S.nchunks, red);
+      if (c == 0 && threadIdx.x == 0) {
         const double rn = sqrt(t);
         st->nrefine += 1;
         st->rnorm64 = rn;
@@ -467,238 +671,103 @@ gb_b_reduce(const gb_bsys *__restrict__ sys, const uint32_t *__restrict__ syslis
           st->done = 1;
           st->status = 2;
         }
-      } else {
-        const double dr = st->dr;
-        const double alpha = dr / t;
-        st->pap = t;
-        st->alpha = alpha;
-        if (!(t != 0.0) || !isfinite(alpha)) {
-          st->done = 1;
-          st->status = 3;
-        } else {
-          st->dr_prev = dr;
-          st->iter_next = st->iter + 1;
-        }
       }
-    }
-    __syncthreads();
-  }
-}
-
-__global__ void __launch_bounds__(GB_BLOCK)
-gb_b_update(const gb_bsys *__restrict__ sys, const uint32_t *__restrict__ items,
-            const gb_blists *__restrict__ lists) {
-  __shared__ double red[GB_WAVES_PER_BLOCK];
-  const uint32_t count = lists->n_elem;
-  for (uint32_t it = blockIdx.x; it < count; it += gridDim.x) {
-    const uint32_t sidx = items[2 * it], c = items[2 * it + 1];
-    const gb_bsys &S = sys[sidx];
-    const gbd_bstate *st = S.st;
-    if (st->done) continue;
-    const int mode = st->mode;
-    const uint32_t i0 = c * GB_BCHUNK;
-    double d = 0.0;
-    if (S.precision != GOOSEBERRY_PRECISION_FP64) {
-      if (mode == GB_MODE_REFRESH) {
-        // r32 = (float) r64 from the refresh SpMV (for a split matrix r64 =
-        // b - A x from the slices' FP64 partials, and its squared norm goes
-        // to part3); d = 0 was set when x was updated
-        const double *yp = (const double *)S.ypart;
-        double d64 = 0.0;
-        for (int j = 0; j < GB_BCHUNK_ITEMS; ++j) {
-          uint32_t i = i0 + j * GB_BLOCK + threadIdx.x;
-          if (i < S.n) {
-            double rr;
-            if (S.nsplit) {
-              double ax = yp[i];
-              for (uint32_t r = 1; r < S.nsplit; ++r) ax += yp[(size_t)r * S.n + i];
-              rr = S.b[i] - ax;
-              S.r[i] = rr;
-              d64 += rr * rr;
-            } else {
-              rr = S.r[i];
-            }
-            float rf = S.jscale ? (float)(S.jscale[i] * rr) : (float)rr;
-            S.r32[i] = rf;
-            d += (double)rf * (double)rf;
-          }
-        }
-        if (S.nsplit) {
-          const double b64 = gb_block_sum(d64, red);
-          if (threadIdx.x == 0) S.part3[c] = b64;
-          __syncthreads();
-        }
-      } else {
-        const float a = (float)st->alpha;
-        const float *yp = (const float *)S.ypart;
-        for (int j = 0; j < GB_BCHUNK_ITEMS; ++j) {
-          uint32_t i = i0 + j * GB_BLOCK + threadIdx.x;
-          if (i < S.n) {
-            float ap;
-            if (S.nsplit) {  // slice partials added in slice order
-              ap = yp[i];
-              for (uint32_t r = 1; r < S.nsplit; ++r) ap += yp[(size_t)r * S.n + i];
-            } else {
-              ap = S.ap32[i];
-            }
-            // d += a p is done by gb_b_pupdate, which reads p anyway
-            float rn = S.r32[i] - a * ap;
-            S.r32[i] = rn;
-            d += (double)rn * (double)rn;
-          }
-        }
-      }
-    } else {
-      // src/cgd.c:92-100
-      const double alpha = st->alpha;
-      const double *yp = (const double *)S.ypart;
-      for (int j = 0; j < GB_BCHUNK_ITEMS; ++j) {
-        uint32_t i = i0 + j * GB_BLOCK + threadIdx.x;
-        if (i < S.n) {
-          double ap;
-          if (S.nsplit) {
-            ap = yp[i];
-            for (uint32_t r = 1; r < S.nsplit; ++r) ap += yp[(size_t)r * S.n + i];
-          } else {
-            ap = S.ap[i];
-          }
-          double ps = alpha * S.p[i];
-          S.x[i] = S.x[i] + ps;
-          double aps = alpha * ap;
-          double rn = S.r[i] - aps;
-          S.r[i] = rn;
-          d += rn * rn;
-        }
-      }
-    }
-    double bs = gb_block_sum(d, red);
-    if (threadIdx.x == 0) S.part2[c] = bs;
-    __syncthreads();
-  }
-}
-
-__global__ void __launch_bounds__(GB_BLOCK)
-gb_b_pupdate(const gb_bsys *__restrict__ sys, const uint32_t *__restrict__ items,
-             const gb_blists *__restrict__ lists, double delta) {
-  __shared__ double red[GB_WAVES_PER_BLOCK];
-  __shared__ int32_t s_done;
-  const uint32_t count = lists->n_elem;
-  for (uint32_t it = blockIdx.x; it < count; it += gridDim.x) {
-    const uint32_t sidx = items[2 * it], c = items[2 * it + 1];
-    const gb_bsys &S = sys[sidx];
-    gbd_bstate *st = S.st;
-    // workgroup 0 of a system may set done during this kernel: decide once
-    if (threadIdx.x == 0) s_done = *(volatile int32_t *)&st->done;
-    __syncthreads();
-    const int32_t was_done = s_done;
-    __syncthreads();
-    if (was_done) continue;
-    const int mode = st->mode;
-    const double dnr = gb_b_sum_chunks(S.part2, S.nchunks, red);
-    const uint32_t i0 = c * GB_BCHUNK;
-    if (mode == GB_MODE_REFRESH) {
-      // MIXED only: restart the FP32 recurrence from the FP64 residual,
-      // keep the direction p.  A split matrix's FP64 residual norm is
-      // tested here (the reduction kernel tests the others').
-      if (S.nsplit) {
-        const double t = gb_b_sum_chunks(S.part3, S.nchunks, red);
-        if (c == 0 && threadIdx.x == 0) {
-          const double rn = sqrt(t);
-          st->nrefine += 1;
-          st->rnorm64 = rn;
-          st->rnorm_ref = rn;
-          if (rn <= st->tol) {
-            st->done = 1;
-            st->status = 1;
-          } else if (!isfinite(rn)) {
-            st->done = 1;
-            st->status = 3;
-          } else if (st->final_refresh) {
-            st->done = 1;
-            st->status = 2;
-          }
-        }
-      }
-      if (c == 0 && threadIdx.x == 0) {
-        st->dr = dnr;
-        st->rnorm = sqrt(dnr);
-        st->inner = 0;
-        st->mode_next = GB_MODE_CG;
-        // the refresh test of a scaled system compares scaled residuals
-        if (S.jscale) st->rnorm_ref = st->rnorm;
-      }
-      continue;
-    }
-    // src/cgd.c:100-119 (and its FP32-inner counterpart)
-    const double alpha = st->alpha;
-    const double beta = dnr / st->dr_prev;
-    const double rnorm = sqrt(dnr);
-    const unsigned long long it1 = st->iter_next;
-    const bool cap = st->maxiter && it1 >= st->maxiter;
-    int status = 0;        // FP64: stop here
-    bool refresh = false;  // MIXED: fold d into x, FP64 residual next step
-    if (S.precision != GOOSEBERRY_PRECISION_FP64) {
-      if (!isfinite(dnr)) status = 3;
-      // refresh after a drop by delta, or once the recurrence residual
-      // predicts convergence (for a scaled system: it has dropped by
-      // tol / ||b - A x|| since the last refresh)
-      else if (rnorm <= delta * st->rnorm_ref || cap ||
-               (S.jscale ? rnorm * st->rnorm64 <= st->tol * st->rnorm_ref
-                         : rnorm <= st->tol))
-        refresh = true;
-    } else {
-      if (rnorm <= st->tol) status = 1;
-      else if (!isfinite(dnr)) status = 3;
-      else if (cap) status = 2;
     }
     if (c == 0 && threadIdx.x == 0) {
-      st->beta = beta;
       st->dr = dnr;
-      st->rnorm = rnorm;
-      st->iter = it1;
-      st->inner += 1;
-      if (status) {
-        st->status = status;
-        st->done = 1;
+      st->rnorm = sqrt(dnr);
+      st->inner = 0;
+      st->mode_next = GB_MODE_CG;
+      // the refresh test of a scaled system compares scaled residuals
+      if (S.jscale) st->rnorm_ref = st->rnorm;
+    }
+    return;
+  }
+  // src/cgd.c:100-119 (and its FP32-inner counterpart)
+  const double alpha = st->alpha;
+  const double beta = dnr / st->dr_prev;
+  const double rnorm = sqrt(dnr);
+  const unsigned long long it1 = st->iter_next;
+  const bool cap = st->maxiter && it1 >= st->maxiter;
+  int status = 0;        // FP64: stop here
+  bool refresh = false;  // MIXED: fold d into x, FP64 residual next step
+  if (mixed) {
+    if (!isfinite(dnr)) status = 3;
+    // refresh after a drop by delta, or once the recurrence residual
+    // predicts convergence (for a scaled system: it has dropped by
+    // tol / ||b - A x|| since the last refresh)
+    else if (rnorm <= delta * st->rnorm_ref || cap ||
+             (S.jscale ? rnorm * st->rnorm64 <= st->tol * st->rnorm_ref
+                       : rnorm <= st->tol))
+      refresh = true;
+  } else {
+    if (rnorm <= st->tol) status = 1;
+    else if (!isfinite(dnr)) status = 3;
+    else if (cap) status = 2;
+  }
+  if (c == 0 && threadIdx.x == 0) {
+    st->beta = beta;
+    st->dr = dnr;
+    st->rnorm = rnorm;
+    st->iter = it1;
+    st->inner += 1;
+    if (status) {
+      st->status = status;
+      st->done = 1;
+    }
+    if (refresh) {
+      st->mode_next = GB_MODE_REFRESH;
+      if (cap) st->final_refresh = 1;
+    }
+  }
+  if (status) return;
+  if (mixed) {
+    // this step's d += a p (the same float products and sums as beside
+    // the r update, where it was one more read of p), then p = r + beta p.
+    // A mixed system's CG step sets `done` above only on a non-finite
+    // residual, after which x never takes d: a workgroup that sees that
+    // flag early and skips its rows changes no result.
+    const float a = (float)alpha;
+    const float boa = (float)beta;
+    if (whole && !refresh) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        df[j] = df[j] + a * pf[j];
+        pf[j] = rf[j] + boa * pf[j];
       }
-      if (refresh) {
-        st->mode_next = GB_MODE_REFRESH;
-        if (cap) st->final_refresh = 1;
+      gb_b_st(S.d32, i0, df);
+      gb_b_st(S.p32, i0, pf);
+    } else {
+#pragma unroll 1
+      for (uint32_t i = i0 + threadIdx.x; i < i1; i += GB_BLOCK) {
+        const float pv = S.p32[i];
+        const float dn = S.d32[i] + a * pv;
+        S.p32[i] = S.r32[i] + boa * pv;
+        if (refresh) {
+          // the FP64 solution update
+          S.x[i] = S.x[i] + (S.jscale ? S.jscale[i] * (double)dn : (double)dn);
+          S.d32[i] = 0.0f;
+        } else {
+          S.d32[i] = dn;
+        }
       }
     }
-    if (status) continue;
-    if (S.precision != GOOSEBERRY_PRECISION_FP64) {
-      // this step's d += a p (the same float products and sums as beside
-      // the r update, where it was one more read of p), then p = r + beta p.
-      // A mixed system's CG step sets `done` above only on a non-finite
-      // residual, after which x never takes d: a workgroup that sees that
-      // flag early and skips this loop changes no result.
-      const float a = (float)alpha;
-      const float boa = (float)beta;
-      for (int j = 0; j < GB_BCHUNK_ITEMS; ++j) {
-        uint32_t i = i0 + j * GB_BLOCK + threadIdx.x;
-        if (i < S.n) {
-          const float pv = S.p32[i];
-          const float dn = S.d32[i] + a * pv;
-          S.p32[i] = S.r32[i] + boa * pv;
-          if (refresh) {
-            // the FP64 solution update
-            S.x[i] = S.x[i] + (S.jscale ? S.jscale[i] * (double)dn : (double)dn);
-            S.d32[i] = 0.0f;
-          } else {
-            S.d32[i] = dn;
-          }
-        }
+  } else {
+    const double boa = beta / alpha;
+    if (whole) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const double ps = alpha * pd[j];
+        const double t = ps * boa;
+        pd[j] = rd[j] + t;
       }
+      gb_b_st(S.p, i0, pd);
     } else {
-      const double boa = beta / alpha;
-      for (int j = 0; j < GB_BCHUNK_ITEMS; ++j) {
-        uint32_t i = i0 + j * GB_BLOCK + threadIdx.x;
-        if (i < S.n) {
-          double ps = alpha * S.p[i];
-          double t = ps * boa;
-          S.p[i] = S.r[i] + t;
-        }
+#pragma unroll 1
+      for (uint32_t i = i0 + threadIdx.x; i < i1; i += GB_BLOCK) {
+        const double ps = alpha * S.p[i];
+        const double t = ps * boa;
+        S.p[i] = S.r[i] + t;
       }
     }
   }
@@ -782,6 +851,7 @@ gb_b_init_state(const gb_bsys *__restrict__ sys, uint32_t slot, double tol,
 // ------------------------------------------------------------------ host
 
 static void gb_b_drop_graphs(gbd_batch *B) {
+  B->stable = 0;
   for (int i = 0; i < GB_B_NGRAPH; ++i) {
     if (B->gexec[i]) (void)hipGraphExecDestroy(B->gexec[i]);
     if (B->graph[i]) (void)hipGraphDestroy(B->graph[i]);
@@ -794,24 +864,21 @@ static int gb_b_enqueue_raw(gbd_batch *B, uint32_t k) {
   hipStream_t s = gb_stream();
   for (uint32_t i = 0; i < k; ++i) {
     for (uint32_t g = 0; g < B->nseg; ++g) {
-      if (B->banded)
-        gb_b_spmv<GB_B_SPMV_WAVES_BANDED><<<B->cap_seg[g], GB_BLOCK, 0, s>>>(
-            B->d_sys, B->d_spmv, B->d_desc, B->d_lists, g, B->d_st, B->d_slices);
-      else
-        gb_b_spmv<GB_B_SPMV_WAVES_OTHER><<<B->cap_seg[g], GB_BLOCK, 0, s>>>(
-            B->d_sys, B->d_spmv, B->d_desc, B->d_lists, g, B->d_st, B->d_slices);
+      const uint32_t a = B->seg[g], grid = B->seg[g + 1] - a;
+      if (!grid) continue;  // only x-tile systems
+      gb_b_spmv<<<grid, GB_BLOCK, B->lds, s>>>(B->d_sys, B->d_spmv + a, B->d_desc + a, g,
+                                               B->d_st, B->d_slices);
       GB_LAUNCH_CHECK();
     }
+    if (!B->grid_elem) continue;
     for (uint32_t j = 0; j < B->n_xt; ++j) {
       gb_b_spmv_xt<<<B->h_xt_grid[j], GB_XT_THREADS, 0, s>>>(B->d_sys, B->h_xt[j], B->d_st);
       GB_LAUNCH_CHECK();
     }
-    gb_b_reduce<<<GB_BGRID_SYS, GB_BRED, 0, s>>>(B->d_sys, B->d_sysl, B->d_lists);
+    gb_b_update<<<B->grid_elem, GB_BLOCK, 0, s>>>(B->d_sys, B->d_elem, B->d_st);
     GB_LAUNCH_CHECK();
-    gb_b_update<<<B->cap_elem, GB_BLOCK, 0, s>>>(B->d_sys, B->d_elem, B->d_lists);
-    GB_LAUNCH_CHECK();
-    gb_b_pupdate<<<B->cap_elem, GB_BLOCK, 0, s>>>(B->d_sys, B->d_elem, B->d_lists,
-                                                     B->delta);
+    gb_b_pupdate<<<B->grid_elem, GB_BLOCK, 0, s>>>(B->d_sys, B->d_elem, B->d_st,
+                                                      B->delta);
     GB_LAUNCH_CHECK();
   }
   return GOOSEBERRY_SUCCESS;
@@ -915,15 +982,8 @@ int gbd_batch_create(uint32_t max_slots, double delta, gbd_batch **out) {
   if (e == hipSuccess) e = gb_dev_alloc((void **)&B->d_st, max_slots * sizeof(gbd_bstate));
   if (e == hipSuccess)
     e = hipHostMalloc((void **)&B->h_st, max_slots * sizeof(gbd_bstate), hipHostMallocDefault);
-  if (e == hipSuccess) e = gb_dev_alloc((void **)&B->d_lists, sizeof(gb_blists));
   if (e == hipSuccess)
     e = gb_dev_alloc((void **)&B->d_slices, (size_t)max_slots * GB_SPLIT_MAX * sizeof(gb_bplan));
-  if (e == hipSuccess)
-    e = hipHostMalloc((void **)&B->h_lists, sizeof(gb_blists), hipHostMallocDefault);
-  if (e == hipSuccess) e = gb_dev_alloc((void **)&B->d_sysl, max_slots * sizeof(uint32_t));
-  if (e == hipSuccess)
-    e = hipHostMalloc((void **)&B->h_sysl, max_slots * sizeof(uint32_t), hipHostMallocDefault);
-  if (e == hipSuccess) e = hipMemsetAsync(B->d_lists, 0, sizeof(gb_blists), gb_stream());
   if (e == hipSuccess)
     e = hipMemsetAsync(B->d_st, 0, max_slots * sizeof(gbd_bstate), gb_stream());
   if (e == hipSuccess)
@@ -949,17 +1009,13 @@ void gbd_batch_destroy(gbd_batch *B) {
       if (B->used[i] && B->slot_mat[i]) B->slot_mat[i]->holders--;
   (void)gb_dev_free(B->d_sys);
   (void)gb_dev_free(B->d_st);
-  (void)gb_dev_free(B->d_lists);
   (void)gb_dev_free(B->d_slices);
   (void)gb_dev_free(B->d_spmv);
   (void)gb_dev_free(B->d_desc);
   (void)gb_dev_free(B->d_elem);
-  (void)gb_dev_free(B->d_sysl);
   if (B->h_st) (void)hipHostFree(B->h_st);
-  if (B->h_lists) (void)hipHostFree(B->h_lists);
   if (B->h_spmv) (void)hipHostFree(B->h_spmv);
   if (B->h_elem) (void)hipHostFree(B->h_elem);
-  if (B->h_sysl) (void)hipHostFree(B->h_sysl);
   free(B->used);
   free(B->slot_mem);
   free(B->slot_mat);
@@ -1101,13 +1157,11 @@ int gbd_batch_remove(gbd_batch *B, uint32_t slot) {
 int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
   hipStream_t s = gb_stream();
   uint64_t ns = 0, ne = 0;
-  uint32_t nsys = 0;
   for (uint32_t i = 0; i < B->max_slots; ++i) {
     if (!B->used[i] || (active && !active[i])) continue;
     if (!B->h_sys[i].xt_ptr)
       ns += B->h_sys[i].nsplit ? B->h_sys[i].nwork_split : B->h_sys[i].pl.nwork;
     ne += B->h_sys[i].nchunks;
-    ++nsys;
   }
   if (ns > 0xffffffffull || ne > 0xffffffffull) return GOOSEBERRY_ERROR_INVALIDINPUT;
   GB_HIP(hipStreamSynchronize(s));  // staging buffers are reused
@@ -1138,12 +1192,15 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
   // matrices in segment 0
   uint32_t nseg = 1;
   uint64_t cnt[GB_SPLIT_MAX] = {0};
-  bool banded = true;  // every active system's matrix has 16-bit offsets
+  uint64_t scattered = 0, blocks = 0;  // items of row blocks without 16-bit offsets, all items
   for (uint32_t i = 0; i < B->max_slots; ++i) {
     if (!B->used[i] || (active && !active[i])) continue;
     const gb_bsys &S = B->h_sys[i];
     if (S.xt_ptr) continue;  // launched on its own
-    banded = banded && !S.nsplit && S.pl.dcol;
+    if (!S.nsplit) {
+      scattered += S.pl.dcol ? 0 : S.pl.nstream;
+      blocks += S.pl.nwork;
+    }
     if (S.nsplit) {
       if (S.nsplit > nseg) nseg = S.nsplit;
       for (uint32_t r = 0; r < S.nsplit; ++r)
@@ -1152,22 +1209,13 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
       cnt[0] += S.pl.nwork;
     }
   }
-  if (banded != B->banded) {
-    B->banded = banded;
-    gb_b_drop_graphs(B);  // the graphs hold the SpMV build
-  }
-  bool regrid = nseg != B->nseg;
-  for (uint32_t g = 0; g < nseg; ++g) regrid = regrid || resize(cnt[g], B->cap_seg[g]);
-  if (regrid) {
-    for (uint32_t g = 0; g < GB_SPLIT_MAX; ++g)
-      B->cap_seg[g] = g < nseg ? (uint32_t)(cnt[g] + cnt[g] / 2 + GB_BLIST_MIN) : 0;
-    B->nseg = nseg;
-    gb_b_drop_graphs(B);  // the graphs hold the launch grids
-  }
+  // few workgroups per CU where that suits nearly all items (see the constant)
+  const uint32_t lds = blocks && scattered * 10 >= blocks * 9 && nseg == 1 ? GB_SPMV_FEW_LDS : 0;
+  bool regrid = nseg != B->nseg || ne != B->grid_elem || lds != B->lds;
   uint64_t a = 0, c = 0;
-  uint32_t q = 0;
   for (uint32_t g = 0; g < nseg; ++g) {
-    B->h_lists->seg[g] = (uint32_t)a;
+    regrid = regrid || B->seg[g] != a || B->seg[g + 1] != a + cnt[g];
+    B->seg[g] = (uint32_t)a;
     for (uint32_t i = 0; i < B->max_slots; ++i) {
       if (!B->used[i] || (active && !active[i])) continue;
       const gb_bsys &S = B->h_sys[i];
@@ -1175,15 +1223,16 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
       if (S.xt_ptr) nw = 0;
       else if (S.nsplit) nw = g < S.nsplit ? B->h_slice_nwork[(size_t)i * GB_SPLIT_MAX + g] : 0;
       else if (g == 0) nw = S.pl.nwork;
-      for (uint32_t w = 0; w < nw; ++w) {
-        B->h_spmv[2 * a] = i;
-        B->h_spmv[2 * a + 1] = w;
-        ++a;
-      }
+      for (uint32_t w = 0; w < nw; ++w) B->h_spmv[a++] = make_uint2(i, w);
     }
+    B->seg[g + 1] = (uint32_t)a;
   }
-  B->h_lists->seg[nseg] = (uint32_t)a;
-  B->h_lists->nseg = nseg;
+  if (regrid) {
+    B->grid_elem = (uint32_t)ne;
+    B->nseg = nseg;
+    B->lds = lds;
+    gb_b_drop_graphs(B);  // the graphs hold the launch grids
+  }
   // the x-tile systems' launches (the graphs hold them)
   uint32_t nx = 0;
   bool xchanged = false;
@@ -1202,19 +1251,13 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
   for (uint32_t i = 0; i < B->max_slots; ++i) {
     if (!B->used[i] || (active && !active[i])) continue;
     for (uint32_t k = 0; k < B->h_sys[i].nchunks; ++k) {
-      B->h_elem[2 * c] = i;
-      B->h_elem[2 * c + 1] = k;
-      ++c;
+      B->h_elem[c++] = make_uint2(i, k);
     }
-    B->h_sysl[q++] = i;
   }
-  B->h_lists->n_spmv = (uint32_t)ns;
-  B->h_lists->n_elem = (uint32_t)ne;
-  B->h_lists->n_sys = nsys;
   if (ns) {
     GB_HIP(hipMemcpyAsync(B->d_spmv, B->h_spmv, ns * 8, hipMemcpyHostToDevice, s));
     for (uint32_t g = 0; g < nseg; ++g) {
-      const uint32_t a0 = B->h_lists->seg[g], a1 = B->h_lists->seg[g + 1];
+      const uint32_t a0 = B->seg[g], a1 = B->seg[g + 1];
       if (a1 > a0) {
         uint32_t gr = gb_div_up(a1 - a0, GB_BLOCK);
         if (gr > 4096u) gr = 4096u;
@@ -1225,17 +1268,19 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
     }
   }
   if (ne) GB_HIP(hipMemcpyAsync(B->d_elem, B->h_elem, ne * 8, hipMemcpyHostToDevice, s));
-  if (nsys)
-    GB_HIP(hipMemcpyAsync(B->d_sysl, B->h_sysl, (size_t)nsys * 4, hipMemcpyHostToDevice, s));
-  GB_HIP(hipMemcpyAsync(B->d_lists, B->h_lists, sizeof(gb_blists), hipMemcpyHostToDevice, s));
   return GOOSEBERRY_SUCCESS;
 }
 
-// k steps, replayed from graphs of 2^i steps captured on first use.
+// k steps, replayed from graphs of 2^i steps captured on first use once the
+// launches have stayed the same.
 int gbd_batch_step(gbd_batch *B, uint32_t k) {
   hipStream_t s = gb_stream();
   if (!B->d_spmv || !B->d_elem) return GOOSEBERRY_ERROR_INVALIDINPUT;
   if (!gb_graphs_enabled()) return gb_b_enqueue_raw(B, k);
+  if (B->stable < GB_B_STABLE) {
+    B->stable += k;
+    return gb_b_enqueue_raw(B, k);
+  }
   for (int i = GB_B_NGRAPH - 1; i >= 0 && k; --i) {
     const uint32_t len = 1u << i;
     while (k >= len) {

@@ -152,6 +152,20 @@ static inline uint32_t gb_spmv_nwaveblocks(const gbd_matrix *m) {
 static inline uint32_t gb_spmv_nwork(const gbd_matrix *m) {
   return m->nstream + gb_spmv_nwaveblocks(m) + m->nblockrows;
 }
+// Row blocks whose columns scatter over x gather best from three workgroups of
+// 256 threads per CU: with more, their gathers queue up in the caches.  These
+// bytes of LDS, unused, on top of a row-block kernel's own (9 or 18 KB) keep
+// it to three.  Taken where the plan has no 16-bit offsets and nine of ten work
+// items are row blocks; wavefront rows (100 entries: 136 us at eight
+// workgroups per CU, 199 us at three) and banded matrices want them all.
+// Random matrices of 29 entries a row, FP32 / FP64 SpMV, at 8 and 3 workgroups:
+// 100,000 rows 19.0 -> 18.0 / 20.4 -> 19.6 us, 300,007 rows 52.2 -> 43.4 /
+// 54.9 -> 48.3 us, 1,048,576 rows 198 -> 173 / 309 -> 305 us.
+#define GB_SPMV_FEW_LDS 34000u
+static inline uint32_t gb_spmv_few_lds(const gbd_matrix *m) {
+  const bool few = !m->dcol && (uint64_t)m->nstream * 10 >= (uint64_t)gb_spmv_nwork(m) * 9;
+  return few ? GB_SPMV_FEW_LDS : 0;
+}
 // workgroups of one SpMV launch (the number of p.Ap partials with DOT)
 uint32_t gb_spmv_grid(const gbd_matrix *m);
 

@@ -810,7 +810,7 @@ static void gb_spmv_go(const gbd_matrix *m, uint32_t grid, hipStream_t s, const 
   }
   const uint32_t *wave_rows = m->rowbins + (m->nrows - m->nwave - m->nblockrows);
   const uint32_t *block_rows = m->rowbins + (m->nrows - m->nblockrows);
-  gb_spmv_kernel<T, DOT, NARROW, VD><<<grid, GB_BLOCK, 0, s>>>(
+  gb_spmv_kernel<T, DOT, NARROW, VD><<<grid, GB_BLOCK, gb_spmv_few_lds(m), s>>>(
       m->rowptr, m->rowind, NARROW ? m->dcol : nullptr, val, vidx, vtab, x, y, ystride,
       m->cshift, m->bdesc, m->nstream, wave_rows, m->nwave, gb_spmv_nwaveblocks(m), block_rows,
       gb_spmv_nwork(m), m->params.exact, m->params.xcd_remap, partials, cg);
@@ -888,8 +888,9 @@ static int gb_spmv_launch_t(const gbd_matrix *m, const T *val, const uint8_t *vi
 // Bound: the band form by HBM and the latency of its gathers (a million rows
 // of 7 entries, 8 columns: 65.5 us against 208 us for eight SpMVs with a
 // strided result; 152 MB once, 2.3 TB/s), the row form by the accesses to
-// B's rows (random matrices of 29 entries a row, 4 to 32 columns: 1.9 to 2.9
-// times the loop's rate).
+// B's rows (random matrices of 29 entries a row against as many SpMVs: 2, 4
+// and 8 columns 33, 40 and 58 us against 42, 86 and 174 us at 100,000 rows,
+// 11, 13 and 18 us against 12, 24 and 46 us at 10,000).
 #define GB_MM_COLS 8
 
 // Bt[i G + j] = B[j n + i] for the cols (<= G) columns
