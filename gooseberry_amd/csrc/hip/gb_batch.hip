@@ -89,10 +89,10 @@ struct gb_bsys {
   const double *jscale;  // MIXED_JACOBI: D^-1/2, else null
   // an x-tile plan (xt_ptr non-null): the layout, its FP64 values and the
   // FP32 values of the inner solve (plain or Jacobi-scaled)
-  const uint32_t *xt_ptr, *xt_idx;
+  const uint32_t *xt_rb, *xt_ptr, *xt_idx;
   const double *xt_val;
   const float *xt_val32;
-  uint32_t xt_R, xt_W, xt_T, xt_lc;
+  uint32_t xt_W, xt_T, xt_lc;
   int32_t precision;
   int32_t pad;
 };
@@ -391,13 +391,13 @@ gb_b_spmv_xt(const gb_bsys *__restrict__ sys, uint32_t slot,
   if (st->done) return;  // not written during this kernel: uniform
   if (st->mode_next == GB_MODE_REFRESH)
     gb_xt_spmv<double, GB_XT_RESID>(S.xt_ptr, S.xt_idx, S.xt_val, S.x, S.r, 1, S.b, S.part1,
-                                    S.n, S.n, S.xt_R, S.xt_T, S.xt_lc, L);
+                                    S.xt_rb, S.n, S.xt_T, S.xt_lc, L);
   else if (S.precision != GOOSEBERRY_PRECISION_FP64)
     gb_xt_spmv<float, GB_XT_DOT>(S.xt_ptr, S.xt_idx, S.xt_val32, S.p32, S.ap32, 1, nullptr,
-                                 S.part1, S.n, S.n, S.xt_R, S.xt_T, S.xt_lc, L);
+                                 S.part1, S.xt_rb, S.n, S.xt_T, S.xt_lc, L);
   else
     gb_xt_spmv<double, GB_XT_DOT>(S.xt_ptr, S.xt_idx, S.xt_val, S.p, S.ap, 1, nullptr,
-                                  S.part1, S.n, S.n, S.xt_R, S.xt_T, S.xt_lc, L);
+                                  S.part1, S.xt_rb, S.n, S.xt_T, S.xt_lc, L);
 }
 
 // A thread's GB_BCHUNK_ITEMS rows of a whole chunk of an internal vector
@@ -1086,7 +1086,7 @@ int gbd_batch_add(gbd_batch *B, const gbd_matrix *m, const double *d_b,
     S.xt_idx = m->xt_idx;
     S.xt_val = m->xt_val;
     S.xt_val32 = jac ? m->xt_val32j : m->xt_val32;
-    S.xt_R = m->xt_R;
+    S.xt_rb = m->xt_rb;
     S.xt_W = m->xt_W;
     S.xt_T = m->xt_T;
     S.xt_lc = m->xt_lc;

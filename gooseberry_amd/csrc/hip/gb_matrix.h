@@ -42,16 +42,18 @@ struct gbd_matrix {
   uint32_t nvals;
   uint32_t pipe_grid;   // > 0: the SpMV runs the persistent pipelined
                         // row-block kernel on this many workgroups
-  // x tiles (params.xtile = C): the entries grouped by (block of xt_R rows,
-  // tile of C columns), each group in CSR order; entry j of the layout is
-  // xt_idx[j] = (row in block << xt_lc) | (column in tile) with value
-  // xt_val[j], group g = b xt_T + t holding [xt_ptr[g], xt_ptr[g + 1])
+  // x tiles (params.xtile = C): the entries grouped by (block of rows
+  // [xt_rb[b], xt_rb[b + 1]), tile of C columns), each group in CSR order;
+  // entry j of the layout is xt_idx[j] = (row in block << xt_lc) | (column in
+  // tile) with value xt_val[j], group g = b xt_T + t holding
+  // [xt_ptr[g], xt_ptr[g + 1])
+  uint32_t *xt_rb;      // xt_W + 1
   uint32_t *xt_ptr;     // xt_W xt_T + 1
   uint32_t *xt_idx;     // nnz
   double *xt_val;       // nnz
   float *xt_val32;      // nnz, with val32: its values in the layout's order
   float *xt_val32j;     // nnz, with val32j: its values in the layout's order
-  uint32_t xt_R, xt_W, xt_T, xt_lc;
+  uint32_t xt_W, xt_T, xt_lc;
   uint64_t hist[33];
   // column split (params.csplit = P > 1): P views, view r holding the
   // entries of columns [r W, (r + 1) W), W = ceil(ncols / P), in row order;

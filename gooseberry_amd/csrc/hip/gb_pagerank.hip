@@ -226,10 +226,12 @@ gb_pr_colsum_xt(const uint32_t *__restrict__ ptr, uint32_t W, uint32_t T, uint32
   __shared__ uint32_t gst[GB_PRX_THREADS];    // the window's groups: first entry
   __shared__ uint32_t goff[GB_PRX_THREADS + 1];  // and first window position
   __shared__ uint32_t wsum[GB_PRX_THREADS / GB_WAVE];
+  __shared__ uint32_t rounds;  // the chunk's most shared column: its wavefronts
   const uint32_t t = blockIdx.x, tid = threadIdx.x;
   const uint32_t lane = tid & (GB_WAVE - 1), wave = tid / GB_WAVE;
   const uint64_t below = (1ull << lane) - 1;
   const uint32_t C = 1u << lc, cm = C - 1;
+  if (tid == 0) rounds = 0;
   for (uint32_t j = tid; j < C; j += GB_PRX_THREADS) {
     cs[j] = 0.0;
     wset[j] = 0;
@@ -273,6 +275,7 @@ gb_pr_colsum_xt(const uint32_t *__restrict__ ptr, uint32_t W, uint32_t T, uint32
       gb_prx_lds_barrier();
       const uint32_t ws = first ? wset[col] : 0u;
       const bool alone = first && ws == (1u << wave);
+      if (first && !alone) atomicMax(&rounds, (uint32_t)__popc(ws));
       const uint64_t rest = peers & ~(below | (1ull << lane));
       // columns of one wavefront: added now, every wavefront at once
       {
@@ -280,16 +283,24 @@ gb_pr_colsum_xt(const uint32_t *__restrict__ ptr, uint32_t W, uint32_t T, uint32
         sum = gb_prx_chain(sum, v, alone ? rest : 0);
         if (alone) cs[col] = sum;
       }
-      // columns of several wavefronts: wavefront by wavefront, in order
+      // columns of several wavefronts: each wavefront adds in the round of
+      // its rank among the column's wavefronts, so in order; as many rounds
+      // as the most shared column of the chunk has wavefronts (two or three
+      // with scattered columns, 16 with a hub)
       const bool shared_col = first && !alone;
-      for (uint32_t w = 0; w < GB_PRX_THREADS / GB_WAVE; ++w) {
-        if (wave == w) {
-          double sum = shared_col ? cs[col] + v : 0.0;
-          sum = gb_prx_chain(sum, v, shared_col ? rest : 0);
-          if (shared_col) cs[col] = sum;
+      const uint32_t rank = (uint32_t)__popc(ws & ((1u << wave) - 1u));
+      gb_prx_lds_barrier();
+      const uint32_t nround = rounds;
+      for (uint32_t w = 0; w < nround; ++w) {
+        const bool now = shared_col && rank == w;
+        if (__ballot(now)) {
+          double sum = now ? cs[col] + v : 0.0;
+          sum = gb_prx_chain(sum, v, now ? rest : 0);
+          if (now) cs[col] = sum;
         }
         gb_prx_lds_barrier();
       }
+      if (tid == 0) rounds = 0;
       if (first) wset[col] = 0;
       have = nhave;
       col = ncol & cm;

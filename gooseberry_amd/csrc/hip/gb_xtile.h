@@ -1,10 +1,12 @@
 // gb_xtile.h -- the SpMV over the x-tile layout, shared by the matrix path
 // (gb_spmv.hip) and the batched engine (gb_batch.hip).
 //
-// The layout groups a matrix's entries by (block of R rows, tile of
-// C = 2^lc columns), each group in CSR order: ptr[g] .. ptr[g + 1] for group
+// The layout groups a matrix's entries by (row block, tile of C = 2^lc
+// columns), each group in CSR order: ptr[g] .. ptr[g + 1] for group
 // g = block * T + tile, each entry a packed word (row within the block << lc
-// | column within the tile) and a value.  One workgroup owns a row block and
+// | column within the tile) and a value.  Row block b is rows rb[b] ..
+// rb[b + 1], at most GB_XT_RMAX, and the blocks hold about equally many
+// entries where that limit allows.  One workgroup owns a row block and
 // keeps its y in LDS; tile by tile it copies x's tile into LDS and adds its
 // group's products, so the gathers read LDS and only the matrix and x
 // stream.  Each row gets one sum per tile, added to its y in tile order: a
@@ -123,8 +125,9 @@ __device__ __forceinline__ void gb_xt_spmv(const uint32_t *__restrict__ ptr,
                                            const V *__restrict__ val, const V *__restrict__ x,
                                            V *__restrict__ y, uint32_t ystride,
                                            const double *__restrict__ b,
-                                           double *__restrict__ partials, uint32_t nrows,
-                                           uint32_t ncols, uint32_t R, uint32_t T, uint32_t lc,
+                                           double *__restrict__ partials,
+                                           const uint32_t *__restrict__ rb,
+                                           uint32_t ncols, uint32_t T, uint32_t lc,
                                            gb_xt_lds &L) {
   constexpr uint32_t NW = GB_XT_THREADS / GB_WAVE;
   // tiles a step covers: two adjacent tiles in FP32 (their x fits the same
@@ -140,8 +143,8 @@ __device__ __forceinline__ void gb_xt_spmv(const uint32_t *__restrict__ ptr,
   V *whead = (V *)L.whead;
   uint32_t *wfrow = L.wfrow, *wlrow = L.wlrow;
   const uint32_t tid = threadIdx.x, lane = tid & (GB_WAVE - 1), wv = tid / GB_WAVE;
-  const uint32_t r0 = blockIdx.x * R;
-  const uint32_t nr = min(R, nrows - r0);
+  const uint32_t r0 = rb[blockIdx.x];
+  const uint32_t nr = rb[blockIdx.x + 1] - r0;
   const uint32_t C = 1u << lc;
   // with two tiles a step, the second tile's runs add into their own
   // accumulator (the y region's unused half in FP32): a row can have a run

@@ -199,3 +199,43 @@ def test_xtile_batched_solves(gb, oracle, precision):
     assert np.array_equal(res[0][0], x_l) and res[0][1].niter == i_l.niter
     for x, info in res:
         assert info.status == 1
+
+
+@pytest.mark.parametrize("shape", ["head", "tail", "one_row", "few", "limit"])
+def test_xtile_row_blocks_of_equal_entries(gb, oracle, shape):
+    # blocks cut by entries: all long rows first or last, one row that holds
+    # nearly everything (blocks without rows beside it), fewer rows than
+    # workgroups, and so many empty rows that the 8192-row limit decides
+    rng = np.random.default_rng(5)
+    n = {"few": 37, "limit": 1 << 20}.get(shape, 70000)
+    deg = np.full(n, 2)
+    if shape == "head":
+        deg[:300] = 3000
+    elif shape == "tail":
+        deg[-300:] = 3000
+    elif shape == "one_row":
+        deg[33333] = 200000
+    elif shape == "few":
+        deg = rng.integers(0, 400, n)
+    else:
+        deg[:] = 0
+        deg[::4099] = 500
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+    nc = 30011
+    ri = rng.integers(0, nc, rp[-1]).astype(np.uint32)
+    rv = rng.uniform(-1, 1, rp[-1])
+    print("x tiles", shape, flush=True)
+    M = gb.Matrix(rp, ri, rv, ncols=nc, plan={"xtile": 4096})
+    assert M.info()["plan"]["xtile"] == 4096
+    x = rng.uniform(-1, 1, nc)
+    y = M.spmv(x)
+    ref = oracle.spmult(n, nc, 1, rp, ri, rv, x)
+    # |sum - fl(sum)| <= (len - 1) eps sum |terms| for either order
+    mag = np.add.reduceat(np.append(np.abs(rv * x[ri]), 0.0), rp[:-1].astype(np.int64))
+    mag[deg == 0] = 0.0
+    assert np.all(np.abs(y - ref) <= 2 * np.maximum(deg, 1) * 2.3e-16 * mag)
+    assert np.array_equal(y, M.spmv(x))
+    # integers: exact in any order, in FP32 too (sums below 2^24)
+    ii = gb.Matrix(rp, ri, np.ones(rp[-1]), ncols=nc, plan={"xtile": 4096})
+    assert np.array_equal(ii.spmv(np.ones(nc)), deg.astype(np.float64))
+    assert np.array_equal(ii.spmv_f32(np.ones(nc)), deg.astype(np.float32))
