@@ -121,6 +121,7 @@ struct gbd_batch {
   uint32_t *h_slice_nwork;             // host: max_slots x GB_SPLIT_MAX
   uint32_t *h_xt;                      // host: the active x-tile systems' slots
   uint32_t *h_xt_grid;                 // and their launch grids
+  uint32_t *h_xt_lc;                   // and tile widths
   uint32_t n_xt;
   gb_bplan *d_slices;                  // max_slots x GB_SPLIT_MAX slice plans
   uint2 *h_spmv, *h_elem;              // pinned staging
@@ -382,10 +383,11 @@ gb_b_spmv(const gb_bsys *__restrict__ sys, const uint2 *__restrict__ items,
 // the p.Ap partials of a CG step in the system's precision, or in a
 // refresh step the FP64 residual b - A x and its squared-norm partials;
 // one partial per row block
+template <bool WIDE>
 __global__ void __launch_bounds__(GB_XT_THREADS)
 gb_b_spmv_xt(const gb_bsys *__restrict__ sys, uint32_t slot,
              const gbd_bstate *__restrict__ states) {
-  __shared__ gb_xt_lds L;
+  __shared__ gb_xt_lds_t<WIDE> L;
   const gb_bsys &S = sys[slot];
   const gbd_bstate *st = states + slot;
   if (st->done) return;  // not written during this kernel: uniform
@@ -872,7 +874,9 @@ static int gb_b_enqueue_raw(gbd_batch *B, uint32_t k) {
     }
     if (!B->grid_elem) continue;
     for (uint32_t j = 0; j < B->n_xt; ++j) {
-      gb_b_spmv_xt<<<B->h_xt_grid[j], GB_XT_THREADS, 0, s>>>(B->d_sys, B->h_xt[j], B->d_st);
+      auto *k = gb_xt_is_wide(B->h_xt_lc[j]) ? gb_b_spmv_xt<true>
+                                                          : gb_b_spmv_xt<false>;
+      k<<<B->h_xt_grid[j], GB_XT_THREADS, 0, s>>>(B->d_sys, B->h_xt[j], B->d_st);
       GB_LAUNCH_CHECK();
     }
     gb_b_update<<<B->grid_elem, GB_BLOCK, 0, s>>>(B->d_sys, B->d_elem, B->d_st);
@@ -977,6 +981,7 @@ int gbd_batch_create(uint32_t max_slots, double delta, gbd_batch **out) {
   B->h_slice_nwork = (uint32_t *)calloc((size_t)max_slots * GB_SPLIT_MAX, sizeof(uint32_t));
   B->h_xt = (uint32_t *)calloc(max_slots, sizeof(uint32_t));
   B->h_xt_grid = (uint32_t *)calloc(max_slots, sizeof(uint32_t));
+  B->h_xt_lc = (uint32_t *)calloc(max_slots, sizeof(uint32_t));
   B->h_sys = (gb_bsys *)calloc(max_slots, sizeof(gb_bsys));
   hipError_t e = gb_dev_alloc((void **)&B->d_sys, max_slots * sizeof(gb_bsys));
   if (e == hipSuccess) e = gb_dev_alloc((void **)&B->d_st, max_slots * sizeof(gbd_bstate));
@@ -989,7 +994,7 @@ int gbd_batch_create(uint32_t max_slots, double delta, gbd_batch **out) {
   if (e == hipSuccess)
     e = hipMemsetAsync(B->d_sys, 0, max_slots * sizeof(gb_bsys), gb_stream());
   if (e != hipSuccess || !B->used || !B->slot_mem || !B->slot_mat || !B->h_sys ||
-      !B->h_slice_nwork || !B->h_xt || !B->h_xt_grid) {
+      !B->h_slice_nwork || !B->h_xt || !B->h_xt_grid || !B->h_xt_lc) {
     gbd_batch_destroy(B);
     return e != hipSuccess ? gb_hip_fail(e, "gbd_batch_create", __FILE__, __LINE__)
                            : GOOSEBERRY_ERROR_NOMEMORY;
@@ -1022,6 +1027,7 @@ void gbd_batch_destroy(gbd_batch *B) {
   free(B->h_slice_nwork);
   free(B->h_xt);
   free(B->h_xt_grid);
+  free(B->h_xt_lc);
   free(B->h_sys);
   free(B);
 }
@@ -1239,9 +1245,10 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
   for (uint32_t i = 0; i < B->max_slots; ++i) {
     if (!B->used[i] || (active && !active[i]) || !B->h_sys[i].xt_ptr) continue;
     xchanged = xchanged || nx >= B->n_xt || B->h_xt[nx] != i ||
-               B->h_xt_grid[nx] != B->h_sys[i].xt_W;
+               B->h_xt_grid[nx] != B->h_sys[i].xt_W || B->h_xt_lc[nx] != B->h_sys[i].xt_lc;
     B->h_xt[nx] = i;
     B->h_xt_grid[nx] = B->h_sys[i].xt_W;
+    B->h_xt_lc[nx] = B->h_sys[i].xt_lc;
     ++nx;
   }
   if (xchanged || nx != B->n_xt) {

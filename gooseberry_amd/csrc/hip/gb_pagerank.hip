@@ -135,6 +135,12 @@ gb_pr_normalise_xt(const uint32_t *__restrict__ ptr, uint32_t ngroups, uint32_t 
 // every entry of the tile by its column's sum.
 #define GB_PRX_THREADS 1024
 #define GB_PRX_NORM 4
+// Column tiles from which on the walk beats the sort: with fewer, too few
+// workgroups walk (a Zipf graph of 300,000 rows, sums and one iteration: 74
+// tiles 2.06 ms against 1.66 with the sort, 147 tiles 1.61 against 1.90; of
+// 900,000 rows, 110 tiles, 3.71 against 4.35; of 30,000, 30 tiles, 0.82
+// against 0.49).
+#define GB_PRX_TILES 96
 
 // A workgroup barrier that orders LDS only: global loads still in flight
 // (the next chunk's entries) stay in flight across it, where __syncthreads
@@ -448,12 +454,15 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
   // An x-tile or column-split plan reads its own copy of the values, which
   // is normalised below; the CSR's order is then never read.
   const bool own_copy = m->xt_ptr || m->nsplit;
-  // An x-tile plan sums the columns on its own layout, without the sort;
-  // GOOSEBERRY_PAGERANK_SORTED_SUMS (set, not "0") takes the sort instead
-  // (the same bits: a check of one path against the other).
+  // An x-tile plan sums the columns on its own layout, without the sort, where
+  // it has the column tiles to fill the GPU with a workgroup each;
+  // GOOSEBERRY_PAGERANK_SORTED_SUMS set to "0" takes the layout wherever its
+  // tiles fit, set to anything else the sort (the same bits: a check of one
+  // path against the other).
   const char *sorted_env = getenv("GOOSEBERRY_PAGERANK_SORTED_SUMS");
-  const bool tile_sums = m->xt_ptr && nnz &&
-                         !(sorted_env && *sorted_env && strcmp(sorted_env, "0") != 0);
+  bool tile_sums = m->xt_ptr && nnz && (1u << m->xt_lc) <= GB_XT_CMAX;
+  if (sorted_env && *sorted_env) tile_sums = tile_sums && strcmp(sorted_env, "0") == 0;
+  else tile_sums = tile_sums && m->xt_T >= GB_PRX_TILES;
 #define GB_PR_TRY(call)                                         \
   do {                                                          \
     he = (call);                                                \

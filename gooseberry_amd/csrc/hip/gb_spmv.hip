@@ -643,13 +643,13 @@ __global__ void gb_xt_gather(const uint32_t *__restrict__ perm, uint64_t nnz,
 
 // y = A x on the x-tile layout (V = double, or float for the FP32 SpMV);
 // with `partials` (FP64, CG) the block's share of x.Ax as well
-template <typename V, int EPI>
+template <typename V, int EPI, bool WIDE>
 __global__ void __launch_bounds__(GB_XT_THREADS)
 gb_spmv_xtile(const uint32_t *__restrict__ ptr, const uint32_t *__restrict__ idx,
               const V *__restrict__ val, const V *__restrict__ x, V *__restrict__ y,
               uint32_t ystride, double *__restrict__ partials,
               const uint32_t *__restrict__ rb, uint32_t ncols, uint32_t T, uint32_t lc) {
-  __shared__ gb_xt_lds L;
+  __shared__ gb_xt_lds_t<WIDE> L;
   gb_xt_spmv<V, EPI>(ptr, idx, val, x, y, ystride, nullptr, partials, rb, ncols, T, lc, L);
 }
 
@@ -872,7 +872,9 @@ static int gb_spmv_launch_t(const gbd_matrix *m, const T *val, const uint8_t *vi
     else xv = cg ? nullptr : m->xt_val32;
     if (xv) {
       hipStream_t s = gb_stream();
-      gb_spmv_xtile<T, GB_XT_STORE><<<m->xt_W, GB_XT_THREADS, 0, s>>>(
+      auto *k = gb_xt_is_wide(m->xt_lc) ? gb_spmv_xtile<T, GB_XT_STORE, true>
+                                        : gb_spmv_xtile<T, GB_XT_STORE, false>;
+      k<<<m->xt_W, GB_XT_THREADS, 0, s>>>(
           m->xt_ptr, m->xt_idx, xv, x, y, ystride, nullptr, m->xt_rb, m->ncols, m->xt_T,
           m->xt_lc);
       GB_LAUNCH_CHECK();
@@ -1453,15 +1455,24 @@ static int gb_xtile_f32(gbd_matrix *m) {
 // ceil(nrows / CUs) rows (at most GB_XT_RMAX): one workgroup per CU.
 static int gb_xtile_build(gbd_matrix *m) {
   hipStream_t s = gb_stream();
-  const uint32_t n = m->nrows, C = m->params.xtile;
-  uint32_t lc = 0;
+  const uint32_t n = m->nrows;
+  uint32_t C = m->params.xtile, lc = 0;
   while ((1u << lc) < C) ++lc;
   uint32_t R = gb_div_up(n, gb_num_cus());
-  if (R > GB_XT_RMAX) R = GB_XT_RMAX;
+  // the widest tiles are doubled where the rows leave LDS for them, with room
+  // for blocks of equal entries, and both types take fewer steps then (FP32
+  // has two tiles a step already: 9,000 columns 8.2 us plain, 9.1 doubled)
+  const bool wide = C == GB_XT_CMAX && m->ncols > 2 * C && R <= GB_XT_RWIDE / 5 * 4;
+  const uint32_t rmax = wide ? GB_XT_RWIDE : GB_XT_RMAX;
+  if (wide) {
+    C = GB_XT_WIDE;
+    ++lc;
+  }
+  if (R > rmax) R = rmax;
   if (R == 0) R = 1;
   const uint32_t W = gb_div_up(n, R);
-  // the least weight per row that keeps the blocks within GB_XT_RMAX rows
-  const uint64_t room = (uint64_t)W * (GB_XT_RMAX - 2);
+  // the least weight per row that keeps the blocks within rmax rows
+  const uint64_t room = (uint64_t)W * (rmax - 2);
   uint64_t k = 0;
   if (room > n) {
     k = m->nnz / (room - n) + 1;

@@ -5,8 +5,8 @@
 // columns), each group in CSR order: ptr[g] .. ptr[g + 1] for group
 // g = block * T + tile, each entry a packed word (row within the block << lc
 // | column within the tile) and a value.  Row block b is rows rb[b] ..
-// rb[b + 1], at most GB_XT_RMAX, and the blocks hold about equally many
-// entries where that limit allows.  One workgroup owns a row block and
+// rb[b + 1], at most GB_XT_RMAX (GB_XT_RWIDE with doubled tiles), and the
+// blocks hold about equally many entries where that limit allows.  One workgroup owns a row block and
 // keeps its y in LDS; tile by tile it copies x's tile into LDS and adds its
 // group's products, so the gathers read LDS and only the matrix and x
 // stream.  Each row gets one sum per tile, added to its y in tile order: a
@@ -22,10 +22,22 @@
 
 #define GB_XT_THREADS 1024
 #define GB_XT_RMAX 8192  // rows of y a workgroup keeps in LDS
+// Matrices of few rows per workgroup have the LDS for tiles twice as wide
+// (GB_XT_WIDE columns of FP64 x, 128 KB) beside a block of GB_XT_RWIDE rows.
+// A step costs 3.3 us before its first entry (staging x, two barriers, the
+// carries) and a 300,000-row Zipf graph takes 4.4 us for one, so half as many
+// steps: FP64 / FP32 us, plain and doubled, at 30,000 rows 20.9 / 13.1 and
+// 16.5 / 11.3, at 300,000 165.0 / 101.6 and 140.4 / 85.8, at 800,000
+// 435 / 262 and 370 / 229.
+#define GB_XT_WIDE (2 * GB_XT_CMAX)
+#define GB_XT_RWIDE 3968
 #define GB_XT_DEPTH 1    // chunks a wavefront has in flight (on the Zipf matrix:
                          // FP64 1.56-1.59 ms at 1, 1.60 at 2, 1.72 at 3;
                          // FP32 1.08 ms at 1, 1.13 at 2)
 #define GB_XT_PAD 4      // zero entries past the end of the layout's arrays
+
+// whether a layout of 2^lc columns a tile takes the wide kernels
+static inline bool gb_xt_is_wide(uint32_t lc) { return (1u << lc) > GB_XT_CMAX; }
 
 // what the workgroup does with its block of y = A x
 enum {
@@ -93,9 +105,11 @@ __device__ __forceinline__ float gb_readlane_val(float v, uint32_t l) {
 
 // The LDS a workgroup of the x-tile SpMV uses, declared once by each
 // kernel and viewed as V (the FP32 SpMV uses the first halves)
+template <uint32_t CMAX, uint32_t RMAX>
 struct gb_xt_lds {
-  double xs[GB_XT_CMAX];  // the current tile of x
-  double ys[GB_XT_RMAX];  // the block's y
+  static constexpr uint32_t cmax = CMAX, rmax = RMAX;
+  double xs[CMAX];  // the current tile of x
+  double ys[RMAX];  // the block's y
   double wcarry[GB_XT_THREADS / GB_WAVE];  // a range's first run, cut off
                                            // from the one before
   double whead[GB_XT_THREADS / GB_WAVE];   // a range's last run, started in it
@@ -104,6 +118,8 @@ struct gb_xt_lds {
   uint32_t wlrow[GB_XT_THREADS / GB_WAVE]; // last run's row | started here (bit 31)
   double red[GB_XT_THREADS / GB_WAVE];     // the block's partial
 };
+template <bool WIDE>
+using gb_xt_lds_t = gb_xt_lds<WIDE ? GB_XT_WIDE : GB_XT_CMAX, WIDE ? GB_XT_RWIDE : GB_XT_RMAX>;
 
 // y = A x on the x-tile layout for the block blockIdx.x (grid = the row
 // blocks).  A group's entries are cut into one contiguous range per
@@ -119,7 +135,7 @@ struct gb_xt_lds {
 // where it starts, which adds the following ranges' parts in order.  The
 // layout's arrays hold GB_XT_PAD zero entries past the end, so a lane's
 // vector never reads past them.
-template <typename V, int EPI>
+template <typename V, int EPI, typename LDS>
 __device__ __forceinline__ void gb_xt_spmv(const uint32_t *__restrict__ ptr,
                                            const uint32_t *__restrict__ idx,
                                            const V *__restrict__ val, const V *__restrict__ x,
@@ -128,14 +144,14 @@ __device__ __forceinline__ void gb_xt_spmv(const uint32_t *__restrict__ ptr,
                                            double *__restrict__ partials,
                                            const uint32_t *__restrict__ rb,
                                            uint32_t ncols, uint32_t T, uint32_t lc,
-                                           gb_xt_lds &L) {
+                                           LDS &L) {
   constexpr uint32_t NW = GB_XT_THREADS / GB_WAVE;
   // tiles a step covers: two adjacent tiles in FP32 (their x fits the same
   // 64 KB of LDS; on the Zipf matrix 1.01 ms against 1.07 ms a tile a
   // step), one in FP64; the second tile's rows carry bit 15 in their keys,
   // so that no run spans the two tiles
   constexpr uint32_t TP = sizeof(V) == 4 ? 2 : 1;
-  constexpr uint32_t XPT = TP * GB_XT_CMAX / GB_XT_THREADS;  // x values a thread stages
+  constexpr uint32_t XPT = TP * LDS::cmax / GB_XT_THREADS;  // x values a thread stages
   constexpr uint32_t NONE = 0xffffffffu;
   V *xs = (V *)L.xs;
   V *ys = (V *)L.ys;
@@ -149,7 +165,7 @@ __device__ __forceinline__ void gb_xt_spmv(const uint32_t *__restrict__ ptr,
   // with two tiles a step, the second tile's runs add into their own
   // accumulator (the y region's unused half in FP32): a row can have a run
   // in each tile, and two wavefronts must not update one word at once
-  V *ys2 = ys + GB_XT_RMAX;
+  V *ys2 = ys + LDS::rmax;
   for (uint32_t i = tid; i < nr; i += GB_XT_THREADS) {
     ys[i] = (V)0;
     if (TP > 1) ys2[i] = (V)0;

@@ -245,3 +245,21 @@ def test_pagerank_tile_sums_match_sorted_sums(gb, case, monkeypatch):
     assert (it, ns) == (its, nss) == (niter, ns)
     assert np.array_equal(x, xs)
     assert err == errs
+
+
+@pytest.mark.parametrize("n,xtile", [(95 * 256, 256), (95 * 256 + 1, 256), (20000, 8192),
+                                     (8100, 8192)])
+def test_pagerank_sums_by_number_of_tiles(gb, n, xtile, monkeypatch):
+    # fewer than 96 tiles, and the doubled tiles, take the sort, more the walk
+    # over the layout; either forced gives the same bits
+    rp, ri, rv = _hub_graph(n, 11)
+    M = gb.Matrix(rp, ri, rv, plan={"xtile": xtile})
+    got = []
+    for env in (None, "0", "1"):
+        if env is None:
+            monkeypatch.delenv("GOOSEBERRY_PAGERANK_SORTED_SUMS", raising=False)
+        else:
+            monkeypatch.setenv("GOOSEBERRY_PAGERANK_SORTED_SUMS", env)
+        x, it, err, ns = M.pagerank(0.85, 8, 0.0)
+        got.append((x.tobytes(), it, err, ns))
+    assert got[0] == got[1] == got[2]

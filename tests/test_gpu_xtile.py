@@ -239,3 +239,71 @@ def test_xtile_row_blocks_of_equal_entries(gb, oracle, shape):
     ii = gb.Matrix(rp, ri, np.ones(rp[-1]), ncols=nc, plan={"xtile": 4096})
     assert np.array_equal(ii.spmv(np.ones(nc)), deg.astype(np.float64))
     assert np.array_equal(ii.spmv_f32(np.ones(nc)), deg.astype(np.float32))
+
+
+def _long_rows(rng, n, m, shape):
+    deg = rng.integers(0, 6, n)
+    if shape == "head":
+        deg[:300] = 3000
+    elif shape == "one_row":
+        deg[n // 2] = 200000
+    elif shape == "sparse":  # the blocks' row limit decides
+        deg[:] = 0
+        deg[::1021] = 500
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+    return deg, rp, rng.integers(0, m, int(rp[-1])).astype(np.uint32)
+
+
+# 4/5 of 3968 rows a workgroup is the line between the two layouts at 256
+# workgroups; 16384 columns are two plain tiles, 16385 two doubled ones, 49155
+# two FP32 steps of which the second is partial
+@pytest.mark.parametrize("n,m,shape", [
+    (37, 49155, "head"), (70000, 8193, "head"), (70000, 16384, "one_row"),
+    (70000, 16385, "head"), (70000, 49155, "one_row"),
+    (256 * 3174, 49155, "sparse"), (256 * 3174 + 1, 49155, "sparse")])
+def test_xtile_doubled_tiles(gb, oracle, n, m, shape):
+    rng = np.random.default_rng(n + m)
+    deg, rp, ri = _long_rows(rng, n, m, shape)
+    rv, x = rng.uniform(-1, 1, ri.size), rng.uniform(-1, 1, m)
+    print("doubled x tiles", n, m, shape, flush=True)
+    M = gb.Matrix(rp, ri, rv, ncols=m, plan={"xtile": 8192})
+    assert M.info()["plan"]["xtile"] == 8192
+    y = M.spmv(x)
+    ref = oracle.spmult(n, m, 1, rp, ri, rv, x)
+    # |sum - fl(sum)| <= (len - 1) eps sum |terms| for either order
+    mag = np.add.reduceat(np.append(np.abs(rv * x[ri]), 0.0), rp[:-1].astype(np.int64))
+    mag[deg == 0] = 0.0
+    assert np.all(np.abs(y - ref) <= 2 * np.maximum(deg, 1) * 2.3e-16 * mag)
+    assert np.array_equal(y, M.spmv(x))
+    # integers below 2^24 are exact in any order, in FP32 too
+    xi = rng.integers(0, 8, m)
+    ii = gb.Matrix(rp, ri, np.ones(ri.size), ncols=m, plan={"xtile": 8192})
+    exact = oracle.spmult(n, m, 1, rp, ri, np.ones(ri.size), xi.astype(np.float64))
+    assert np.array_equal(ii.spmv(xi.astype(np.float64)), exact)
+    assert np.array_equal(ii.spmv_f32(xi.astype(np.float64)).astype(np.float64), exact)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_xtile_batched_widths_in_turn(gb, oracle, precision):
+    # doubled and plain tiles side by side and one after the other in a slot:
+    # each system solves as it does alone
+    M0 = gb.generate_spd(60000, 5, gb.DEGREE_ZIPF, 1.5, 2, 400)
+    rp, ri, rv = M0.download()
+    b = gb.uniform(6, rp.size - 1)
+    W = gb.Matrix(rp, ri, rv, plan={"xtile": 8192})
+    N = gb.Matrix(rp, ri, rv, plan={"xtile": 4096})
+    (xw, iw), = _batch(gb, [(W, b)], precision)
+    (xn, inn), = _batch(gb, [(N, b)], precision)
+    for x, info in ((xw, iw), (xn, inn)):
+        assert info.status == 1
+        assert np.linalg.norm(b - oracle.spmv(rp, ri, rv, x)) <= 1.05e-10 * np.linalg.norm(b)
+    both = _batch(gb, [(W, b), (N, b)], precision)
+    assert np.array_equal(both[0][0], xw) and np.array_equal(both[1][0], xn)
+    B = gb.Batch(1)
+    for M, x in ((W, xw), (N, xn), (W, xw)):
+        db, dx = gb.DeviceArray.from_host(b), gb.DeviceArray(b.size)
+        s = B.add(M, db, dx, 1e-10, gb.TOL_RELATIVE, 0, precision)
+        B.solve()
+        assert np.array_equal(dx.numpy(), x)
+        B.remove(s)
+    B.free()
