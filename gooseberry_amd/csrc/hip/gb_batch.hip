@@ -947,8 +947,8 @@ static gb_bplan gb_b_plan_of(const gbd_matrix *m, uint32_t base, bool jacobi) {
   P.rowind = m->rowind;
   P.dcol = m->dcol;
   P.blk = m->blk;
-  P.wave_rows = m->rowbins + (m->nrows - m->nwave - m->nblockrows);
-  P.block_rows = m->rowbins + (m->nrows - m->nblockrows);
+  P.wave_rows = gb_wave_rows(m);
+  P.block_rows = gb_block_rows(m);
   P.val = m->val;
   P.val32 = jacobi ? m->val32j : m->val32;
   P.nstream = m->nstream;

@@ -28,6 +28,7 @@ struct gbd_matrix {
   uint32_t nwave;       // rows processed one wavefront per row
   uint32_t nblockrows;  // rows processed one workgroup per row
   uint32_t *rowbins;    // stable bin permutation: short | wave | block rows
+                        // (null when all rows are short)
   int16_t *dcol;        // nnz or null: row-block entries' column - (block's
                         // first row + cshift) (valid only in the row blocks)
   uint32_t cshift;      // 0, or a row part's first row in the whole matrix
@@ -83,6 +84,14 @@ struct gbd_matrix {
   uint32_t holders;   // batch slots holding pointers into the plan: while
                       // nonzero the plan must not be rebuilt or freed
 };
+
+// the plan's wave rows and block rows
+static inline const uint32_t *gb_wave_rows(const gbd_matrix *m) {
+  return m->rowbins ? m->rowbins + (m->nrows - m->nwave - m->nblockrows) : nullptr;
+}
+static inline const uint32_t *gb_block_rows(const gbd_matrix *m) {
+  return m->rowbins ? m->rowbins + (m->nrows - m->nblockrows) : nullptr;
+}
 
 #define GB_SPLIT_MAX 64
 // columns of x an x-tile plan stages in LDS at most

@@ -530,3 +530,54 @@ def test_pipelined_row_blocks_same_bits(gb, oracle, grid, wide_values):
     xr, it, _, _ = oracle.cgd(rp, ri, rv, b, 1e-10 * np.linalg.norm(b))
     assert i1.status == 1 and abs(int(i1.niter) - it) <= 2
     assert np.linalg.norm(b - oracle.spmv(rp, ri, rv, x1)) <= 1.05e-10 * np.linalg.norm(b)
+
+
+def _plan_counts(rp, p):
+    # row blocks, wave rows, block rows and length histogram, row by row
+    rp = rp.astype(np.int64)
+    n = rp.size - 1
+    ln = np.diff(rp)
+    cls = np.where(ln <= p["short_max"], 0, np.where(ln <= p["wave_max"], 1, 2))
+    w = rp[:-1] // p["window"]
+    pw = np.concatenate([[-1], w[:-1]])
+    pc = np.concatenate([[1], cls[:-1]])
+    first = np.maximum.accumulate(np.where(pw != w, np.arange(n), 0))
+    start = (pc != 0) | (pw != w) | ((np.arange(n) - first) % p["rowcap"] == 0)
+    hist = np.bincount(np.floor(np.log2(ln + 1)).astype(int), minlength=33)
+    return int(np.sum(start & (cls == 0))), int(np.sum(cls == 1)), int(np.sum(cls == 2)), hist
+
+
+# 64 rows a wavefront, 262144 rows a turn of the largest grid; runs of empty
+# rows make windows begin far before the wavefront that asks for them
+@pytest.mark.parametrize("n,shape", [(1, "mixed"), (63, "mixed"), (64, "mixed"), (65, "mixed"),
+                                     (257, "empty"), (5000, "mixed"), (262145, "gaps"),
+                                     (300000, "stencil")])
+@pytest.mark.parametrize("plan", [None, {"window": 64, "rowcap": 7, "short_max": 3,
+                                         "wave_max": 20}])
+def test_plan_row_blocks(gb, oracle, n, shape, plan):
+    rng = np.random.default_rng(n)
+    if shape == "mixed":
+        deg = rng.integers(0, 12, n)
+        deg[rng.integers(0, n, 1 + n // 40)] = 150
+        deg[n // 2] = 6000
+    elif shape == "empty":
+        deg = np.zeros(n, np.int64)
+    elif shape == "gaps":
+        deg = np.zeros(n, np.int64)
+        deg[::9001] = 40
+        deg[5::7001] = 3
+    else:
+        deg = np.full(n, 7)
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+    ri = rng.integers(0, n, int(rp[-1])).astype(np.uint32)
+    rv, x = rng.uniform(-1, 1, ri.size), rng.uniform(-1, 1, n)
+    M = gb.Matrix(rp, ri, rv, ncols=n, plan=plan)
+    i = M.info()
+    nst, nw, nb, hist = _plan_counts(rp, i["plan"])
+    assert (i["nblocks_stream"], i["nrows_wave"], i["nrows_block"]) == (nst, nw, nb)
+    assert i["hist"] == hist.tolist()
+    ref = oracle.spmult(n, n, 1, rp, ri, rv, x)
+    # |sum - fl(sum)| <= (len - 1) eps sum |terms| for either order
+    mag = np.add.reduceat(np.append(np.abs(rv * x[ri]), 0.0), rp[:-1].astype(np.int64))
+    mag[deg == 0] = 0.0
+    assert np.all(np.abs(M.spmv(x) - ref) <= 2 * np.maximum(deg, 1) * 2.3e-16 * mag)
