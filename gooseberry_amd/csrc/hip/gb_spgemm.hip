@@ -131,6 +131,7 @@ gb_sg_classify(uint32_t anrows, uint32_t bncols, const uint32_t *__restrict__ ar
     atomicAdd(&count[threadIdx.x], h[threadIdx.x]);
 }
 
+#define GB_SG_PER 16       // rows of a wavefront at most (one lane each for their bounds)
 #define GB_SG_HASH_BITS 7
 #define GB_SG_HASH (1u << GB_SG_HASH_BITS)  // slots per wavefront row (>= 2 x 64)
 #define GB_SG_EMPTY 0xffffffffu            // no column reaches 2^32 - 1
@@ -142,11 +143,29 @@ __device__ __forceinline__ void gb_sg_wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// One wavefront per short row.  COUNT: cnt[i] = distinct columns; FILL:
-// the row's entries at crowptr[i]; DENSE: the sums into cdense row i.
+// a product and the next lane whose product goes to the same column (its own
+// lane at the end): a column's products are walked by one 16-byte LDS read and
+// four instructions each
+struct __align__(16) gb_sg_link {
+  double val;
+  uint32_t next;
+};
+
+// Short rows, `per` consecutive list rows per wavefront (gb_sg_per).  A row is
+// a chain of three loads (A's entries, the B rows' bounds, B's entries), so
+// the next row's bounds and the one after's entries are loaded while a row's
+// products are added.  COUNT: cnt[i] = distinct columns; FILL: the row's
+// entries at crowptr[i]; DENSE: the sums into cdense row i; STAGE: cnt[i], and
+// the row's entries at its first product position (pbase) with a list (other
+// classes' rows are staged between), without one all rows of the wavefront
+// one after another from the first one's position on: they have at most as
+// many entries as products.  (A row
+// to a wavefront, each staged at its own first product: 347 us for 729,000
+// rows of 49 products and 25 columns, now 260; the stage's lines half empty,
+// 124 us to put them in place, now 85.)
 template <int MODE>
 __global__ void __launch_bounds__(GB_BLOCK)
-gb_sg_wave(uint32_t nlist, const uint32_t *__restrict__ list,
+gb_sg_wave(uint32_t nlist, uint32_t per, const uint32_t *__restrict__ list,
            const uint32_t *__restrict__ arowptr, const uint32_t *__restrict__ arowind,
            const double *__restrict__ arowval, const uint32_t *__restrict__ browptr,
            const uint32_t *__restrict__ browind, const double *__restrict__ browval,
@@ -156,97 +175,127 @@ gb_sg_wave(uint32_t nlist, const uint32_t *__restrict__ list,
            const uint32_t *__restrict__ pbase) {
   __shared__ uint32_t hkey[GB_WAVES_PER_BLOCK][GB_SG_HASH];
   __shared__ unsigned long long hmask[GB_WAVES_PER_BLOCK][GB_SG_HASH];
-  __shared__ double hval[GB_WAVES_PER_BLOCK][GB_WAVE];
-  const uint32_t w = blockIdx.x * GB_WAVES_PER_BLOCK + threadIdx.x / GB_WAVE;
+  __shared__ gb_sg_link hlink[GB_WAVES_PER_BLOCK][GB_WAVE];
   const uint32_t lane = threadIdx.x & (GB_WAVE - 1);
-  if (w >= nlist) return;  // the whole wavefront
-  // one row per wavefront: its scalars live in scalar registers
-  const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)(list ? list[w] : w));
-  const uint32_t j0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)arowptr[i]);
-  const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)arowptr[i + 1]) - j0;
-  // lane a < m: A entry j0 + a and the B row it selects
-  uint32_t bstart = 0, blen = 0;
-  double x = 0.0;
-  if (lane < m) {
-    const uint32_t l = arowind[j0 + lane];
-    bstart = browptr[l];
-    blen = browptr[l + 1] - bstart;
-    x = arowval[j0 + lane];
-  }
-  const uint32_t incl = gb_wave_scan_incl(blen);
-  const uint32_t excl = incl - blen;
-  const uint32_t P = (uint32_t)__builtin_amdgcn_readlane((int)incl, GB_WAVE - 1);  // <= 64
-  // product t = lane comes from the last A entry a whose products start at
-  // or before t (entries selecting empty rows start where the next starts)
-  uint32_t a = 0;
-  for (uint32_t u = 0; u < m; ++u)
-    if ((uint32_t)__builtin_amdgcn_readlane((int)excl, (int)u) <= lane) a = u;
-  const uint32_t ex_a = (uint32_t)__shfl((int)excl, (int)a, GB_WAVE);
-  const uint32_t bs_a = (uint32_t)__shfl((int)bstart, (int)a, GB_WAVE);
-  const double x_a = __shfl(x, (int)a, GB_WAVE);
-  const bool live = lane < P;
-  uint32_t col = 0xffffffffu;
-  double val = 0.0;
-  if (live) {
-    const uint32_t k = bs_a + (lane - ex_a);
-    col = browind[k];
-    val = x_a * browval[k];
-  }
-  // the row's columns in a small LDS hash table: slot -> column and the
-  // mask of lanes holding it; a lane is its column's head when no lower
-  // lane is in the mask, and the head adds the other lanes' products in
-  // lane (= scan) order
+  const uint64_t w0 = ((uint64_t)blockIdx.x * GB_WAVES_PER_BLOCK + threadIdx.x / GB_WAVE) * per;
+  if (w0 >= nlist) return;  // the whole wavefront
+  const uint32_t nrow = (uint32_t)__builtin_amdgcn_readfirstlane(
+      (int)(nlist - w0 < per ? (uint32_t)(nlist - w0) : per));
   uint32_t *key = hkey[threadIdx.x / GB_WAVE];
   unsigned long long *msk = hmask[threadIdx.x / GB_WAVE];
-  double *hv = hval[threadIdx.x / GB_WAVE];
-  key[lane] = GB_SG_EMPTY;
-  key[lane + GB_WAVE] = GB_SG_EMPTY;
-  msk[lane] = 0ull;
-  msk[lane + GB_WAVE] = 0ull;
-  hv[lane] = val;
-  gb_sg_wave_sync();
-  uint32_t slot = 0;
-  if (live) {
-    uint32_t h = (col * 2654435761u) >> (32 - GB_SG_HASH_BITS);
-    for (;;) {  // at most 64 columns in 128 slots: a free or equal slot exists
-      const uint32_t prev = atomicCAS(&key[h], GB_SG_EMPTY, col);
-      if (prev == GB_SG_EMPTY || prev == col) break;
-      h = (h + 1) & (GB_SG_HASH - 1);
-    }
-    slot = h;
-    atomicOr(&msk[slot], 1ull << lane);
+  gb_sg_link *lnk = hlink[threadIdx.x / GB_WAVE];
+  // lane r < nrow: row r's number, A entries, place and entries
+  uint32_t ri = 0, rj = 0, rm = 0, ro = 0, rcnt = 0;
+  if (lane < nrow) {
+    ri = list ? list[w0 + lane] : (uint32_t)w0 + lane;
+    rj = arowptr[ri];
+    rm = arowptr[ri + 1] - rj;
+    if (MODE == GB_SG_FILL) ro = crowptr[ri];
+    if (MODE == GB_SG_STAGE) ro = pbase[rj];
   }
-  gb_sg_wave_sync();
-  bool head = false;
-  double sum = 0.0;
-  if (live) {
-    const unsigned long long mk = msk[slot];
-    head = (mk & ((1ull << lane) - 1ull)) == 0;
-    if (head && MODE != GB_SG_COUNT) {
-      sum = MODE == GB_SG_DENSE ? 0.0 + val : val;
-      unsigned long long rest = mk & ~((2ull << lane) - 1ull);  // lanes above this one
-      while (rest) {
-        sum += hv[__ffsll(rest) - 1];
-        rest &= rest - 1ull;
+  const bool placed = MODE == GB_SG_FILL || list;  // each row at its own place
+  uint32_t o = (uint32_t)__builtin_amdgcn_readfirstlane((int)ro);
+  // lane a < m: A entry a of a row (its column l, one row ahead), the B row
+  // it selects and its value
+  uint32_t l = 0, bstart = 0, bend = 0;
+  double x = 0.0;
+  auto load_a = [&](uint32_t r) {
+    const uint32_t j0 = (uint32_t)__builtin_amdgcn_readlane((int)rj, (int)r);
+    if (lane < (uint32_t)__builtin_amdgcn_readlane((int)rm, (int)r)) l = arowind[j0 + lane];
+  };
+  auto load_b = [&](uint32_t r) {
+    const uint32_t j0 = (uint32_t)__builtin_amdgcn_readlane((int)rj, (int)r);
+    bstart = bend = 0;
+    if (lane < (uint32_t)__builtin_amdgcn_readlane((int)rm, (int)r)) {
+      bstart = browptr[l];
+      bend = browptr[l + 1];
+      x = arowval[j0 + lane];
+    }
+  };
+  load_a(0);
+  load_b(0);
+  if (nrow > 1) load_a(1);
+  for (uint32_t r = 0; r < nrow; ++r) {
+    const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)rm, (int)r);
+    const uint32_t blen = bend - bstart;
+    const uint32_t incl = gb_wave_scan_incl(blen);
+    const uint32_t excl = incl - blen;
+    const uint32_t P = (uint32_t)__builtin_amdgcn_readlane((int)incl, GB_WAVE - 1);  // <= 64
+    // product t = lane comes from the last A entry a whose products start at
+    // or before t (entries selecting empty rows start where the next starts)
+    uint32_t a = 0;
+    for (uint32_t u = 0; u < m; ++u)
+      if ((uint32_t)__builtin_amdgcn_readlane((int)excl, (int)u) <= lane) a = u;
+    const uint32_t k0 =
+        (uint32_t)__shfl((int)(bstart - excl), (int)a, GB_WAVE);  // mod 2^32
+    const double x_a = __shfl(x, (int)a, GB_WAVE);
+    const bool live = lane < P;
+    uint32_t col = 0xffffffffu;
+    double bv = 0.0;
+    if (live) {
+      const uint32_t k = k0 + lane;
+      col = browind[k];
+      bv = browval[k];
+    }
+    if (r + 1 < nrow) load_b(r + 1);
+    if (r + 2 < nrow) load_a(r + 2);
+    // the row's columns in a small LDS hash table: slot -> column and the
+    // mask of lanes holding it; a lane is its column's head when no lower
+    // lane is in the mask, and the head adds the other lanes' products in
+    // lane (= scan) order, each lane naming the next
+    key[lane] = GB_SG_EMPTY;
+    key[lane + GB_WAVE] = GB_SG_EMPTY;
+    msk[lane] = 0ull;
+    msk[lane + GB_WAVE] = 0ull;
+    gb_sg_wave_sync();
+    uint32_t slot = 0;
+    if (live) {
+      uint32_t h = (col * 2654435761u) >> (32 - GB_SG_HASH_BITS);
+      for (;;) {  // at most 64 columns in 128 slots: a free or equal slot exists
+        const uint32_t prev = atomicCAS(&key[h], GB_SG_EMPTY, col);
+        if (prev == GB_SG_EMPTY || prev == col) break;
+        h = (h + 1) & (GB_SG_HASH - 1);
+      }
+      slot = h;
+      atomicOr(&msk[slot], 1ull << lane);
+    }
+    gb_sg_wave_sync();
+    const unsigned long long mk = live ? msk[slot] : 0ull;
+    const bool head = live && (mk & ((1ull << lane) - 1ull)) == 0;
+    double sum = 0.0;
+    if (MODE != GB_SG_COUNT) {
+      const double val = x_a * bv;
+      const unsigned long long rest = mk & ~((2ull << lane) - 1ull);  // lanes above this one
+      uint32_t next = rest ? (uint32_t)__builtin_ctzll(rest) : lane;
+      lnk[lane] = {val, next};
+      gb_sg_wave_sync();
+      if (head) {
+        sum = MODE == GB_SG_DENSE ? 0.0 + val : val;
+        for (uint32_t at = lane; next != at;) {
+          at = next;
+          const gb_sg_link q = lnk[at];
+          sum += q.val;
+          next = q.next;
+        }
       }
     }
-  }
-  const uint64_t heads = __ballot(head);
-  if (MODE == GB_SG_COUNT || MODE == GB_SG_STAGE) {
-    if (lane == 0) cnt[i] = (uint32_t)__popcll(heads);
-  }
-  if (MODE != GB_SG_COUNT && head) {
+    const uint64_t heads = __ballot(head);
+    const uint32_t n = (uint32_t)__popcll(heads);
+    if (lane == r) rcnt = n;
     if (MODE == GB_SG_FILL || MODE == GB_SG_STAGE) {
-      // STAGE: the row's staging slots start at its first product position
-      // (pbase[j0]) and it has at most P <= its product count entries
-      const uint32_t rank = (uint32_t)__popcll(heads & ((1ull << lane) - 1ull));
-      const uint32_t o = (MODE == GB_SG_FILL ? crowptr[i] : pbase[j0]) + rank;
-      crowind[o] = col;
-      crowval[o] = sum;
-    } else {
-      cdense[(size_t)i * bncols + col] = sum;
+      if (placed) o = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)r);
+      if (head) {
+        const uint32_t at = o + (uint32_t)__popcll(heads & ((1ull << lane) - 1ull));
+        crowind[at] = col;
+        crowval[at] = sum;
+      }
+      o += n;
     }
+    if (MODE == GB_SG_DENSE && head)
+      cdense[(size_t)(uint32_t)__builtin_amdgcn_readlane((int)ri, (int)r) * bncols + col] = sum;
+    gb_sg_wave_sync();
   }
+  if ((MODE == GB_SG_COUNT || MODE == GB_SG_STAGE) && lane < nrow) cnt[ri] = rcnt;
 }
 
 // One wavefront (and workgroup) per medium row of at most CAP distinct
@@ -424,46 +473,47 @@ gb_sg_unstage_wave(uint32_t nlist, const uint32_t *__restrict__ list,
   }
 }
 
-// the staged short rows to their places, GB_BLOCK list rows per workgroup:
-// row i's cnt[i] entries from its staging slots (pbase[arowptr[i]] on) to
-// crowptr[i] on.  The workgroup numbers its rows' entries k = 0, 1, ...
-// (a scan of the counts); thread t copies entries t, t + GB_BLOCK, ...,
-// finding each one's row by binary search over the scan, so consecutive
-// entries go to consecutive places.
+// the staged short rows to their places, one wavefront per gb_sg_wave
+// wavefront of `per` list rows.  Without a list they lie one after another in
+// the stage and in C, one copy; else four rows at a time, 16 lanes a row.
 __global__ void __launch_bounds__(GB_BLOCK)
-gb_sg_unstage(uint32_t nlist, const uint32_t *__restrict__ list,
+gb_sg_unstage(uint32_t nlist, uint32_t per, const uint32_t *__restrict__ list,
               const uint32_t *__restrict__ arowptr, const uint32_t *__restrict__ pbase,
               const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ sind,
               const double *__restrict__ sval, const uint32_t *__restrict__ crowptr,
               uint32_t *__restrict__ crowind, double *__restrict__ crowval) {
-  __shared__ uint32_t lds4[GB_WAVES_PER_BLOCK];
-  __shared__ uint32_t first[GB_BLOCK + 1];  // block entry number of each row's first
-  __shared__ uint32_t src[GB_BLOCK], dst[GB_BLOCK];
-  const uint32_t w = blockIdx.x * GB_BLOCK + threadIdx.x;
-  uint32_t c = 0;
-  if (w < nlist) {
-    const uint32_t i = list ? list[w] : w;
-    c = cnt[i];
-    src[threadIdx.x] = pbase[arowptr[i]];
-    dst[threadIdx.x] = crowptr[i];
-  }
-  uint32_t total = 0;
-  const uint32_t e = gb_block_scan_excl(c, lds4, &total);
-  first[threadIdx.x] = e;
-  if (threadIdx.x == 0) first[GB_BLOCK] = total;
-  __syncthreads();
-  for (uint32_t k = threadIdx.x; k < total; k += GB_BLOCK) {
-    // the last row r with first[r] <= k (rows without entries share their
-    // first with the next row, and the search skips them)
-    uint32_t lo = 0, hi = GB_BLOCK - 1;
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi + 1) / 2;
-      if (first[mid] <= k) lo = mid;
-      else hi = mid - 1;
+  const uint32_t lane = threadIdx.x & (GB_WAVE - 1);
+  const uint64_t w0 = ((uint64_t)blockIdx.x * GB_WAVES_PER_BLOCK + threadIdx.x / GB_WAVE) * per;
+  if (w0 >= nlist) return;
+  const uint32_t nrow = (uint32_t)__builtin_amdgcn_readfirstlane(
+      (int)(nlist - w0 < per ? (uint32_t)(nlist - w0) : per));
+  if (!list) {
+    const uint32_t i0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)w0);
+    const size_t from = pbase[arowptr[i0]], to = crowptr[i0];
+    const uint32_t n = crowptr[i0 + nrow] - (uint32_t)to;
+#pragma unroll 4
+    for (uint32_t q = lane; q < n; q += GB_WAVE) {
+      crowind[to + q] = sind[from + q];
+      crowval[to + q] = sval[from + q];
     }
-    const uint32_t d = k - first[lo];
-    crowind[dst[lo] + d] = sind[src[lo] + d];
-    crowval[dst[lo] + d] = sval[src[lo] + d];
+    return;
+  }
+  uint32_t c = 0, src = 0, dst = 0;
+  if (lane < nrow) {
+    const uint32_t i = list[w0 + lane];
+    c = cnt[i];
+    src = pbase[arowptr[i]];
+    dst = crowptr[i];
+  }
+  for (uint32_t r4 = 0; r4 < nrow; r4 += GB_WAVE / 16u) {
+    const uint32_t r = r4 + lane / 16u;  // lanes from nrow on hold no entries
+    const uint32_t n = (uint32_t)__shfl((int)c, (int)r, GB_WAVE);
+    const size_t from = (uint32_t)__shfl((int)src, (int)r, GB_WAVE);
+    const size_t to = (uint32_t)__shfl((int)dst, (int)r, GB_WAVE);
+    for (uint32_t q = lane & 15u; q < n; q += 16u) {
+      crowind[to + q] = sind[from + q];
+      crowval[to + q] = sval[from + q];
+    }
   }
 }
 
@@ -623,6 +673,18 @@ static uint32_t gb_sg_grid(uint64_t n) {
   return g ? (uint32_t)g : 1u;
 }
 
+// short rows per wavefront: one until the launch fills the GPU's wavefronts
+// (8192) twice, then more, so that their loads overlap and the stage is dense.
+// The whole square of a 3D stencil of 729,000 rows took 1092 us at one row,
+// 863 at 4, 857 at 8, 851 at 16; of 262,000 rows 603, 551, 545 and 549.
+static uint32_t gb_sg_per(uint32_t nshort) {
+  const uint32_t per = nshort / 16384u;
+  return per < 1u ? 1u : (per > GB_SG_PER ? GB_SG_PER : per);
+}
+static uint32_t gb_sg_short_grid(uint32_t nshort) {
+  return gb_div_up(nshort, GB_WAVES_PER_BLOCK * gb_sg_per(nshort));
+}
+
 // the medium rows of one class in one mode (dense and the staged or final
 // arrays as the short rows' kernel takes them)
 template <int MODE>
@@ -752,14 +814,14 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
       GB_SG_TRY(gb_dev_alloc((void **)&sval, (size_t)e64 * 8));
     }
     if (nshort && staged) {
-      gb_sg_wave<GB_SG_STAGE><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, list, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
-          nullptr, cnt, sind, sval, nullptr, 0, off);
+      gb_sg_wave<GB_SG_STAGE><<<gb_sg_short_grid(nshort), GB_BLOCK, 0, s>>>(
+          nshort, gb_sg_per(nshort), list, d_arowptr, d_arowind, d_arowval, d_browptr,
+          d_browind, d_browval, nullptr, cnt, sind, sval, nullptr, 0, off);
       GB_SG_TRY(hipGetLastError());
     } else if (nshort) {
-      gb_sg_wave<GB_SG_COUNT><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, list, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
-          nullptr, cnt, nullptr, nullptr, nullptr, 0, nullptr);
+      gb_sg_wave<GB_SG_COUNT><<<gb_sg_short_grid(nshort), GB_BLOCK, 0, s>>>(
+          nshort, gb_sg_per(nshort), list, d_arowptr, d_arowind, d_arowval, d_browptr,
+          d_browind, d_browval, nullptr, cnt, nullptr, nullptr, nullptr, 0, nullptr);
       GB_SG_TRY(hipGetLastError());
     }
     if (nmed && staged)
@@ -772,9 +834,9 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
                                           nullptr, nullptr, nullptr, 0, nullptr));
   } else {
     if (nshort) {
-      gb_sg_wave<GB_SG_DENSE><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, list, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
-          nullptr, nullptr, nullptr, nullptr, d_cdense, bncols, nullptr);
+      gb_sg_wave<GB_SG_DENSE><<<gb_sg_short_grid(nshort), GB_BLOCK, 0, s>>>(
+          nshort, gb_sg_per(nshort), list, d_arowptr, d_arowind, d_arowval, d_browptr,
+          d_browind, d_browval, nullptr, nullptr, nullptr, nullptr, d_cdense, bncols, nullptr);
       GB_SG_TRY(hipGetLastError());
     }
     if (nmed)
@@ -854,13 +916,14 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
     GB_SG_TRY(gb_dev_alloc((void **)&crowind, ((size_t)cnnz + 1) * 4));
     GB_SG_TRY(gb_dev_alloc((void **)&crowval, ((size_t)cnnz + 1) * 8));
     if (nshort && staged) {
-      gb_sg_unstage<<<gb_div_up(nshort, GB_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, list, d_arowptr, off, cnt, sind, sval, crowptr, crowind, crowval);
+      gb_sg_unstage<<<gb_sg_short_grid(nshort), GB_BLOCK, 0, s>>>(
+          nshort, gb_sg_per(nshort), list, d_arowptr, off, cnt, sind, sval, crowptr, crowind,
+          crowval);
       GB_SG_TRY(hipGetLastError());
     } else if (nshort) {
-      gb_sg_wave<GB_SG_FILL><<<gb_div_up(nshort, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(
-          nshort, list, d_arowptr, d_arowind, d_arowval, d_browptr, d_browind, d_browval,
-          crowptr, nullptr, crowind, crowval, nullptr, 0, nullptr);
+      gb_sg_wave<GB_SG_FILL><<<gb_sg_short_grid(nshort), GB_BLOCK, 0, s>>>(
+          nshort, gb_sg_per(nshort), list, d_arowptr, d_arowind, d_arowval, d_browptr,
+          d_browind, d_browval, crowptr, nullptr, crowind, crowval, nullptr, 0, nullptr);
       GB_SG_TRY(hipGetLastError());
     }
     if (nmed && staged) {

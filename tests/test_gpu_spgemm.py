@@ -98,6 +98,39 @@ def test_spgemm_row_classes(gb, oracle, bncols, stage, monkeypatch):
         assert np.array_equal(bits(dense), bits(oracle.spmultsp(a, b, bncols)))
 
 
+@pytest.mark.parametrize("stage", ["staged", "two_pass"])
+@pytest.mark.parametrize("n,mixed", [(32767, False), (32769, False), (70001, True),
+                                     (270001, False), (270001, True)])
+def test_spgemm_rows_per_wavefront(gb, oracle, n, mixed, stage, monkeypatch):
+    # up to 16 consecutive short rows go to a wavefront (from 32768 rows on),
+    # one after another in the stage unless rows of other classes lie between
+    if stage == "two_pass":
+        monkeypatch.setenv("GOOSEBERRY_SPGEMM_STAGE_MAX", "0")
+    rng = np.random.default_rng(n)
+    k, bncols = 300, 60
+    blen = rng.integers(0, 12, k)
+    blen[0], blen[1], blen[2] = 64, 32, 0
+    brp = np.concatenate([[0], np.cumsum(blen)]).astype(np.uint32)
+    b = (brp, rng.integers(0, bncols, brp[-1]).astype(np.uint32), rng.uniform(-1, 1, brp[-1]))
+    m = rng.integers(0, 6, n)  # at most 5 entries of 11 products
+    m[[7, 1000, n - 1]] = 1
+    if mixed:
+        m[rng.integers(0, n, n // 50)] = 12
+    arp = np.concatenate([[0], np.cumsum(m)]).astype(np.uint32)
+    ari = rng.integers(2, k, int(arp[-1])).astype(np.uint32)
+    if not mixed:
+        ari[arp[[7, 1000, n - 1]]] = [0, 1, 0]  # rows of 64, 32 and 64 products
+    a = (arp, ari, rng.uniform(-1, 1, ari.size))
+    print("spgemm rows per wavefront", n, mixed, stage, flush=True)
+    rp, ri, rv = gb.spmultsp_sp(n, k, bncols, a, b)
+    orp, ori, orv = oracle.spmultsp_sp(a, b, bncols)
+    assert np.array_equal(rp, orp) and np.array_equal(ri, ori)
+    assert np.array_equal(bits(rv), bits(orv))
+    if stage == "staged":
+        assert np.array_equal(bits(gb.spmultsp(n, k, bncols, a, b)),
+                              bits(oracle.spmultsp(a, b, bncols)))
+
+
 def test_spgemm_one_medium_class(gb, oracle):
     # every row in one class of medium rows (no list of rows is made), with
     # a negative zero that a lone product keeps and the dense result turns
