@@ -411,8 +411,7 @@ static int gb_cm_block(uint32_t start, uint32_t end, const uint32_t *rowptr,
   // the least-degree order of the block's vertices, equal degrees by
   // vertex; no degree exceeds the block rows' entry count
   GB_CM_TRY(hipMemcpyAsync(&h[0], rowptr + start, 4, hipMemcpyDeviceToHost, s));
-  GB_CM_TRY(hipMemcpyAsync(&h[1], rowptr + end, 4, hipMemcpyDeviceToHost, s));
-  GB_CM_TRY(hipStreamSynchronize(s));
+  GB_CM_TRY(gb_fetch(&h[1], rowptr + end, 4));
   maxdeg = h[1] - h[0];
   GB_CM_RV(gbd_countingsort_kv_unchecked(deg, nullptr, 0, maxdeg, nb, S, nullptr));
   gb_cm_rank<<<gb_cm_grid(nb), GB_BLOCK, 0, s>>>(nb, S, srank);
@@ -429,18 +428,15 @@ static int gb_cm_block(uint32_t start, uint32_t end, const uint32_t *rowptr,
     gb_cm_find<false><<<gb_cm_grid(nb - cursor), GB_BLOCK, 0, s>>>(cursor, nb, S, posof, iso,
                                                                    dv);
     GB_CM_TRY(hipGetLastError());
-    GB_CM_TRY(hipMemcpyAsync(&h[1], dv, 4, hipMemcpyDeviceToHost, s));
-    GB_CM_TRY(hipStreamSynchronize(s));
+    GB_CM_TRY(gb_fetch(&h[1], dv, 4));
     const uint32_t idx = h[1];
     if (idx >= nb) {  // cannot happen while vertices remain
       rv = GOOSEBERRY_ERROR_UNKNOWN;
       goto done;
     }
     uint32_t sv = 0, siso = 0;
-    GB_CM_TRY(hipMemcpyAsync(&sv, S + idx, 4, hipMemcpyDeviceToHost, s));
-    GB_CM_TRY(hipStreamSynchronize(s));
-    GB_CM_TRY(hipMemcpyAsync(&siso, iso + sv, 4, hipMemcpyDeviceToHost, s));
-    GB_CM_TRY(hipStreamSynchronize(s));
+    GB_CM_TRY(gb_fetch(&sv, S + idx, 4));
+    GB_CM_TRY(gb_fetch(&siso, iso + sv, 4));
     if (siso) {
       // a start with no neighbour is a component of its own, and so is
       // every following unplaced one up to the first that has neighbours
@@ -448,8 +444,7 @@ static int gb_cm_block(uint32_t start, uint32_t end, const uint32_t *rowptr,
       GB_CM_TRY(hipGetLastError());
       gb_cm_find<true><<<gb_cm_grid(nb - idx), GB_BLOCK, 0, s>>>(idx, nb, S, posof, iso, dv);
       GB_CM_TRY(hipGetLastError());
-      GB_CM_TRY(hipMemcpyAsync(&h[1], dv, 4, hipMemcpyDeviceToHost, s));
-      GB_CM_TRY(hipStreamSynchronize(s));
+      GB_CM_TRY(gb_fetch(&h[1], dv, 4));
       const uint32_t f = h[1];
       gb_cm_isoflag<<<gb_cm_grid(f - idx), GB_BLOCK, 0, s>>>(idx, f, S, posof, flag);
       GB_CM_TRY(hipGetLastError());
@@ -475,8 +470,7 @@ static int gb_cm_block(uint32_t start, uint32_t end, const uint32_t *rowptr,
         gb_cm_serial<<<1, GB_BLOCK, 0, s>>>(start, end, rowptr, rowind, srank, posof, claim,
                                             perm, dv + 1);
         GB_CM_TRY(hipGetLastError());
-        GB_CM_TRY(hipMemcpyAsync(h, dv + 1, 12, hipMemcpyDeviceToHost, s));
-        GB_CM_TRY(hipStreamSynchronize(s));
+        GB_CM_TRY(gb_fetch(h, dv + 1, 12));
         sr = h[0];
         no = h[1];
         if (h[2] == 0) break;     // component done
@@ -490,8 +484,7 @@ static int gb_cm_block(uint32_t start, uint32_t end, const uint32_t *rowptr,
                                                           perm, posof, claim, list, dv + 1);
       GB_CM_TRY(hipGetLastError());
       uint32_t L = 0;
-      GB_CM_TRY(hipMemcpyAsync(&L, dv + 1, 4, hipMemcpyDeviceToHost, s));
-      GB_CM_TRY(hipStreamSynchronize(s));
+      GB_CM_TRY(gb_fetch(&L, dv + 1, 4));
       if (L && L <= GB_CM_LDS_SORT && no - sr <= GB_CM_LDS_SORT) {
         gb_cm_segplace<<<1, GB_CM_SORT_THREADS, 0, s>>>(L, sr, no, no, start, list, claim,
                                                        srank, S, posof, perm);

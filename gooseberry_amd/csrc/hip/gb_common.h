@@ -37,6 +37,8 @@ int gb_ensure_init();
 // pool (no device-wide synchronisation, no trip to the driver per request).
 hipError_t gb_dev_alloc(void **p, size_t bytes);
 hipError_t gb_dev_free(void *p);
+// a small result to the host, waiting for the stream
+hipError_t gb_fetch(void *h_dst, const void *d_src, size_t bytes);
 bool gb_graphs_enabled();  // false when GOOSEBERRY_NO_GRAPHS is set
 uint32_t gb_num_cus();     // compute units of the device
 

@@ -237,8 +237,7 @@ int gbd_generate_spd(uint32_t n, uint64_t seed, int law, double zipf_s,
   GB_GEN_TRY(hipGetLastError());
   gb_gen_sum64<<<grid < 1024u ? grid : 1024u, GB_BLOCK, 0, s>>>(off, n, tot);
   GB_GEN_TRY(hipGetLastError());
-  GB_GEN_TRY(hipMemcpyAsync(&m64, tot, sizeof(m64), hipMemcpyDeviceToHost, s));
-  GB_GEN_TRY(hipStreamSynchronize(s));
+  GB_GEN_TRY(gb_fetch(&m64, tot, sizeof(m64)));
   // every index and row pointer of the result must fit 32 bits
   if (2 * m64 + n > 0xffffffffull) {
     rv = GOOSEBERRY_ERROR_INVALIDINPUT;

@@ -796,8 +796,7 @@ int gbd_parse_csr(const char *d_txt, uint64_t len, uint32_t *r_nrows, uint32_t *
   }
   GB_IN_RV(gbd_scan_u32(ccnt, ccnt, nchunks, ccnt + nchunks));
   GB_IN_RV(gbd_scan_u32(tcnt, tcnt, nchunks, tcnt + nchunks));
-  GB_IN_TRY(hipMemcpyAsync(&nl, ccnt + nchunks, 4, hipMemcpyDeviceToHost, s));
-  GB_IN_TRY(hipStreamSynchronize(s));
+  GB_IN_TRY(gb_fetch(&nl, ccnt + nchunks, 4));
   if (nl == 0xffffffffu) {
     rv = GOOSEBERRY_ERROR_INVALIDINPUT;
     goto done;
@@ -842,8 +841,7 @@ int gbd_parse_csr(const char *d_txt, uint64_t len, uint32_t *r_nrows, uint32_t *
         GB_IN_TRY(hipGetLastError());
       }
     }
-    GB_IN_TRY(hipMemcpyAsync(&h, meta, sizeof(h), hipMemcpyDeviceToHost, s));
-    GB_IN_TRY(hipStreamSynchronize(s));
+    GB_IN_TRY(gb_fetch(&h, meta, sizeof(h)));
     if (h.total > 0xffffffffull) {
       if (!general) continue;
       rv = GOOSEBERRY_ERROR_INVALIDINPUT;  // beyond 32-bit row pointers
@@ -882,8 +880,7 @@ int gbd_parse_csr(const char *d_txt, uint64_t len, uint32_t *r_nrows, uint32_t *
             rowval, fix, fixcap, &meta->nfix);
         GB_IN_TRY(hipGetLastError());
       }
-      GB_IN_TRY(hipMemcpyAsync(&h, meta, sizeof(h), hipMemcpyDeviceToHost, s));
-      GB_IN_TRY(hipStreamSynchronize(s));
+      GB_IN_TRY(gb_fetch(&h, meta, sizeof(h)));
       if (h.odd || h.nfix <= fixcap) break;
     }
     if (h.odd) continue;  // not plain text
@@ -968,8 +965,7 @@ int gbd_parse_mtx_body(const char *d_txt, uint64_t len, uint64_t off, uint32_t n
     GB_MX_TRY(hipGetLastError());
   }
   GB_MX_RV(gbd_scan_u32(ccnt, ccnt, nchunks, ccnt + nchunks));
-  GB_MX_TRY(hipMemcpyAsync(&nl, ccnt + nchunks, 4, hipMemcpyDeviceToHost, s));
-  GB_MX_TRY(hipStreamSynchronize(s));
+  GB_MX_TRY(gb_fetch(&nl, ccnt + nchunks, 4));
   if (nl == 0xffffffffu) {
     rv = GOOSEBERRY_ERROR_INVALIDINPUT;
     goto done;
@@ -979,8 +975,7 @@ int gbd_parse_mtx_body(const char *d_txt, uint64_t len, uint64_t off, uint32_t n
     gb_in_nl_pos<false><<<(uint32_t)nchunks, GB_BLOCK, 0, s>>>(txt, blen, ccnt, nullptr, ls,
                                                             nullptr);
     GB_MX_TRY(hipGetLastError());
-    GB_MX_TRY(hipMemcpyAsync(&last, ls + nl, 8, hipMemcpyDeviceToHost, s));
-    GB_MX_TRY(hipStreamSynchronize(s));
+    GB_MX_TRY(gb_fetch(&last, ls + nl, 8));
   }
   nlines = nl + (blen > last ? 1u : 0u);
   // entry lines and their ranks
@@ -990,8 +985,7 @@ int gbd_parse_mtx_body(const char *d_txt, uint64_t len, uint64_t off, uint32_t n
     GB_MX_TRY(hipGetLastError());
   }
   GB_MX_RV(gbd_scan_u32(ent, ent, nlines, ent + nlines));
-  GB_MX_TRY(hipMemcpyAsync(&nent, ent + nlines, 4, hipMemcpyDeviceToHost, s));
-  GB_MX_TRY(hipStreamSynchronize(s));
+  GB_MX_TRY(gb_fetch(&nent, ent + nlines, 4));
   nnz64 = (uint64_t)nent * (sym ? 2u : 1u);
   if (nnz64 > 0xffffffffull) {
     rv = GOOSEBERRY_ERROR_INVALIDINPUT;
@@ -1014,8 +1008,7 @@ int gbd_parse_mtx_body(const char *d_txt, uint64_t len, uint64_t off, uint32_t n
       GB_MX_TRY(hipGetLastError());
     }
     GB_MX_TRY(hipMemcpyAsync(hflags, flags, 8, hipMemcpyDeviceToHost, s));
-    GB_MX_TRY(hipMemcpyAsync(&hnfix, nfix, 4, hipMemcpyDeviceToHost, s));
-    GB_MX_TRY(hipStreamSynchronize(s));
+    GB_MX_TRY(gb_fetch(&hnfix, nfix, 4));
     if (hnfix <= fixcap) break;
     (void)gb_dev_free(fix);
     fix = nullptr;

@@ -519,8 +519,7 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
   GB_PR_RV(gbd_scan_u32(flag, idx, n, idx + n));
   gb_pr_sink_compact<<<gb_div_up(n, GB_BLOCK), GB_BLOCK, 0, s>>>(n, m->rowptr, idx, sinks);
   GB_PR_TRY(hipGetLastError());
-  GB_PR_TRY(hipMemcpyAsync(&nsinks, idx + n, 4, hipMemcpyDeviceToHost, s));
-  GB_PR_TRY(hipStreamSynchronize(s));
+  GB_PR_TRY(gb_fetch(&nsinks, idx + n, 4));
 
   // the normalised matrix: the same structure and plan over nval (null with
   // a plan of its own copy: its launches read only that copy)
@@ -580,8 +579,7 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
       GB_PR_TRY(hipGetLastError());
       gb_pr_err_final<<<1, GB_BLOCK, 0, s>>>(part, GB_PR_ERR_GRID, err);
       GB_PR_TRY(hipGetLastError());
-      GB_PR_TRY(hipMemcpyAsync(&e, err, 8, hipMemcpyDeviceToHost, s));
-      GB_PR_TRY(hipStreamSynchronize(s));
+      GB_PR_TRY(gb_fetch(&e, err, 8));
       if (e <= minerror * minerror) {
         ++i;
         finished = true;

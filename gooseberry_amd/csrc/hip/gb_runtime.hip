@@ -54,6 +54,14 @@ __attribute__((constructor)) static void gb_record_load_cpus() {
   g_load_cpus_ok = sched_getaffinity(0, sizeof(g_load_cpus), &g_load_cpus) == 0;
 }
 
+// Small results for the host come through pinned slots: a copy of a few
+// bytes to pageable memory and the wait for it took 23 us, to pinned memory
+// 14.  More callers at once than slots take the pageable copy.
+#define GB_FETCH_SLOTS 32
+#define GB_FETCH_BYTES 512
+static char *g_fetch = nullptr;  // GB_FETCH_SLOTS slots, for the process
+static std::atomic<uint32_t> g_fetch_used{0};
+
 static void gb_do_init_on_device() {
   int ndev = 0;
   hipError_t e = hipGetDeviceCount(&ndev);
@@ -94,6 +102,11 @@ static void gb_do_init_on_device() {
     return;
   }
   g_cache_cap = tot / 8 < (32ull << 30) ? tot / 8 : (32ull << 30);
+  if (hipHostMalloc((void **)&g_fetch, GB_FETCH_SLOTS * GB_FETCH_BYTES,
+                    hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    g_fetch = nullptr;
+  }
   // GOOSEBERRY_NO_GRAPHS (set, not "0"): launch CG and batch steps one by
   // one instead of replaying captured graphs, for tracing tools that do not
   // follow graph launches
@@ -125,18 +138,31 @@ uint32_t gb_num_cus() {
   return g_num_cus;
 }
 
-// Large blocks (4 MiB and up, sizes rounded to 2 MiB) that the library
-// frees are kept here and handed back to a later allocation of the same
-// rounded size, the most recently freed first.  The default pool gave such blocks back to the driver at
-// free despite its release threshold: a free of a few hundred MiB took
+// Blocks that the library frees are kept here and handed back to a later
+// allocation of the same rounded size, the most recently freed first: sizes
+// are rounded to 2 MiB from 4 MiB on, below that to a quarter of the power
+// of two they reach.  The default pool gave large blocks back to the driver
+// at free despite its release threshold: a free of a few hundred MiB took
 // 0.65-2.5 ms and the next allocation of that size 50-350 us, several
-// milliseconds per sparse product.  Every library launch and copy runs on
+// milliseconds per sparse product.  Small blocks cost it 10 us a pair, and
+// 33 us where eight are allocated before they are freed: most of the 540 us
+// that a 1,000-row sparse product with its plan took, 155 with these blocks
+// kept and gb_fetch.  Every library launch and copy runs on
 // g_stream, so a block's reuse is ordered after its last use exactly as a
-// pool block's is.  The cache holds at most g_cache_cap bytes (oldest
-// blocks go back first), is emptied when an allocation finds the device
-// out of memory, and its bytes count as free in gbd_device_memory.
-#define GB_CACHE_MIN (4ull << 20)
+// pool block's is.  The cache holds at most g_cache_cap bytes and
+// GB_CACHE_BLOCKS blocks (the oldest go back first), is emptied when an
+// allocation finds the device out of memory, and its bytes count as free in
+// gbd_device_memory.
+#define GB_CACHE_LARGE (4ull << 20)
 #define GB_CACHE_ROUND (2ull << 20)
+#define GB_CACHE_BLOCKS 1024
+
+static size_t gb_cache_round(size_t bytes) {
+  if (bytes >= GB_CACHE_LARGE) return (bytes + GB_CACHE_ROUND - 1) & ~(GB_CACHE_ROUND - 1);
+  if (bytes <= 256) return 256;
+  const size_t step = (size_t)1 << (61 - __builtin_clzll(bytes));
+  return (bytes + step - 1) & ~(step - 1);
+}
 
 static std::mutex g_cache_mu;
 static std::unordered_map<void *, size_t> g_cache_live;  // handed out: size
@@ -189,8 +215,7 @@ hipError_t gb_launch_status() {
 hipError_t gb_dev_alloc(void **p, size_t bytes) {
   *p = nullptr;
   if (gb_fault_fires(GB_FAULT_ALLOC)) return hipErrorOutOfMemory;
-  if (bytes < GB_CACHE_MIN) return hipMallocAsync(p, bytes ? bytes : 16, g_stream);
-  const size_t r = (bytes + GB_CACHE_ROUND - 1) & ~(GB_CACHE_ROUND - 1);
+  const size_t r = gb_cache_round(bytes);
   {
     std::lock_guard<std::mutex> lk(g_cache_mu);
     // the block of this size freed last (its lines are the likeliest to
@@ -228,7 +253,8 @@ hipError_t gb_dev_free(void *p) {
       const size_t r = it->second;
       g_cache_live.erase(it);
       if (r <= g_cache_cap) {
-        while (g_cache_bytes + r > g_cache_cap) gb_cache_evict_oldest();
+        while (g_cache_bytes + r > g_cache_cap || g_cache_fifo.size() >= GB_CACHE_BLOCKS)
+          gb_cache_evict_oldest();
         g_cache_fifo.emplace_back(r, p);
         g_cache_free.emplace(r, std::prev(g_cache_fifo.end()));
         g_cache_bytes += r;
@@ -237,6 +263,29 @@ hipError_t gb_dev_free(void *p) {
     }
   }
   return hipFreeAsync(p, g_stream);
+}
+
+hipError_t gb_fetch(void *h_dst, const void *d_src, size_t bytes) {
+  int slot = -1;
+  if (g_fetch && bytes <= GB_FETCH_BYTES) {
+    uint32_t used = g_fetch_used.load();
+    while (used != 0xffffffffu) {
+      const int i = __builtin_ctz(~used);
+      if (g_fetch_used.compare_exchange_weak(used, used | 1u << i)) {
+        slot = i;
+        break;
+      }
+    }
+  }
+  void *to = slot < 0 ? h_dst : g_fetch + (size_t)slot * GB_FETCH_BYTES;
+  hipError_t e = hipMemcpyAsync(to, d_src, bytes, hipMemcpyDeviceToHost, g_stream);
+  const hipError_t es = hipStreamSynchronize(g_stream);
+  if (e == hipSuccess) e = es;
+  if (slot >= 0) {
+    if (e == hipSuccess) memcpy(h_dst, to, bytes);
+    g_fetch_used.fetch_and(~(1u << slot));
+  }
+  return e;
 }
 
 int gb_ensure_init() {

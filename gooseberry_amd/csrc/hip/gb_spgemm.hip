@@ -763,8 +763,7 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
         (size_t)anrows * bncols, d_cdense);
     GB_SG_TRY(hipGetLastError());
   }
-  GB_SG_TRY(hipMemcpyAsync(&annz, d_arowptr + anrows, 4, hipMemcpyDeviceToHost, s));
-  GB_SG_TRY(hipStreamSynchronize(s));
+  GB_SG_TRY(gb_fetch(&annz, d_arowptr + anrows, 4));
   GB_SG_TRY(gb_dev_alloc((void **)&len, ((size_t)annz + 1) * 4));
   GB_SG_TRY(gb_dev_alloc((void **)&off, ((size_t)annz + 1) * 4));
   // every product position must fit 32 bits: the total in 64 bits first
@@ -775,8 +774,7 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
     gb_sg_len<<<g > 1024u ? 1024u : g, GB_BLOCK, 0, s>>>(annz, d_arowind, d_browptr, len, tot);
     GB_SG_TRY(hipGetLastError());
   }
-  GB_SG_TRY(hipMemcpyAsync(&e64, tot, 8, hipMemcpyDeviceToHost, s));
-  GB_SG_TRY(hipStreamSynchronize(s));
+  GB_SG_TRY(gb_fetch(&e64, tot, 8));
   if (e64 > 0xfffffffeull) {
     rv = GOOSEBERRY_ERROR_INVALIDINPUT;
     goto done;
@@ -795,8 +793,7 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
                                                             cls, count);
     GB_SG_TRY(hipGetLastError());
   }
-  GB_SG_TRY(hipMemcpyAsync(hcount, count, GB_SG_NCLASS * 4, hipMemcpyDeviceToHost, s));
-  GB_SG_TRY(hipStreamSynchronize(s));
+  GB_SG_TRY(gb_fetch(hcount, count, GB_SG_NCLASS * 4));
   nshort = hcount[GB_SG_CSHORT];
   nlong = hcount[GB_SG_CSORT];
   nmed = anrows - nshort - nlong;
@@ -852,8 +849,7 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
                                                         len2);
     GB_SG_TRY(hipGetLastError());
     GB_SG_RV(gbd_scan_u32(len2, off2, annz, off2 + annz));
-    GB_SG_TRY(hipMemcpyAsync(&E, off2 + annz, 4, hipMemcpyDeviceToHost, s));
-    GB_SG_TRY(hipStreamSynchronize(s));
+    GB_SG_TRY(gb_fetch(&E, off2 + annz, 4));
   }
   if (E) {
     GB_SG_TRY(gb_dev_alloc((void **)&erow, (size_t)E * 4));
@@ -879,8 +875,7 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
     gb_sg_runflag<<<gb_sg_grid(E), GB_BLOCK, 0, s>>>(E, ord, erow, ecol, flag);
     GB_SG_TRY(hipGetLastError());
     GB_SG_RV(gbd_scan_u32(flag, rid, E, rid + E));
-    GB_SG_TRY(hipMemcpyAsync(&nruns, rid + E, 4, hipMemcpyDeviceToHost, s));
-    GB_SG_TRY(hipStreamSynchronize(s));
+    GB_SG_TRY(gb_fetch(&nruns, rid + E, 4));
     GB_SG_TRY(gb_dev_alloc((void **)&runstart, ((size_t)nruns + 1) * 4));
     gb_sg_runstart<<<gb_sg_grid(E), GB_BLOCK, 0, s>>>(E, flag, rid, runstart);
     GB_SG_TRY(hipGetLastError());
@@ -911,8 +906,7 @@ int gbd_spgemm(uint32_t anrows, uint32_t ancols, uint32_t bncols,
   if (!dense) {
     GB_SG_TRY(gb_dev_alloc((void **)&crowptr, ((size_t)anrows + 1) * 4));
     GB_SG_RV(gbd_scan_u32(cnt, crowptr, anrows, crowptr + anrows));
-    GB_SG_TRY(hipMemcpyAsync(&cnnz, crowptr + anrows, 4, hipMemcpyDeviceToHost, s));
-    GB_SG_TRY(hipStreamSynchronize(s));
+    GB_SG_TRY(gb_fetch(&cnnz, crowptr + anrows, 4));
     GB_SG_TRY(gb_dev_alloc((void **)&crowind, ((size_t)cnnz + 1) * 4));
     GB_SG_TRY(gb_dev_alloc((void **)&crowval, ((size_t)cnnz + 1) * 8));
     if (nshort && staged) {

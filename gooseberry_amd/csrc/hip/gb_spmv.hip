@@ -1334,8 +1334,7 @@ static int gb_vdict_build(const void *vals, int width, uint64_t nnz, uint8_t **r
   unsigned long long hk[GB_VD_GTAB];
   uint32_t hover = 0;
   GB_HIP(hipMemcpyAsync(hk, gkeys, sizeof(hk), hipMemcpyDeviceToHost, s));
-  GB_HIP(hipMemcpyAsync(&hover, over, 4, hipMemcpyDeviceToHost, s));
-  GB_HIP(hipStreamSynchronize(s));
+  GB_HIP(gb_fetch(&hover, over, 4));
   unsigned long long keys[GB_VDICT_MAX];
   uint32_t nk = 0;
   for (uint32_t i = 0; i < GB_VD_GTAB && !hover; ++i) {
@@ -1408,8 +1407,7 @@ static int gb_vdict_f32(gbd_matrix *m) {
   hipStream_t s = gb_stream();
   double h64[GB_VDICT_MAX];
   float h32[GB_VDICT_MAX];
-  GB_HIP(hipMemcpyAsync(h64, m->vtab, sizeof(h64), hipMemcpyDeviceToHost, s));
-  GB_HIP(hipStreamSynchronize(s));
+  GB_HIP(gb_fetch(h64, m->vtab, sizeof(h64)));
   for (uint32_t i = 0; i < GB_VDICT_MAX; ++i) h32[i] = (float)h64[i];
   GB_HIP(gb_dev_alloc((void **)&m->vtab32, sizeof(h32)));
   GB_HIP(hipMemcpyAsync(m->vtab32, h32, sizeof(h32), hipMemcpyHostToDevice, s));
@@ -1718,8 +1716,7 @@ static int gb_plan_build(gbd_matrix *m) {
   GB_LAUNCH_CHECK();
   int rv = gbd_scan_u32(flag, idx, n, (uint32_t *)(count + GB_PLAN_NST));
   if (rv != GOOSEBERRY_SUCCESS) return rv;
-  GB_HIP(hipMemcpyAsync(hc, count, sizeof(hc), hipMemcpyDeviceToHost, s));
-  GB_HIP(hipStreamSynchronize(s));
+  GB_HIP(gb_fetch(hc, count, sizeof(hc)));
   for (int i = 0; i < 33; ++i) m->hist[i] = hc[i];
   const uint32_t nst = (uint32_t)hc[GB_PLAN_NST];
   m->nstream = nst;
@@ -1756,8 +1753,7 @@ static int gb_plan_build(gbd_matrix *m) {
     gb_plan_narrow<<<nst, GB_BLOCK, 0, s>>>(m->rowptr, m->rowind, m->blk, m->cshift, m->dcol,
                                             bad);
     GB_LAUNCH_CHECK();
-    GB_HIP(hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, s));
-    GB_HIP(hipStreamSynchronize(s));
+    GB_HIP(gb_fetch(&hbad, bad, 4));
     GB_HIP(gb_dev_free(bad));
     if (hbad) {
       GB_HIP(gb_dev_free(m->dcol));
@@ -1818,8 +1814,7 @@ int gbd_csr_check(uint32_t nrows, uint32_t ncols, const uint32_t *d_rowptr,
   hipStream_t s = gb_stream();
   // nnz from the device, then every row pointer and column index checked
   uint32_t *bad = nullptr, hbad = 0, nnz = 0;
-  GB_HIP(hipMemcpyAsync(&nnz, d_rowptr + nrows, 4, hipMemcpyDeviceToHost, s));
-  GB_HIP(hipStreamSynchronize(s));
+  GB_HIP(gb_fetch(&nnz, d_rowptr + nrows, 4));
   GB_HIP(gb_dev_alloc((void **)&bad, 4));
   GB_HIP(hipMemsetAsync(bad, 0, 4, s));
   uint64_t work = (uint64_t)nrows > nnz ? nrows : nnz;
@@ -1888,8 +1883,7 @@ int gbd_matrix_create_trusted(uint32_t nrows, uint32_t ncols, uint32_t *d_rowptr
 // One 64-bit row pointer read back (the part boundaries' binary search).
 static int gb_rowptr64_at(const uint64_t *d_rowptr64, uint32_t i, uint64_t *v) {
   hipStream_t s = gb_stream();
-  GB_HIP(hipMemcpyAsync(v, d_rowptr64 + i, 8, hipMemcpyDeviceToHost, s));
-  GB_HIP(hipStreamSynchronize(s));
+  GB_HIP(gb_fetch(v, d_rowptr64 + i, 8));
   return GOOSEBERRY_SUCCESS;
 }
 
@@ -2205,8 +2199,7 @@ int gbd_matrix_make_f32_jacobi(gbd_matrix *m) {
     gb_jacobi_scale<<<g, GB_BLOCK, 0, s>>>(m->rowptr, m->rowind, m->val, n, m->jscale, bad);
     GB_LAUNCH_CHECK();
   }
-  GB_HIP(hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, s));
-  GB_HIP(hipStreamSynchronize(s));
+  GB_HIP(gb_fetch(&hbad, bad, 4));
   GB_HIP(gb_dev_free(bad));
   if (hbad) {
     GB_HIP(gb_dev_free(m->jscale));

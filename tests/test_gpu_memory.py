@@ -1,7 +1,7 @@
-"""Device memory: blocks of 4 MiB and up that the library frees are kept and
-handed back to the next allocation of the same rounded size (2 MiB
-granularity); the kept bytes count as free in gooseberry_device_memory; a
-reused block serves a new computation correctly."""
+"""Device memory: blocks that the library frees are kept and handed back to the
+next allocation of the same rounded size (2 MiB steps from 4 MiB on, quarters
+of a power of two below); the kept bytes count as free in
+gooseberry_device_memory; a reused block serves a new computation correctly."""
 import numpy as np
 import pytest
 
@@ -48,3 +48,31 @@ def test_reused_blocks_give_the_same_results(gb, oracle):
         assert np.max(np.abs(y - want)) <= 1e-14 * np.max(np.abs(want))
         del M
         junk.free()
+
+
+@pytest.mark.parametrize("n", [1, 32, 33, 160, 161, 4000, 524287, 524289])
+def test_small_blocks_reused_and_whole(gb, n):
+    # sizes around the steps of the rounding (256 bytes, quarters of a power of
+    # two, 4 MiB): every block holds its own contents to its last element
+    print("small blocks", n, flush=True)
+    first = [gb.DeviceArray.from_host(np.full(n, i + 0.5)) for i in range(6)]
+    ptrs = {x.ptr for x in first}
+    for x in first:
+        x.free()
+    again = [gb.DeviceArray.from_host(np.full(n, -i - 0.5)) for i in range(6)]
+    assert {x.ptr for x in again} == ptrs
+    for i, x in enumerate(again):
+        assert np.array_equal(x.numpy(), np.full(n, -i - 0.5))
+        x.free()
+
+
+def test_many_small_blocks_are_given_back(gb):
+    # more blocks than the cache keeps: the oldest go back to the pool
+    xs = [gb.DeviceArray.from_host(np.full(8, float(i))) for i in range(1500)]
+    assert all(np.array_equal(x.numpy(), np.full(8, float(i))) for i, x in enumerate(xs))
+    for x in xs:
+        x.free()
+    ys = [gb.DeviceArray.from_host(np.full(8, -float(i))) for i in range(1500)]
+    assert all(np.array_equal(y.numpy(), np.full(8, -float(i))) for i, y in enumerate(ys))
+    for y in ys:
+        y.free()
