@@ -8,8 +8,9 @@
 // their first product.  A row's products are numbered t = 0, 1, ... in that
 // scan order.  Rows take one of three paths:
 //
-// Short rows (at most 64 products from at most 64 entries of A): one
-// wavefront per row, lane t holding product t.  The lanes enter their
+// Short rows (at most 64 products from at most 64 entries of A): a
+// wavefront takes up to 16 of them one after another, lane t holding product
+// t of the row.  The lanes enter their
 // columns in a 128-slot LDS hash table, each slot keeping the mask of lanes
 // with its column: a lane with no lower lane in its mask is the head of its
 // column, and its sum is its own product followed by the other lanes' in
@@ -17,7 +18,7 @@
 // columns in first-appearance order (a ballot gives each head its rank).
 //
 // Medium rows (at most 4096 distinct columns, by the lesser of the row's
-// products and C's columns): one wavefront per row again, 64 products a step
+// products and C's columns): one wavefront per row, 64 products a step
 // in t order, the columns found so far in an LDS hash table with each
 // column's rank (the order of its first product) and running sum.
 //
@@ -33,7 +34,8 @@
 // the reference's zeroed row does, so a lone -0.0 becomes +0.0).  The sparse
 // result needs each row's entry count before the rows can be placed: the
 // short and medium rows write their entries in first-appearance order to a
-// staging area at the row's first product position, with their counts; the
+// staging area at the row's first product position (where all rows are short,
+// a wavefront's rows follow one another there), with their counts; the
 // scan of the counts gives the row pointers and a copy puts the staged rows
 // in place.  (When the staging area would pass its limit, 8 GiB unless
 // GOOSEBERRY_SPGEMM_STAGE_MAX says otherwise, these rows are counted in
