@@ -87,12 +87,11 @@ struct gb_bsys {
   double *part3;    // nchunks partials of ||b - A x||^2 (split matrices)
   gbd_bstate *st;
   const double *jscale;  // MIXED_JACOBI: D^-1/2, else null
-  // an x-tile plan (xt_ptr non-null): the layout, its FP64 values and the
-  // FP32 values of the inner solve (plain or Jacobi-scaled)
-  const uint32_t *xt_rb, *xt_ptr, *xt_idx;
-  const double *xt_val;
+  // an x-tile plan (xt.ptr non-null): the layout (the matrix's xt in FP64, its
+  // xt32 in mixed precision) and the FP32 values of the inner solve (plain
+  // or Jacobi-scaled)
+  gb_xt xt;
   const float *xt_val32;
-  uint32_t xt_W, xt_T, xt_lc;
   int32_t precision;
   int32_t pad;
 };
@@ -383,6 +382,7 @@ gb_b_spmv(const gb_bsys *__restrict__ sys, const uint2 *__restrict__ items,
 // the p.Ap partials of a CG step in the system's precision, or in a
 // refresh step the FP64 residual b - A x and its squared-norm partials;
 // one partial per row block
+// (WIDE: doubled tiles, which only FP64 systems have)
 template <bool WIDE>
 __global__ void __launch_bounds__(GB_XT_THREADS)
 gb_b_spmv_xt(const gb_bsys *__restrict__ sys, uint32_t slot,
@@ -391,15 +391,20 @@ gb_b_spmv_xt(const gb_bsys *__restrict__ sys, uint32_t slot,
   const gb_bsys &S = sys[slot];
   const gbd_bstate *st = states + slot;
   if (st->done) return;  // not written during this kernel: uniform
-  if (st->mode_next == GB_MODE_REFRESH)
-    gb_xt_spmv<double, GB_XT_RESID>(S.xt_ptr, S.xt_idx, S.xt_val, S.x, S.r, 1, S.b, S.part1,
-                                    S.xt_rb, S.n, S.xt_T, S.xt_lc, L);
-  else if (S.precision != GOOSEBERRY_PRECISION_FP64)
-    gb_xt_spmv<float, GB_XT_DOT>(S.xt_ptr, S.xt_idx, S.xt_val32, S.p32, S.ap32, 1, nullptr,
-                                 S.part1, S.xt_rb, S.n, S.xt_T, S.xt_lc, L);
-  else
-    gb_xt_spmv<double, GB_XT_DOT>(S.xt_ptr, S.xt_idx, S.xt_val, S.p, S.ap, 1, nullptr,
-                                  S.part1, S.xt_rb, S.n, S.xt_T, S.xt_lc, L);
+  if constexpr (!WIDE) {
+    if (st->mode_next == GB_MODE_REFRESH) {
+      gb_xt_spmv<double, GB_XT_RESID>(S.xt.ptr, S.xt.idx, S.xt.val, S.x, S.r, 1, S.b, S.part1,
+                                      S.xt.rb, S.n, S.xt.T, S.xt.lc, L);
+      return;
+    }
+    if (S.precision != GOOSEBERRY_PRECISION_FP64) {
+      gb_xt_spmv<float, GB_XT_DOT>(S.xt.ptr, S.xt.idx, S.xt_val32, S.p32, S.ap32, 1, nullptr,
+                                   S.part1, S.xt.rb, S.n, S.xt.T, S.xt.lc, L);
+      return;
+    }
+  }
+  gb_xt_spmv<double, GB_XT_DOT>(S.xt.ptr, S.xt.idx, S.xt.val, S.p, S.ap, 1, nullptr, S.part1,
+                                S.xt.rb, S.n, S.xt.T, S.xt.lc, L);
 }
 
 // A thread's GB_BCHUNK_ITEMS rows of a whole chunk of an internal vector
@@ -493,7 +498,7 @@ gb_b_update(const gb_bsys *__restrict__ sys, const uint2 *__restrict__ items,
     if (first) st->mode = mode;
   } else {
     // one partial per SpMV work item (per row block on an x-tile plan)
-    const uint32_t np = S.xt_ptr ? S.xt_W : nsplit ? S.nwork_split : S.pl.nwork;
+    const uint32_t np = S.xt.ptr ? S.xt.W : nsplit ? S.nwork_split : S.pl.nwork;
     const double t = gb_b_sum_chunks(S.part1, np, red);  // barriers inside
     if (s_done) return;
     int status = 0;
@@ -906,7 +911,8 @@ static uint32_t gb_b_nwork_split(const gbd_matrix *m) {
 static gb_b_layout gb_b_plan_layout(const gbd_matrix *m, int precision) {
   const size_t n = m->nrows ? m->nrows : 1;
   size_t nwork = m->nsplit ? gb_b_nwork_split(m) : gb_spmv_nwork(m);
-  if (m->xt_ptr && m->xt_W > nwork) nwork = m->xt_W;
+  // (both x-tile layouts have the same number of row blocks)
+  if (m->xt.ptr && m->xt.W > nwork) nwork = m->xt.W;
   const size_t nch = gb_b_nchunks(m->nrows);
   const size_t np1 = (nwork > nch ? nwork : nch) + 1;
   const size_t np2 = nch + 1;
@@ -1051,7 +1057,7 @@ int gbd_batch_add(gbd_batch *B, const gbd_matrix *m, const double *d_b,
   if (jac && (!m->val32j || !m->jscale || (m->nsplit && !m->sval32j)))
     return GOOSEBERRY_ERROR_INVALIDINPUT;
   // an x-tile plan: the layout's copy of the inner solve's FP32 values
-  if (m->xt_ptr && precision != GOOSEBERRY_PRECISION_FP64 &&
+  if (m->xt.ptr && precision != GOOSEBERRY_PRECISION_FP64 &&
       !(jac ? m->xt_val32j : m->xt_val32))
     return GOOSEBERRY_ERROR_INVALIDINPUT;
   uint32_t slot = 0;
@@ -1087,15 +1093,9 @@ int gbd_batch_add(gbd_batch *B, const gbd_matrix *m, const double *d_b,
   }
   S.st = B->d_st + slot;
   S.precision = precision;
-  if (m->xt_ptr) {
-    S.xt_ptr = m->xt_ptr;
-    S.xt_idx = m->xt_idx;
-    S.xt_val = m->xt_val;
+  if (m->xt.ptr) {
+    S.xt = precision == GOOSEBERRY_PRECISION_FP64 ? m->xt : m->xt32;
     S.xt_val32 = jac ? m->xt_val32j : m->xt_val32;
-    S.xt_rb = m->xt_rb;
-    S.xt_W = m->xt_W;
-    S.xt_T = m->xt_T;
-    S.xt_lc = m->xt_lc;
   }
   hipStream_t s = gb_stream();
   gb_bplan *hsl = nullptr;
@@ -1165,7 +1165,7 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
   uint64_t ns = 0, ne = 0;
   for (uint32_t i = 0; i < B->max_slots; ++i) {
     if (!B->used[i] || (active && !active[i])) continue;
-    if (!B->h_sys[i].xt_ptr)
+    if (!B->h_sys[i].xt.ptr)
       ns += B->h_sys[i].nsplit ? B->h_sys[i].nwork_split : B->h_sys[i].pl.nwork;
     ne += B->h_sys[i].nchunks;
   }
@@ -1202,7 +1202,7 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
   for (uint32_t i = 0; i < B->max_slots; ++i) {
     if (!B->used[i] || (active && !active[i])) continue;
     const gb_bsys &S = B->h_sys[i];
-    if (S.xt_ptr) continue;  // launched on its own
+    if (S.xt.ptr) continue;  // launched on its own
     if (!S.nsplit) {
       scattered += S.pl.dcol ? 0 : S.pl.nstream;
       blocks += S.pl.nwork;
@@ -1226,7 +1226,7 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
       if (!B->used[i] || (active && !active[i])) continue;
       const gb_bsys &S = B->h_sys[i];
       uint32_t nw = 0;
-      if (S.xt_ptr) nw = 0;
+      if (S.xt.ptr) nw = 0;
       else if (S.nsplit) nw = g < S.nsplit ? B->h_slice_nwork[(size_t)i * GB_SPLIT_MAX + g] : 0;
       else if (g == 0) nw = S.pl.nwork;
       for (uint32_t w = 0; w < nw; ++w) B->h_spmv[a++] = make_uint2(i, w);
@@ -1243,12 +1243,12 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
   uint32_t nx = 0;
   bool xchanged = false;
   for (uint32_t i = 0; i < B->max_slots; ++i) {
-    if (!B->used[i] || (active && !active[i]) || !B->h_sys[i].xt_ptr) continue;
+    if (!B->used[i] || (active && !active[i]) || !B->h_sys[i].xt.ptr) continue;
     xchanged = xchanged || nx >= B->n_xt || B->h_xt[nx] != i ||
-               B->h_xt_grid[nx] != B->h_sys[i].xt_W || B->h_xt_lc[nx] != B->h_sys[i].xt_lc;
+               B->h_xt_grid[nx] != B->h_sys[i].xt.W || B->h_xt_lc[nx] != B->h_sys[i].xt.lc;
     B->h_xt[nx] = i;
-    B->h_xt_grid[nx] = B->h_sys[i].xt_W;
-    B->h_xt_lc[nx] = B->h_sys[i].xt_lc;
+    B->h_xt_grid[nx] = B->h_sys[i].xt.W;
+    B->h_xt_lc[nx] = B->h_sys[i].xt.lc;
     ++nx;
   }
   if (xchanged || nx != B->n_xt) {

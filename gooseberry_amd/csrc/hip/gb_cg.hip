@@ -748,7 +748,7 @@ static gbd_cg_state g_scratch_hst;     // its polled state (pageable host memory
 static void gb_cg_geometry_one(gbd_cg *cg) {
   const gbd_matrix *m = cg->m;
   cg->grid_one = 0;
-  if (!cg->n || m->nwave || m->nblockrows || m->nsplit || m->nparts || m->xt_ptr || m->cshift)
+  if (!cg->n || m->nwave || m->nblockrows || m->nsplit || m->nparts || m->xt.ptr || m->cshift)
     return;
   uint32_t cus = gb_num_cus();
   if (cus > GB_CGP_GRID) cus = GB_CGP_GRID;

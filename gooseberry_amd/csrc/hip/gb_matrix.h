@@ -9,6 +9,18 @@
 #define GB_STREAM_LDS 2304
 #define GB_STREAM_ITERS (GB_STREAM_LDS / GB_BLOCK)
 
+// An x-tile layout (C = 2^lc columns a tile): the entries grouped by (block
+// of rows [rb[b], rb[b + 1]), tile), each group in CSR order; entry j of the
+// layout is idx[j] = (row in block << lc) | (column in tile) with value
+// val[j], group g = b T + t holding [ptr[g], ptr[g + 1])
+struct gb_xt {
+  uint32_t *rb;   // W + 1
+  uint32_t *ptr;  // W T + 1; null without x tiles
+  uint32_t *idx;  // nnz
+  double *val;    // nnz
+  uint32_t W, T, lc;
+};
+
 struct gbd_matrix {
   uint32_t nrows, ncols;
   uint64_t nnz;
@@ -43,18 +55,13 @@ struct gbd_matrix {
   uint32_t nvals;
   uint32_t pipe_grid;   // > 0: the SpMV runs the persistent pipelined
                         // row-block kernel on this many workgroups
-  // x tiles (params.xtile = C): the entries grouped by (block of rows
-  // [xt_rb[b], xt_rb[b + 1]), tile of C columns), each group in CSR order;
-  // entry j of the layout is xt_idx[j] = (row in block << xt_lc) | (column in
-  // tile) with value xt_val[j], group g = b xt_T + t holding
-  // [xt_ptr[g], xt_ptr[g + 1])
-  uint32_t *xt_rb;      // xt_W + 1
-  uint32_t *xt_ptr;     // xt_W xt_T + 1
-  uint32_t *xt_idx;     // nnz
-  double *xt_val;       // nnz
-  float *xt_val32;      // nnz, with val32: its values in the layout's order
-  float *xt_val32j;     // nnz, with val32j: its values in the layout's order
-  uint32_t xt_W, xt_T, xt_lc;
+  // x tiles (params.xtile = C): xt is what FP64 products read.  FP32 products
+  // and the FP64 residuals of mixed solves read xt32, made with the FP32
+  // values: tiles of C columns and blocks of equal rows always (its arrays
+  // are xt's own where that has them too).  See gb_xtile_build.
+  gb_xt xt, xt32;
+  float *xt_val32;      // nnz, with val32: its values in xt32's order
+  float *xt_val32j;     // nnz, with val32j: its values in xt32's order
   uint64_t hist[33];
   // column split (params.csplit = P > 1): P views, view r holding the
   // entries of columns [r W, (r + 1) W), W = ceil(ncols / P), in row order;
@@ -182,7 +189,7 @@ uint32_t gb_spmv_grid(const gbd_matrix *m);
 
 // p.Ap partials written by one SpMV launch with DOT (one per workgroup)
 static inline uint32_t gb_spmv_npartials(const gbd_matrix *m) {
-  return (m->nsplit || m->nparts || m->xt_ptr) ? gb_split_sum_grid(m) : gb_spmv_grid(m);
+  return (m->nsplit || m->nparts || m->xt.ptr) ? gb_split_sum_grid(m) : gb_spmv_grid(m);
 }
 
 // Enqueue y = A x; when cg != nullptr also write the per-workgroup partial

@@ -453,16 +453,16 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
   hipError_t he = hipSuccess;
   // An x-tile or column-split plan reads its own copy of the values, which
   // is normalised below; the CSR's order is then never read.
-  const bool own_copy = m->xt_ptr || m->nsplit;
+  const bool own_copy = m->xt.ptr || m->nsplit;
   // An x-tile plan sums the columns on its own layout, without the sort, where
   // it has the column tiles to fill the GPU with a workgroup each;
   // GOOSEBERRY_PAGERANK_SORTED_SUMS set to "0" takes the layout wherever its
   // tiles fit, set to anything else the sort (the same bits: a check of one
   // path against the other).
   const char *sorted_env = getenv("GOOSEBERRY_PAGERANK_SORTED_SUMS");
-  bool tile_sums = m->xt_ptr && nnz && (1u << m->xt_lc) <= GB_XT_CMAX;
+  bool tile_sums = m->xt.ptr && nnz && (1u << m->xt.lc) <= GB_XT_CMAX;
   if (sorted_env && *sorted_env) tile_sums = tile_sums && strcmp(sorted_env, "0") == 0;
-  else tile_sums = tile_sums && m->xt_T >= GB_PRX_TILES;
+  else tile_sums = tile_sums && m->xt.T >= GB_PRX_TILES;
 #define GB_PR_TRY(call)                                         \
   do {                                                          \
     he = (call);                                                \
@@ -496,8 +496,8 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
     // column sums and the layout's quotients, one workgroup per column tile
     GB_PR_TRY(gb_dev_alloc((void **)&snval, ((size_t)nnz + GB_XT_PAD) * 8));
     GB_PR_TRY(hipMemsetAsync(snval + nnz, 0, GB_XT_PAD * 8, s));
-    gb_pr_colsum_xt<<<m->xt_T, GB_PRX_THREADS, 0, s>>>(m->xt_ptr, m->xt_W, m->xt_T, m->xt_lc,
-                                                     m->xt_idx, m->xt_val, n, indeg, snval);
+    gb_pr_colsum_xt<<<m->xt.T, GB_PRX_THREADS, 0, s>>>(m->xt.ptr, m->xt.W, m->xt.T, m->xt.lc,
+                                                     m->xt.idx, m->xt.val, n, indeg, snval);
     GB_PR_TRY(hipGetLastError());
   } else {
     // column sums in row order (column indices were validated with the matrix)
@@ -533,7 +533,7 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
   mm.nvals = 0;
   mm.nsplit = 0;
   mm.split = nullptr;
-  if (m->xt_ptr && nnz) {
+  if (m->xt.ptr && nnz) {
     // an x-tile plan: the layout's copy of the values divided by the same
     // column sums (the same quotient per entry), with the layout's zero
     // entries past the end (its SpMV reads vectors); made above with the
@@ -541,12 +541,12 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
     if (!tile_sums) {
       GB_PR_TRY(gb_dev_alloc((void **)&snval, ((size_t)nnz + GB_XT_PAD) * 8));
       GB_PR_TRY(hipMemsetAsync(snval + nnz, 0, GB_XT_PAD * 8, s));
-      const uint32_t ng = m->xt_W * m->xt_T;
+      const uint32_t ng = m->xt.W * m->xt.T;
       gb_pr_normalise_xt<<<ng < 65536u ? ng : 65536u, GB_BLOCK, 0, s>>>(
-          m->xt_ptr, ng, m->xt_T, m->xt_lc, m->xt_idx, m->xt_val, indeg, snval);
+          m->xt.ptr, ng, m->xt.T, m->xt.lc, m->xt.idx, m->xt.val, indeg, snval);
       GB_PR_TRY(hipGetLastError());
     }
-    mm.xt_val = snval;
+    mm.xt.val = snval;
   }
   if (m->nsplit && nnz) {
     // a column-split plan: the slices' copy of the values divided by the

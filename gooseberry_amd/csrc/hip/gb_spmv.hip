@@ -904,19 +904,22 @@ static int gb_spmv_launch_t(const gbd_matrix *m, const T *val, const uint8_t *vi
                             double *partials, const gbd_cg_state *cg) {
   if (m->nsplit) return gb_spmv_launch_split<T>(m, x, y, ystride, partials, cg);
   if (m->nparts) return gb_spmv_launch_parts<T>(m, x, y, ystride, partials, cg);
-  if (m->xt_ptr) {
-    // x tiles: the FP64 values, or their FP32 copy in the layout's order
+  if (m->xt.ptr) {
+    // x tiles: the FP64 values, or their FP32 copy in the other layout's order
     // (made with the matrix's FP32 copy; CG runs in FP64 only)
+    const gb_xt &X = sizeof(T) == 8 ? m->xt : m->xt32;
     const T *xv;
-    if constexpr (sizeof(T) == 8) xv = m->xt_val;
-    else xv = cg ? nullptr : m->xt_val32;
+    auto *k = gb_spmv_xtile<T, GB_XT_STORE, false>;
+    if constexpr (sizeof(T) == 8) {
+      xv = X.val;
+      if (gb_xt_is_wide(X.lc)) k = gb_spmv_xtile<T, GB_XT_STORE, true>;
+    } else {
+      xv = cg ? nullptr : m->xt_val32;
+    }
     if (xv) {
       hipStream_t s = gb_stream();
-      auto *k = gb_xt_is_wide(m->xt_lc) ? gb_spmv_xtile<T, GB_XT_STORE, true>
-                                        : gb_spmv_xtile<T, GB_XT_STORE, false>;
-      k<<<m->xt_W, GB_XT_THREADS, 0, s>>>(
-          m->xt_ptr, m->xt_idx, xv, x, y, ystride, nullptr, m->xt_rb, m->ncols, m->xt_T,
-          m->xt_lc);
+      k<<<X.W, GB_XT_THREADS, 0, s>>>(X.ptr, X.idx, xv, x, y, ystride, nullptr, X.rb, m->ncols,
+                                      X.T, X.lc);
       GB_LAUNCH_CHECK();
       if constexpr (sizeof(T) == 8) {
         if (cg) {
@@ -1140,7 +1143,7 @@ static void gb_spmm_rows_go(const gbd_matrix *m, const double *b, double *bt, do
 // not on column splits, x tiles or row parts (kernels of their own), nor on
 // exact plans (whose longer rows are folded in another order).
 static bool gb_spmm_several(const gbd_matrix *m, uint32_t bncols) {
-  return bncols > 1 && !m->nsplit && !m->nparts && !m->xt_ptr && !m->params.exact &&
+  return bncols > 1 && !m->nsplit && !m->nparts && !m->xt.ptr && !m->params.exact &&
          gb_spmv_nwork(m) > 0 && m->ncols > 0;
 }
 
@@ -1427,17 +1430,21 @@ static void gb_vdict_free(gbd_matrix *m) {
 
 // ------------------------------------------------------------- host side
 
+static void gb_xt_drop(gb_xt *X) {
+  (void)gb_dev_free(X->rb);
+  (void)gb_dev_free(X->ptr);
+  (void)gb_dev_free(X->idx);
+  (void)gb_dev_free(X->val);
+  memset(X, 0, sizeof(*X));
+}
+
 static void gb_xtile_free(gbd_matrix *m) {
-  (void)gb_dev_free(m->xt_rb);
-  (void)gb_dev_free(m->xt_ptr);
-  (void)gb_dev_free(m->xt_idx);
-  (void)gb_dev_free(m->xt_val);
   (void)gb_dev_free(m->xt_val32);
   (void)gb_dev_free(m->xt_val32j);
-  m->xt_rb = m->xt_ptr = m->xt_idx = nullptr;
-  m->xt_val = nullptr;
   m->xt_val32 = m->xt_val32j = nullptr;
-  m->xt_W = m->xt_T = m->xt_lc = 0;
+  if (m->xt32.ptr != m->xt.ptr) gb_xt_drop(&m->xt32);
+  memset(&m->xt32, 0, sizeof(m->xt32));
+  gb_xt_drop(&m->xt);
 }
 
 // The Jacobi-scaled FP32 values in the layout's order: the same
@@ -1458,110 +1465,161 @@ gb_xt_jacobi_vals(const uint32_t *__restrict__ ptr, uint32_t ngroups, uint32_t T
   }
 }
 
-// The layout's FP32 copies of the values the matrix has in FP32 (val32,
-// val32j), made with them or with the layout, whichever comes second
+static int gb_xtile_layout(const gbd_matrix *m, bool equal_rows, gb_xt *X);
+static bool gb_xt_equal_rows(const gbd_matrix *m);
+
+// The FP32 copies of the values the matrix has in FP32 (val32, val32j), in
+// the order of xt32, which the first of them makes; they come with the FP32
+// values or with the x tiles, whichever is second
 static int gb_xtile_f32(gbd_matrix *m) {
-  if (!m->xt_ptr) return GOOSEBERRY_SUCCESS;
+  if (!m->xt.ptr) return GOOSEBERRY_SUCCESS;
   hipStream_t s = gb_stream();
   const size_t nz = m->nnz;
+  if ((m->val32 || m->val32j) && !m->xt32.ptr) {
+    if (gb_xt_equal_rows(m)) {
+      m->xt32 = m->xt;
+    } else {
+      const int rv = gb_xtile_layout(m, true, &m->xt32);
+      if (rv != GOOSEBERRY_SUCCESS) return rv;
+    }
+  }
   if (m->val32 && !m->xt_val32) {
     GB_HIP(gb_dev_alloc((void **)&m->xt_val32, (nz + GB_XT_PAD) * sizeof(float)));
     GB_HIP(hipMemsetAsync(m->xt_val32 + nz, 0, GB_XT_PAD * sizeof(float), s));
     if (nz) {
-      gb_to_f32<<<gb_div_up(nz, GB_BLOCK), GB_BLOCK, 0, s>>>(m->xt_val, m->xt_val32, nz);
+      gb_to_f32<<<gb_div_up(nz, GB_BLOCK), GB_BLOCK, 0, s>>>(m->xt32.val, m->xt_val32, nz);
       GB_LAUNCH_CHECK();
     }
   }
   if (m->val32j && m->jscale && !m->xt_val32j) {
     GB_HIP(gb_dev_alloc((void **)&m->xt_val32j, (nz + GB_XT_PAD) * sizeof(float)));
     GB_HIP(hipMemsetAsync(m->xt_val32j + nz, 0, GB_XT_PAD * sizeof(float), s));
-    const uint32_t ng = m->xt_W * m->xt_T;
+    const gb_xt &X = m->xt32;
+    const uint32_t ng = X.W * X.T;
     if (nz && ng) {
       gb_xt_jacobi_vals<<<ng < 65536u ? ng : 65536u, GB_BLOCK, 0, s>>>(
-          m->xt_ptr, ng, m->xt_T, m->xt_rb, m->xt_lc, m->xt_idx, m->xt_val, m->jscale,
-          m->xt_val32j);
+          X.ptr, ng, X.T, X.rb, X.lc, X.idx, X.val, m->jscale, m->xt_val32j);
       GB_LAUNCH_CHECK();
     }
   }
   return GOOSEBERRY_SUCCESS;
 }
 
-// The x-tile layout: keys = (row block, column tile) per entry, a stable
-// sort of the entries by key (each group keeps CSR order), then the packed
-// words and values gathered in that order.  Row blocks of
-// ceil(nrows / CUs) rows (at most GB_XT_RMAX): one workgroup per CU.
-static int gb_xtile_build(gbd_matrix *m) {
-  hipStream_t s = gb_stream();
+// Row blocks of an x-tile plan, one workgroup per CU (more where the rows do
+// not fit LDS): ceil(nrows / CUs) rows each, or about as many entries each.
+//
+// FP64 products (SpMV, CG, batches, PageRank) take blocks of equal entries,
+// and doubled tiles where the rows leave LDS for them.  What FP32 reads keeps
+// blocks of equal rows and the tiles as asked for: a row's sum is grouped by
+// tile and by where its entries fall in the block's ranges, and in FP32 another
+// grouping takes a mixed solve another way to another place within its
+// tolerance.  With FP64's layout, x of Zipf systems of 400,000 rows moved by up
+// to 1.1e-9 of its norm at a relative residual of 1e-10 (FP64's own sums move
+// in the 16th digit), and 37 ms a solve became 26.  Matrices of more entries
+// than GB_XT_TWO_MAX (two layouts and both sorts' scratch would pass half of
+// the device) have the one of equal rows for both.
+#define GB_XT_TWO_MAX (1ull << 30)
+
+struct gb_xt_geometry {
+  uint32_t R, W, T, lc;
+  uint64_t k;  // weight of a row beside its entries (gb_xt_bounds); 0: equal rows
+};
+
+static gb_xt_geometry gb_xt_plan(const gbd_matrix *m, bool equal_rows) {
   const uint32_t n = m->nrows;
-  uint32_t C = m->params.xtile, lc = 0;
-  while ((1u << lc) < C) ++lc;
-  uint32_t R = gb_div_up(n, gb_num_cus());
-  // the widest tiles are doubled where the rows leave LDS for them, with room
-  // for blocks of equal entries, and both types take fewer steps then (FP32
-  // has two tiles a step already: 9,000 columns 8.2 us plain, 9.1 doubled)
-  const bool wide = C == GB_XT_CMAX && m->ncols > 2 * C && R <= GB_XT_RWIDE / 5 * 4;
+  uint32_t C = m->params.xtile;
+  gb_xt_geometry G;
+  G.lc = 0;
+  while ((1u << G.lc) < C) ++G.lc;
+  G.R = gb_div_up(n, gb_num_cus());
+  if (m->nnz > GB_XT_TWO_MAX) equal_rows = true;
+  // the widest tiles are doubled where there are more than two of them and the
+  // rows leave LDS, with room for blocks of equal entries
+  const bool wide =
+      !equal_rows && C == GB_XT_CMAX && m->ncols > 2 * C && G.R <= GB_XT_RWIDE / 5 * 4;
   const uint32_t rmax = wide ? GB_XT_RWIDE : GB_XT_RMAX;
   if (wide) {
     C = GB_XT_WIDE;
-    ++lc;
+    ++G.lc;
   }
-  if (R > rmax) R = rmax;
-  if (R == 0) R = 1;
-  const uint32_t W = gb_div_up(n, R);
+  if (G.R > rmax) G.R = rmax;
+  if (G.R == 0) G.R = 1;
+  G.W = gb_div_up(n, G.R);
+  G.T = gb_div_up(m->ncols ? m->ncols : 1, C);
   // the least weight per row that keeps the blocks within rmax rows
-  const uint64_t room = (uint64_t)W * (rmax - 2);
-  uint64_t k = 0;
-  if (room > n) {
-    k = m->nnz / (room - n) + 1;
-    if (k < 4) k = 4;
+  const uint64_t room = (uint64_t)G.W * (rmax - 2);
+  G.k = 0;
+  if (!equal_rows && room > n) {
+    G.k = m->nnz / (room - n) + 1;
+    if (G.k < 4) G.k = 4;
   }
-  const uint32_t T = gb_div_up(m->ncols ? m->ncols : 1, C);
-  const uint64_t groups = (uint64_t)W * T;
+  return G;
+}
+
+// whether the FP64 products' layout is the one of equal rows
+static bool gb_xt_equal_rows(const gbd_matrix *m) {
+  return gb_xt_plan(m, false).k == 0 && !gb_xt_is_wide(m->xt.lc);
+}
+
+// One layout: keys = (row block, column tile) per entry, a stable sort of the
+// entries by key (each group keeps CSR order), then the packed words and
+// values gathered in that order.
+static int gb_xtile_layout(const gbd_matrix *m, bool equal_rows, gb_xt *X) {
+  hipStream_t s = gb_stream();
+  const uint32_t n = m->nrows;
+  const gb_xt_geometry G = gb_xt_plan(m, equal_rows);
+  const uint64_t groups = (uint64_t)G.W * G.T;
   if (groups >= 0xffffffffull || m->nnz + GB_XT_THREADS >= 0xffffffffull) {
-    gb_set_error("x tiles of %u columns: too many groups (%llu) or entries", C,
+    gb_set_error("x tiles of %u columns: too many groups (%llu) or entries", 1u << G.lc,
                  (unsigned long long)groups);
     return GOOSEBERRY_ERROR_INVALIDINPUT;
   }
+  memset(X, 0, sizeof(*X));
   uint32_t *keys = nullptr, *word = nullptr, *perm = nullptr;
   const size_t nz = m->nnz;
   hipError_t e = gb_dev_alloc((void **)&keys, nz * 4);
   if (e == hipSuccess) e = gb_dev_alloc((void **)&word, nz * 4);
   if (e == hipSuccess) e = gb_dev_alloc((void **)&perm, nz * 4);
-  if (e == hipSuccess) e = gb_dev_alloc((void **)&m->xt_rb, ((size_t)W + 1) * 4);
-  if (e == hipSuccess) e = gb_dev_alloc((void **)&m->xt_ptr, (groups + 1) * 4);
+  if (e == hipSuccess) e = gb_dev_alloc((void **)&X->rb, ((size_t)G.W + 1) * 4);
+  if (e == hipSuccess) e = gb_dev_alloc((void **)&X->ptr, (groups + 1) * 4);
   // zero entries past the end: the SpMV reads the layout E entries a lane
-  if (e == hipSuccess) e = gb_dev_alloc((void **)&m->xt_idx, (nz + GB_XT_PAD) * 4);
-  if (e == hipSuccess) e = gb_dev_alloc((void **)&m->xt_val, (nz + GB_XT_PAD) * 8);
-  if (e == hipSuccess) e = hipMemsetAsync(m->xt_idx + nz, 0, GB_XT_PAD * 4, s);
-  if (e == hipSuccess) e = hipMemsetAsync(m->xt_val + nz, 0, GB_XT_PAD * 8, s);
+  if (e == hipSuccess) e = gb_dev_alloc((void **)&X->idx, (nz + GB_XT_PAD) * 4);
+  if (e == hipSuccess) e = gb_dev_alloc((void **)&X->val, (nz + GB_XT_PAD) * 8);
+  if (e == hipSuccess) e = hipMemsetAsync(X->idx + nz, 0, GB_XT_PAD * 4, s);
+  if (e == hipSuccess) e = hipMemsetAsync(X->val + nz, 0, GB_XT_PAD * 8, s);
   int rv = e == hipSuccess ? GOOSEBERRY_SUCCESS : GOOSEBERRY_ERROR_NOMEMORY;
   if (rv == GOOSEBERRY_SUCCESS) {
-    gb_xt_bounds<<<gb_div_up(W + 1, GB_BLOCK), GB_BLOCK, 0, s>>>(m->rowptr, n, W, k, R,
-                                                                 m->xt_rb);
+    gb_xt_bounds<<<gb_div_up(G.W + 1, GB_BLOCK), GB_BLOCK, 0, s>>>(m->rowptr, n, G.W, G.k, G.R,
+                                                                   X->rb);
     gb_xt_keys<<<gb_div_up(n, GB_BLOCK / 16), GB_BLOCK, 0, s>>>(
-        m->rowptr, m->rowind, n, m->xt_rb, W, T, lc, keys, word);
+        m->rowptr, m->rowind, n, X->rb, G.W, G.T, G.lc, keys, word);
     if (gb_launch_status() != hipSuccess) rv = GOOSEBERRY_ERROR_DEVICE;
   }
   if (rv == GOOSEBERRY_SUCCESS)
     rv = gbd_countingsort_kv_unchecked(keys, nullptr, 0, (uint32_t)(groups - 1), nz, perm,
-                                       m->xt_ptr);
+                                       X->ptr);
   if (rv == GOOSEBERRY_SUCCESS) {
     const uint64_t g = gb_div_up(nz, GB_BLOCK);
     gb_xt_gather<<<g > 65536 ? 65536u : (uint32_t)g, GB_BLOCK, 0, s>>>(perm, nz, word, m->val,
-                                                                      m->xt_idx, m->xt_val);
+                                                                      X->idx, X->val);
     if (gb_launch_status() != hipSuccess) rv = GOOSEBERRY_ERROR_DEVICE;
   }
   (void)gb_dev_free(keys);
   (void)gb_dev_free(word);
   (void)gb_dev_free(perm);
   if (rv != GOOSEBERRY_SUCCESS) {
-    gb_xtile_free(m);
+    gb_xt_drop(X);
     return rv;
   }
-  m->xt_W = W;
-  m->xt_T = T;
-  m->xt_lc = lc;
-  rv = gb_xtile_f32(m);
+  X->W = G.W;
+  X->T = G.T;
+  X->lc = G.lc;
+  return GOOSEBERRY_SUCCESS;
+}
+
+static int gb_xtile_build(gbd_matrix *m) {
+  int rv = gb_xtile_layout(m, false, &m->xt);
+  if (rv == GOOSEBERRY_SUCCESS) rv = gb_xtile_f32(m);
   if (rv != GOOSEBERRY_SUCCESS) gb_xtile_free(m);
   return rv;
 }
@@ -2150,7 +2208,7 @@ static int gb_parts_refuse(const gbd_matrix *m, const char *what) {
 }
 
 int gbd_matrix_make_f32(gbd_matrix *m) {
-  if (m->val32) return GOOSEBERRY_SUCCESS;
+  if (m->val32) return gb_xtile_f32(m);  // there, unless memory ran out
   GB_HIP(gb_dev_alloc((void **)&m->val32, (m->nnz ? m->nnz : 1) * sizeof(float)));
   if (m->nnz) {
     gb_to_f32<<<gb_div_up(m->nnz, GB_BLOCK), GB_BLOCK, 0, gb_stream()>>>(
@@ -2183,7 +2241,7 @@ int gbd_matrix_make_f32(gbd_matrix *m) {
 }
 
 int gbd_matrix_make_f32_jacobi(gbd_matrix *m) {
-  if (m->val32j) return GOOSEBERRY_SUCCESS;
+  if (m->val32j) return gb_xtile_f32(m);  // there, unless memory ran out
   int rp = gb_parts_refuse(m, "Jacobi scaling");
   if (rp != GOOSEBERRY_SUCCESS) return rp;
   hipStream_t s = gb_stream();

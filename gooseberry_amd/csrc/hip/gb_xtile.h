@@ -5,8 +5,10 @@
 // columns), each group in CSR order: ptr[g] .. ptr[g + 1] for group
 // g = block * T + tile, each entry a packed word (row within the block << lc
 // | column within the tile) and a value.  Row block b is rows rb[b] ..
-// rb[b + 1], at most GB_XT_RMAX (GB_XT_RWIDE with doubled tiles), and the
-// blocks hold about equally many entries where that limit allows.  One workgroup owns a row block and
+// rb[b + 1], at most GB_XT_RMAX (GB_XT_RWIDE with doubled tiles).  A matrix
+// has one layout for FP64 products (blocks of about equally many entries) and
+// one for FP32 products and mixed solves (blocks of equal rows); the rules are
+// beside gb_xtile_layout.  One workgroup owns a row block and
 // keeps its y in LDS; tile by tile it copies x's tile into LDS and adds its
 // group's products, so the gathers read LDS and only the matrix and x
 // stream.  Each row gets one sum per tile, added to its y in tile order: a
@@ -26,9 +28,8 @@
 // (GB_XT_WIDE columns of FP64 x, 128 KB) beside a block of GB_XT_RWIDE rows.
 // A step costs 3.3 us before its first entry (staging x, two barriers, the
 // carries) and a 300,000-row Zipf graph takes 4.4 us for one, so half as many
-// steps: FP64 / FP32 us, plain and doubled, at 30,000 rows 20.9 / 13.1 and
-// 16.5 / 11.3, at 300,000 165.0 / 101.6 and 140.4 / 85.8, at 800,000
-// 435 / 262 and 370 / 229.
+// steps: FP64 us, plain and doubled, at 30,000 rows 20.9 and 16.5, at 300,000
+// 165.0 and 140.4, at 800,000 435 and 370.  (FP32 keeps plain tiles.)
 #define GB_XT_WIDE (2 * GB_XT_CMAX)
 #define GB_XT_RWIDE 3968
 #define GB_XT_DEPTH 1    // chunks a wavefront has in flight (on the Zipf matrix:

@@ -307,3 +307,50 @@ def test_xtile_batched_widths_in_turn(gb, oracle, precision):
         assert np.array_equal(dx.numpy(), x)
         B.remove(s)
     B.free()
+
+
+def test_xtile_f32_sums_keep_their_order(gb):
+    # FP32 products on x tiles group a row's sum by tiles of 8192 columns, the
+    # even and the odd tiles apart, and by the sixteen ranges of a block of
+    # ceil(n / 256) rows, whatever the FP64 products' layout is.  Row 2: one
+    # value in each of the first three tiles, (2^24 - 2^24) + 1 = 1, where tiles
+    # of 16384 give (2^24 + 1) - 2^24 = 0.  Row 0, of as many entries as row 1
+    # of its block: its first range holds 512 entries, so that the ones at
+    # entries 256 and 257 are added to 2^24 one by one and lost; a block of its
+    # own would have 256 in a range and the ones' sum 2 kept.
+    n, m, big = 512, 49155, 2.0 ** 24
+    ri = np.concatenate([np.arange(4096), np.arange(4096), [0, 8192, 16384], np.full(n - 3, 7)])
+    rv = np.zeros(ri.size)
+    rv[[0, 256, 257]] = big, 1, 1
+    rv[8192:8195] = big, 1, -big
+    rp = np.concatenate([[0, 4096, 8192], np.arange(8195, 8195 + n - 2)]).astype(np.uint32)
+    M = gb.Matrix(rp, ri.astype(np.uint32), rv, ncols=m, plan={"xtile": 8192})
+    y64 = M.spmv(np.ones(m))
+    y32 = M.spmv_f32(np.ones(m))
+    assert list(y32[:4]) == [big, 0, 1, 0]
+    assert list(y64[:4]) == [big + 2, 0, 1, 0]
+    # one layout does not touch the other
+    assert np.array_equal(M.spmv(np.ones(m)), y64) and np.array_equal(M.spmv_f32(np.ones(m)), y32)
+
+
+@pytest.mark.parametrize("jacobi", [False, True])
+def test_xtile_mixed_solves_beside_fp64(gb, jacobi):
+    # a mixed solve's bits do not depend on what else its matrix was used for
+    # or on whether the plan or the FP32 values came first
+    M0 = gb.generate_spd(60000, 5, gb.DEGREE_ZIPF, 1.5, 2, 400)
+    rp, ri, rv = M0.download()
+    b = gb.uniform(6, rp.size - 1)
+    precision = gb.PRECISION_MIXED_JACOBI if jacobi else gb.PRECISION_MIXED
+    A = gb.Matrix(rp, ri, rv, plan={"xtile": 8192})
+    (x, info), = _batch(gb, [(A, b)], precision)
+    assert info.status == 1
+    B = gb.Matrix(rp, ri, rv)
+    _batch(gb, [(B, b)], precision)
+    B.spmv(b)
+    B.replan({"xtile": 8192})
+    y = B.spmv(b)
+    (xf, _), = _batch(gb, [(B, b)], gb.PRECISION_FP64)
+    (x2, info2), (xf2, _) = _batch(gb, [(B, b)], precision)[0], _batch(gb, [(B, b)], 0)[0]
+    assert np.array_equal(x, x2) and info2.niter == info.niter
+    assert np.array_equal(xf, xf2) and np.array_equal(B.spmv(b), y)
+    assert np.array_equal(A.spmv(b), y)
