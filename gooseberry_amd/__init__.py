@@ -46,6 +46,7 @@ TOL_RELATIVE = 1
 
 FAULT_ALLOC = 0
 FAULT_LAUNCH = 1
+FAULT_CG_WAIT = 2
 
 REQUEST_CANCELLED = 4
 REQUEST_TIMEDOUT = 5
@@ -296,7 +297,9 @@ def lib():
 
 def inject_fault(kind, after):
     """Test hook: the (after+1)-th device allocation (FAULT_ALLOC) or kernel
-    launch check (FAULT_LAUNCH) from now on fails once; after < 0 disarms."""
+    launch check (FAULT_LAUNCH) from now on fails once, or in exchange `after`
+    of the next one-launch CG run a workgroup's wait runs out (FAULT_CG_WAIT);
+    after < 0 disarms."""
     check(lib().gooseberry_inject_fault(kind, int(after)), "gooseberry_inject_fault")
 
 

@@ -193,7 +193,8 @@ typedef struct gbd_cg_state {
   uint64_t maxiter;/* 0 = unbounded */
   int32_t done;    /* 1: stop (converged, breakdown or maxiter) */
   int32_t status;  /* 0 running, 1 converged, 2 maxiter, 3 breakdown */
-  uint32_t ticket[4];
+  int32_t waited;  /* a one-launch run gave up a wait: nothing else here counts */
+  uint32_t pad[3];
 } gbd_cg_state;
 
 typedef struct gbd_cg gbd_cg;
@@ -212,9 +213,9 @@ int gbd_cg_enqueue(gbd_cg *cg, uint32_t k);
  * ring) to the host. */
 /* whether the workspace's solves run whole batches of iterations in one
  * launch (any number: the launch stops where the solve does).  Such a run whose
- * workgroups did not get to run side by side ends with the status
- * GBD_CG_WAITED; gbd_cg_several_launches turns to one launch per step. */
-#define GBD_CG_WAITED 4
+ * workgroups did not get to run side by side leaves `waited` set in the state,
+ * whatever else it says, and the solve has to start again;
+ * gbd_cg_several_launches turns to one launch per step. */
 int gbd_cg_one_launch(const gbd_cg *cg);
 void gbd_cg_several_launches(gbd_cg *cg);
 int gbd_cg_poll(gbd_cg *cg, gbd_cg_state *st, double *h_trace);

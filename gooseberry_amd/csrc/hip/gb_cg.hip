@@ -128,6 +128,7 @@ gb_cg_init_state(const double *__restrict__ partials, uint32_t np,
     st->maxiter = maxiter;
     st->status = 0;
     st->done = 0;
+    st->waited = 0;
     if (s == 0.0) {  // b == 0: x = 0 is the solution
       st->done = 1;
       st->status = 1;
@@ -386,9 +387,14 @@ gb_cg_update_xp(double *__restrict__ x, const double *__restrict__ r,
 // gb_cg_update_xp; the dot products are grouped by thread and workgroup in
 // this kernel's own fixed way.
 //
-// The grid is at most the CUs, so the workgroups run side by side; a wait
-// that does not end within `spins` reads sets the status GBD_CG_WAITED
-// and ends the launch (the host then starts again on the other kernels).
+// The grid is at most the CUs, so the workgroups run side by side.  A workgroup
+// whose wait does not end within `spins` reads sets the state's `waited` and
+// leaves, without its rows of x; the others then run out of time in a later
+// exchange, or, if this was the last, end the solve.  So `waited` is a word
+// that only the set-up clears and no other end of a run touches, and the host
+// looks at it before all else: the solve starts again on the other kernels.
+// Workgroups may still be starting when it is set, and one thread decides for
+// each of them whether it runs.
 //
 // Bound: the latency of two exchanges (1.4 us for 16 workgroups to 2.5 us for
 // 256, in a kernel of exchanges alone) and of the gathers.  Per iteration,
@@ -423,13 +429,15 @@ struct gb_cgp_lds {
   uint32_t col[GB_CGP_ENTRIES];
   double part[GB_CGP_GRID];
   double red[GB_CGP_THREADS / GB_WAVE];
-  uint32_t bad;
+  uint32_t stop;  // no run, or a wait given up
 };
 
 // the sum of every workgroup's d, in a fixed order, on every thread; round
-// counts the exchanges of the launch.  False when a wait ran out.
+// counts the exchanges of the launch.  False when a wait ran out.  (In exchange
+// `lost` the last workgroup's does, whatever it reads: GB_FAULT_CG_WAIT.)
 __device__ __forceinline__ bool gb_cgp_sum(double d, uint64_t *slots, uint32_t round,
-                                           uint32_t spins, gb_cgp_lds &L, double *sum) {
+                                           uint32_t spins, uint32_t lost, gb_cgp_lds &L,
+                                           double *sum) {
   const uint32_t tid = threadIdx.x, W = gridDim.x;
   d = gb_wave_sum(d);
   if ((tid & (GB_WAVE - 1)) == 0) L.red[tid / GB_WAVE] = d;
@@ -462,14 +470,15 @@ __device__ __forceinline__ bool gb_cgp_sum(double d, uint64_t *slots, uint32_t r
     while ((v = __hip_atomic_load(&mine[tid * GB_CGP_PAD], __ATOMIC_RELAXED,
                                   __HIP_MEMORY_SCOPE_AGENT)) == GB_CGP_EMPTY) {
       if (++n > spins) {
-        L.bad = 1;
+        L.stop = 1;
         break;
       }
     }
+    if (round == lost && blockIdx.x == W - 1) L.stop = 1;
     L.part[tid] = __longlong_as_double((long long)v);
   }
   __syncthreads();
-  if (L.bad) return false;
+  if (L.stop) return false;
   if (tid == 0)  // the round before: everyone has read it
     __hip_atomic_store(&slots[((size_t)((round + 2) % 3) * GB_CGP_GRID + blockIdx.x) *
                               GB_CGP_PAD],
@@ -493,16 +502,19 @@ __global__ void __launch_bounds__(GB_CGP_THREADS)
 gb_cg_persist(const uint32_t *__restrict__ rowptr, const uint32_t *__restrict__ rowind,
               const double *__restrict__ val, uint32_t n, uint32_t rows, double *x, double *r,
               double *p0, double *p1, uint64_t *slots, gbd_cg_state *st, double *trace,
-              uint32_t trace_cap, uint32_t k, uint32_t spins) {
+              uint32_t trace_cap, uint32_t k, uint32_t spins, uint32_t lost) {
   constexpr uint32_t T = GB_CGP_THREADS;
   constexpr uint32_t U = 8;  // entries of a row whose gathers are in flight
   __shared__ gb_cgp_lds L;
   const uint32_t tid = threadIdx.x;
-  if (st->done || st->status) return;  // every workgroup alike: nothing is written yet
+  if (tid == 0)
+    L.stop = *(volatile int32_t *)&st->done | *(volatile int32_t *)&st->status |
+             __hip_atomic_load(&st->waited, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (L.stop) return;  // the whole workgroup: set again only past the next barrier
   const uint32_t row0 = blockIdx.x * rows;
   const uint32_t end = n - row0 < rows ? n : row0 + rows;
   const uint32_t k0 = rowptr[row0], k1 = rowptr[end];
-  if (tid == 0) L.bad = 0;
   for (uint32_t e = tid; e < k1 - k0; e += T) {
     L.col[e] = rowind[k0 + e];
     L.val[e] = val[k0 + e];
@@ -577,7 +589,7 @@ gb_cg_persist(const uint32_t *__restrict__ rowptr, const uint32_t *__restrict__ 
       ao[q] = s;
       d += po[q] * s;
     }
-    if (!gb_cgp_sum(d, slots, round++, spins, L, &pap)) break;
+    if (!gb_cgp_sum(d, slots, round++, spins, lost, L, &pap)) break;
     alpha = dr / pap;
     if (!(pap != 0.0) || !isfinite(alpha)) {
       status = 3;
@@ -602,7 +614,7 @@ gb_cg_persist(const uint32_t *__restrict__ rowptr, const uint32_t *__restrict__ 
       }
     }
     double dnr;
-    if (!gb_cgp_sum(d, slots, round++, spins, L, &dnr)) break;
+    if (!gb_cgp_sum(d, slots, round++, spins, lost, L, &dnr)) break;
     beta = dnr / dr;
     dr_prev = dr;
     dr = dnr;
@@ -614,8 +626,9 @@ gb_cg_persist(const uint32_t *__restrict__ rowptr, const uint32_t *__restrict__ 
     boa = beta / alpha;
     if (trace_cap && blockIdx.x == 0 && tid == 0) trace[(iter - 1) % trace_cap] = rnorm;
   }
-  if (L.bad) {  // set before a barrier that every thread has passed
-    if (tid == 0) st->status = GBD_CG_WAITED;
+  if (L.stop) {  // set before a barrier that every thread has passed
+    if (tid == 0)
+      __hip_atomic_store(&st->waited, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return;
   }
 #pragma unroll
@@ -684,11 +697,11 @@ static void gb_cg_launch_xp(gbd_cg *cg) {
 }
 
 template <int R>
-static void gb_cg_go_persist(gbd_cg *cg, uint32_t k) {
+static void gb_cg_go_persist(gbd_cg *cg, uint32_t k, uint32_t lost) {
   const gbd_matrix *m = cg->m;
   gb_cg_persist<R><<<cg->grid_one, GB_CGP_THREADS, 0, gb_stream()>>>(
       m->rowptr, m->rowind, m->val, cg->n, cg->rows_one, cg->x, cg->r, cg->p, cg->p2,
-      cg->slots, cg->st, cg->trace, cg->trace_cap, k, cg->spins);
+      cg->slots, cg->st, cg->trace, cg->trace_cap, k, cg->spins, lost);
 }
 
 static int gb_cg_enqueue_raw(gbd_cg *cg, uint32_t k) {
@@ -696,9 +709,10 @@ static int gb_cg_enqueue_raw(gbd_cg *cg, uint32_t k) {
     gb_cgp_empty<<<1, GB_BLOCK, 0, gb_stream()>>>(cg->slots);
     GB_LAUNCH_CHECK();
     const uint32_t per = gb_div_up(cg->rows_one, GB_CGP_THREADS);
-    if (per <= 1) gb_cg_go_persist<1>(cg, k);
-    else if (per <= 2) gb_cg_go_persist<2>(cg, k);
-    else gb_cg_go_persist<GB_CGP_ROWS>(cg, k);
+    const uint32_t lost = cg->grid_one > 1 ? gb_fault_cg_wait() : 0xffffffffu;
+    if (per <= 1) gb_cg_go_persist<1>(cg, k, lost);
+    else if (per <= 2) gb_cg_go_persist<2>(cg, k, lost);
+    else gb_cg_go_persist<GB_CGP_ROWS>(cg, k, lost);
     GB_LAUNCH_CHECK();
     return GOOSEBERRY_SUCCESS;
   }

@@ -25,7 +25,8 @@ void gb_set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 hipError_t gb_launch_status();
 #define GB_FAULT_ALLOC 0
 #define GB_FAULT_LAUNCH 1
-#define GB_FAULT_KINDS 2
+#define GB_FAULT_CG_WAIT 2
+#define GB_FAULT_KINDS 3
 #define GB_LAUNCH_CHECK() GB_HIP(gb_launch_status())
 
 hipStream_t gb_stream();
@@ -39,6 +40,8 @@ hipError_t gb_dev_alloc(void **p, size_t bytes);
 hipError_t gb_dev_free(void *p);
 // a small result to the host, waiting for the stream
 hipError_t gb_fetch(void *h_dst, const void *d_src, size_t bytes);
+// the exchange armed by GB_FAULT_CG_WAIT (once; 0xffffffff: none)
+uint32_t gb_fault_cg_wait();
 bool gb_graphs_enabled();  // false when GOOSEBERRY_NO_GRAPHS is set
 uint32_t gb_num_cus();     // compute units of the device
 

@@ -196,14 +196,20 @@ size_t gb_cache_cached_bytes() {
 // Injected faults (gbd_inject_fault, a test hook): with a countdown c >= 0
 // armed for a kind, the c+1-th device allocation (or launch check) from then
 // on reports a failure instead, once; c < 0 disarms.  An injected launch
-// failure is reported after the kernel was launched normally.
-static std::atomic<long long> g_fault[GB_FAULT_KINDS] = {{-1}, {-1}};
+// failure is reported after the kernel was launched normally.  (For
+// GB_FAULT_CG_WAIT c is the number of an exchange of the next one-launch CG run.)
+static std::atomic<long long> g_fault[GB_FAULT_KINDS] = {{-1}, {-1}, {-1}};
 
 static bool gb_fault_fires(int kind) {
   long long v = g_fault[kind].load();
   while (v >= 0)
     if (g_fault[kind].compare_exchange_weak(v, v - 1)) return v == 0;
   return false;
+}
+
+uint32_t gb_fault_cg_wait() {
+  const long long v = g_fault[GB_FAULT_CG_WAIT].exchange(-1);
+  return v < 0 || v >= 0xffffffffll ? 0xffffffffu : (uint32_t)v;
 }
 
 hipError_t gb_launch_status() {

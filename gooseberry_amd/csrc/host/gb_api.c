@@ -799,7 +799,7 @@ START:
     if (rv != GOOSEBERRY_SUCCESS) break;
     rv = gbd_cg_poll(cg, &st, flog ? trace : NULL);
     if (rv != GOOSEBERRY_SUCCESS) break;
-    if (st.status == GBD_CG_WAITED) {
+    if (st.waited) {
       /* the workgroups did not run side by side: again, in several launches */
       gbd_cg_several_launches(cg);
       if (d_b == d_x) return GOOSEBERRY_ERROR_DEVICE;

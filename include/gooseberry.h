@@ -327,9 +327,14 @@ const char * gooseberry_last_device_error(void);
  * entry point that made it -- once; after < 0 disarms.  An injected launch
  * failure is reported after the kernel has run normally, so no kernel is
  * ever left half-launched.  The library stays usable after an injected
- * failure; an interrupted solve must be started again. */
+ * failure; an interrupted solve must be started again.
+ * GOOSEBERRY_FAULT_CG_WAIT: in exchange number `after` (0, 1, ...) of the next
+ * CG run whose workgroups exchange their sums within one launch, one of them
+ * acts as if its wait had run out; the solve then starts again with several
+ * launches an iteration, and succeeds. */
 #define GOOSEBERRY_FAULT_ALLOC 0
 #define GOOSEBERRY_FAULT_LAUNCH 1
+#define GOOSEBERRY_FAULT_CG_WAIT 2
 int gooseberry_inject_fault(
     int kind,
     long long after);

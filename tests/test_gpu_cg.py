@@ -141,6 +141,42 @@ def test_one_launch_scattered_columns_and_repeats(gb, oracle):
     assert true_rel(oracle, rp, ri, rv, x, b) <= 1.05e-10
 
 
+# A wait given up in one launch, by exchange: the first one (workgroups may
+# still be starting), one amid the run, and the last of the run, after which
+# the other workgroups have the solve's end (iteration cap, convergence) and
+# only the one that gave up lacks its rows of x
+@pytest.mark.parametrize("end", ["cap", "converged"])
+@pytest.mark.parametrize("exchange", ["first", "second", "amid", "last"])
+@pytest.mark.parametrize("n,half", [(1025, 2), (40000, 2), (262144, 2), (20000, 40)])
+def test_wait_given_up_is_never_a_result(gb, oracle, monkeypatch, n, half, exchange, end):
+    print("cg wait given up", n, half, exchange, end, flush=True)
+    # waits that do run out afterwards end after some ten milliseconds
+    monkeypatch.setenv("GOOSEBERRY_CG_SPINS", "20000")
+    rp, ri, rv = band_spd(n, half, n)
+    b = gb.uniform(n, n)
+    niter = 3 if end == "cap" else 0
+    tol = 0.0 if end == "cap" else 1e-10
+    x1, i1 = gb.Matrix(rp, ri, rv).cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
+    M = gb.Matrix(rp, ri, rv)
+    last = 2 * int(i1.niter) - 1
+    at = {"first": 0, "second": 1, "amid": last // 2, "last": last}[exchange]
+    gb.inject_fault(gb.FAULT_CG_WAIT, at)
+    try:
+        x2, i2 = M.cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
+    finally:
+        gb.inject_fault(gb.FAULT_CG_WAIT, -1)
+    assert i2.status == i1.status == (2 if end == "cap" else 1)
+    assert abs(int(i2.niter) - int(i1.niter)) <= 2
+    if end == "cap":
+        # three iterations differ only by the order of the dot products
+        assert np.max(np.abs(x1 - x2)) <= 1e-13 * np.max(np.abs(x1))
+    else:
+        assert true_rel(oracle, rp, ri, rv, x2, b) <= 1.05e-10
+    # the matrix stays with the other kernels, and gives what they gave
+    x3, i3 = M.cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
+    assert i3.niter == i2.niter and np.array_equal(x2, x3)
+
+
 @pytest.mark.parametrize("kind", ["zero_b", "nan_b", "zero_matrix", "indefinite"])
 def test_one_launch_stops_as_the_steps_do(gb, monkeypatch, kind):
     rp, ri, rv = gb.laplacian(2, 40)
