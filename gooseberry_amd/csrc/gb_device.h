@@ -215,9 +215,11 @@ int gbd_cg_enqueue(gbd_cg *cg, uint32_t k);
  * launch (any number: the launch stops where the solve does).  Such a run whose
  * workgroups did not get to run side by side leaves `waited` set in the state,
  * whatever else it says, and the solve has to start again;
- * gbd_cg_several_launches turns to one launch per step. */
+ * gbd_cg_several_launches turns to one launch per step.  gbd_cg_b is the b to
+ * start again with: the caller's, or a copy of it when x is in its place. */
 int gbd_cg_one_launch(const gbd_cg *cg);
 void gbd_cg_several_launches(gbd_cg *cg);
+const double *gbd_cg_b(const gbd_cg *cg);
 int gbd_cg_poll(gbd_cg *cg, gbd_cg_state *st, double *h_trace);
 /* Capture k iterations into a hipGraph once and replay it for each
  * gbd_cg_enqueue_graph call. */

@@ -37,6 +37,7 @@ struct gbd_cg {
   double *r, *p, *ap;
   double *p2;         // one-launch runs: the other buffer of p
   uint64_t *slots;    // one-launch runs: the exchanges' slots
+  double *b0;         // one-launch runs with x in the place of b: a copy of b
   double *partials;   // SpMV p.Ap partials (one per SpMV workgroup)
   double *partials2;  // r.r partials (one per elementwise workgroup)
   uint32_t npartials;
@@ -857,6 +858,7 @@ void gbd_cg_destroy(gbd_cg *cg) {
   (void)gb_dev_free(cg->ap);
   (void)gb_dev_free(cg->p2);
   (void)gb_dev_free(cg->slots);
+  (void)gb_dev_free(cg->b0);
   (void)gb_dev_free(cg->partials);
   (void)gb_dev_free(cg->partials2);
   (void)gb_dev_free(cg->st);
@@ -882,6 +884,13 @@ int gbd_cg_start(gbd_cg *cg, const double *d_b, double *d_x, double tol,
     cg->trace_cap = trace_cap;
   }
   if (cg->x != d_x) gb_cg_drop_graph(cg);
+  if (cg->grid_one && d_b == d_x) {
+    // a run that gives up a wait starts again from b
+    const size_t nb = (size_t)(cg->n ? cg->n : 1) * sizeof(double);
+    if (!cg->b0) GB_HIP(gb_dev_alloc((void **)&cg->b0, nb));
+    GB_HIP(hipMemcpyAsync(cg->b0, d_b, nb, hipMemcpyDeviceToDevice, s));
+    d_b = cg->b0;
+  }
   cg->b = d_b;
   cg->x = d_x;
   gb_cg_init<<<cg->grid_elem, GB_BLOCK, 0, s>>>(d_b, d_x, cg->r, cg->p, cg->n,
@@ -949,6 +958,8 @@ int gbd_cg_one_launch(const gbd_cg *cg) { return cg->grid_one != 0; }
 
 void gbd_cg_several_launches(gbd_cg *cg) { cg->grid_one = 0; }
 
+const double *gbd_cg_b(const gbd_cg *cg) { return cg->b; }
+
 size_t gbd_cg_scratch_max() { return GB_CG_SCRATCH_BYTES; }
 
 int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out) {
@@ -961,7 +972,7 @@ int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out) {
   auto al = [](uint64_t b) { return (b + 255) & ~(uint64_t)255; };
   const uint64_t nb = al((uint64_t)(cg->n ? cg->n : 1) * sizeof(double));
   const uint64_t o_p = nb, o_ap = 2 * nb, o_p2 = 3 * nb;
-  const uint64_t o_sl = 4 * nb;
+  const uint64_t o_b0 = 4 * nb, o_sl = 5 * nb;
   const uint64_t o_pa = cg->grid_one ? o_sl + GB_CGP_SLOT_BYTES : 3 * nb;
   const uint64_t o_pa2 = o_pa + al((uint64_t)cg->npartials * sizeof(double));
   const uint64_t o_st = o_pa2 + al((uint64_t)gb_cg_np2(cg) * sizeof(double));
@@ -990,6 +1001,7 @@ int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out) {
   cg->ap = (double *)(base + o_ap);
   if (cg->grid_one) {
     cg->p2 = (double *)(base + o_p2);
+    cg->b0 = (double *)(base + o_b0);
     cg->slots = (uint64_t *)(base + o_sl);
   }
   cg->partials = (double *)(base + o_pa);

@@ -802,7 +802,7 @@ START:
     if (st.waited) {
       /* the workgroups did not run side by side: again, in several launches */
       gbd_cg_several_launches(cg);
-      if (d_b == d_x) return GOOSEBERRY_ERROR_DEVICE;
+      d_b = gbd_cg_b(cg);
       goto START;
     }
     if (flog) {

@@ -5,6 +5,8 @@ relative residual reached and an iteration count within +-2 of the oracle
 at one thread; at full size, size-independent properties (true residual,
 determinism).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -175,6 +177,38 @@ def test_wait_given_up_is_never_a_result(gb, oracle, monkeypatch, n, half, excha
     # the matrix stays with the other kernels, and gives what they gave
     x3, i3 = M.cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
     assert i3.niter == i2.niter and np.array_equal(x2, x3)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("exchange", [None, 0, 5, "last"])
+def test_solve_in_the_place_of_b(gb, monkeypatch, exchange, noalloc):
+    # x written over b: the same bits as beside it, also when a wait was given
+    # up and the solve started again
+    monkeypatch.setenv("GOOSEBERRY_CG_SPINS", "20000")
+    rp, ri, rv = gb.laplacian(2, 200)
+    b = gb.uniform(5, rp.size - 1)
+    db, dx = gb.DeviceArray.from_host(b), gb.DeviceArray(b.size)
+
+    def solve(to):
+        M = gb.Matrix(rp, ri, rv)  # a matrix of its own: none that gave up before
+        info = gb.CgdInfo()
+        f = gb.lib().gooseberry_matrix_cgd_noalloc if noalloc else gb.lib().gooseberry_matrix_cgd
+        log = () if noalloc else (None,)
+        assert f(M.h, db.ptr, to.ptr, 1e-9, gb.TOL_RELATIVE, 0, *log,
+                 ctypes.byref(info)) == gb.SUCCESS
+        return info
+
+    at = exchange if exchange != "last" else 2 * int(solve(dx).niter) - 1
+    got = []
+    for to in (dx, db):
+        if at is not None:
+            gb.inject_fault(gb.FAULT_CG_WAIT, at)
+        try:
+            info = solve(to)
+        finally:
+            gb.inject_fault(gb.FAULT_CG_WAIT, -1)
+        got.append((to.numpy().tobytes(), int(info.niter), info.status, info.rnorm))
+    assert got[0] == got[1] and got[0][2] == 1
 
 
 @pytest.mark.parametrize("kind", ["zero_b", "nan_b", "zero_matrix", "indefinite"])
