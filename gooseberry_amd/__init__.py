@@ -67,7 +67,7 @@ EXPORTED = [
     "gooseberry_event_record", "gooseberry_event_elapsed_ms",
     "gooseberry_matrix_create", "gooseberry_matrix_create_device",
     "gooseberry_matrix_free", "gooseberry_matrix_replan",
-    "gooseberry_matrix_info", "gooseberry_matrix_spmv",
+    "gooseberry_matrix_info", "gooseberry_matrix_kernels", "gooseberry_matrix_spmv",
     "gooseberry_matrix_spmm", "gooseberry_matrix_cgd", "gooseberry_cgd",
     "gooseberry_generate_laplacian", "gooseberry_generate_uniform",
     "gooseberry_batch_create", "gooseberry_batch_free", "gooseberry_batch_add",
@@ -129,6 +129,10 @@ class _MatrixInfo(C.Structure):
                 ("nblocks_stream", C.c_uint32), ("nrows_wave", C.c_uint32),
                 ("nrows_block", C.c_uint32), ("hist", C.c_uint64 * 33),
                 ("index16", C.c_uint32), ("values8", C.c_uint32)]
+
+
+class _MatrixKernels(C.Structure):
+    _fields_ = [("cg_workgroups", C.c_uint32), ("cg_rows", C.c_uint32)]
 
 
 class CgdInfo(C.Structure):
@@ -214,6 +218,7 @@ def _sig(lib):
         "gooseberry_matrix_free": (i32, [_P]),
         "gooseberry_matrix_replan": (i32, [_P, C.POINTER(_Plan)]),
         "gooseberry_matrix_info": (i32, [_P, C.POINTER(_MatrixInfo)]),
+        "gooseberry_matrix_kernels": (i32, [_P, C.POINTER(_MatrixKernels)]),
         "gooseberry_matrix_spmv": (i32, [_P, _P, _P]),
         "gooseberry_matrix_spmm": (i32, [_P, u32, _P, _P]),
         "gooseberry_matrix_cgd": (i32, [_P, _P, _P, f64, i32, sz, _P, C.POINTER(CgdInfo)]),
@@ -507,6 +512,12 @@ class Matrix:
                 "nblocks_stream": i.nblocks_stream, "nrows_wave": i.nrows_wave,
                 "nrows_block": i.nrows_block, "hist": list(i.hist),
                 "index16": i.index16, "values8": i.values8}
+
+    def kernels(self):
+        """Test hook: the kernels the library takes for this matrix."""
+        k = _MatrixKernels()
+        check(lib().gooseberry_matrix_kernels(self.h, C.byref(k)), "gooseberry_matrix_kernels")
+        return {f: getattr(k, f) for f, _ in k._fields_}
 
     def replan(self, plan=None):
         check(lib().gooseberry_matrix_replan(self.h, _plan(plan)), "gooseberry_matrix_replan")

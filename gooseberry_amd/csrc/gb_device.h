@@ -200,7 +200,7 @@ typedef struct gbd_cg_state {
 typedef struct gbd_cg gbd_cg;
 
 /* Workspace for solving with m (vectors r, p, ap, partials, state). */
-int gbd_cg_create(const gbd_matrix *m, gbd_cg **out);
+int gbd_cg_create(gbd_matrix *m, gbd_cg **out);
 void gbd_cg_destroy(gbd_cg *cg);
 /* x = 0, r = b, p = b, dr = b.b; tol is absolute when rel == 0, else
  * relative to ||b||_2.  trace_cap > 0 records rnorm of each iteration in a
@@ -218,6 +218,8 @@ int gbd_cg_enqueue(gbd_cg *cg, uint32_t k);
  * gbd_cg_several_launches turns to one launch per step.  gbd_cg_b is the b to
  * start again with: the caller's, or a copy of it when x is in its place. */
 int gbd_cg_one_launch(const gbd_cg *cg);
+/* the same of a matrix's plan: workgroups (0: several launches) and rows each */
+void gbd_matrix_cg_shape(const gbd_matrix *m, uint32_t *workgroups, uint32_t *rows);
 void gbd_cg_several_launches(gbd_cg *cg);
 const double *gbd_cg_b(const gbd_cg *cg);
 int gbd_cg_poll(gbd_cg *cg, gbd_cg_state *st, double *h_trace);
@@ -229,7 +231,7 @@ int gbd_cg_enqueue_graph(gbd_cg *cg, uint32_t k);
  * kernel by kernel, or in one launch when small).  INVALIDINPUT when m needs more than
  * gbd_cg_scratch_max() bytes.  The workspace is shared by every such solve
  * on the device and is not destroyed; start it with trace_cap = 0. */
-int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out);
+int gbd_cg_scratch(gbd_matrix *m, gbd_cg **out);
 size_t gbd_cg_scratch_max(void);
 
 /* ----------------------------------------------------- batched solves */

@@ -32,7 +32,7 @@
 #define GB_CG_NGRAPH 7  // captured batches of 1, 2, 4, ..., 64 iterations
 
 struct gbd_cg {
-  const gbd_matrix *m;
+  gbd_matrix *m;
   uint32_t n;
   double *r, *p, *ap;
   double *p2;         // one-launch runs: the other buffer of p
@@ -496,6 +496,24 @@ gb_cgp_empty(uint64_t *__restrict__ slots) {
     slots[(size_t)i * GB_CGP_PAD] = GB_CGP_EMPTY;
 }
 
+// most[q]: the most entries that a range of rows[q] rows has, or 0 for none
+#define GB_CGP_TRIES 3
+struct gb_cgp_tries {
+  uint32_t rows[GB_CGP_TRIES];
+};
+__global__ void __launch_bounds__(GB_BLOCK)
+gb_cgp_most(const uint32_t *__restrict__ rowptr, uint32_t n, gb_cgp_tries t,
+            uint32_t *__restrict__ most) {
+  __shared__ uint32_t m;
+  if (threadIdx.x == 0) m = 0;
+  __syncthreads();
+  const uint32_t rows = t.rows[blockIdx.x];
+  for (uint64_t a = (uint64_t)threadIdx.x * rows; rows && a < n; a += (uint64_t)GB_BLOCK * rows)
+    atomicMax(&m, rowptr[n - a < rows ? n : a + rows] - rowptr[a]);
+  __syncthreads();
+  if (threadIdx.x == 0) most[blockIdx.x] = m;
+}
+
 // k iterations (fewer when the solve stops); p0 holds p before and after,
 // p1 is the other buffer
 template <int R>
@@ -756,49 +774,65 @@ static void *g_scratch_addr[GB_CG_SCRATCH_MAXDEV];
 static gbd_cg g_scratch_cg;            // host bookkeeping of the shared workspace
 static gbd_cg_state g_scratch_hst;     // its polled state (pageable host memory)
 
+// the array's address on the current device
+static int gb_cg_scratch_base(unsigned char **base) {
+  int dev = 0;
+  GB_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= GB_CG_SCRATCH_MAXDEV) {
+    gb_set_error("device %d is beyond the %d devices the scratch table covers", dev,
+                 GB_CG_SCRATCH_MAXDEV);
+    return GOOSEBERRY_ERROR_INVALIDINPUT;
+  }
+  if (!g_scratch_addr[dev]) {
+    void *a = nullptr;
+    GB_HIP(hipGetSymbolAddress(&a, HIP_SYMBOL(scratch)));
+    g_scratch_addr[dev] = a;
+  }
+  *base = (unsigned char *)g_scratch_addr[dev];
+  return GOOSEBERRY_SUCCESS;
+}
+
 // Whether the solve runs in one launch, and on which workgroups: the fewest
 // (the exchanges' time grows with them) whose rows' entries fit their LDS,
-// for matrices with short rows only.  The entries of a range of rows are read
-// from the row pointers once per matrix.
-static void gb_cg_geometry_one(gbd_cg *cg) {
-  const gbd_matrix *m = cg->m;
-  cg->grid_one = 0;
-  if (!cg->n || m->nwave || m->nblockrows || m->nsplit || m->nparts || m->xt.ptr || m->cshift)
-    return;
+// for matrices with short rows only.  Found once per plan, by a kernel that
+// counts the entries of the ranges into the scratch array (no solve is using it
+// then), and kept with the matrix: every workspace of it takes the same kernels.
+static int gb_cg_one_find(gbd_matrix *m) {
+  const uint32_t n = m->nrows;
+  m->cg_grid = m->cg_rows = 0;
+  if (!n || m->nwave || m->nblockrows || m->nsplit || m->nparts || m->xt.ptr || m->cshift)
+    return GOOSEBERRY_SUCCESS;
   uint32_t cus = gb_num_cus();
   if (cus > GB_CGP_GRID) cus = GB_CGP_GRID;
-  for (uint32_t W = GB_CGP_WGS; W <= cus; W *= 2) {
+  gb_cgp_tries t = {{0, 0, 0}};
+  uint32_t W = GB_CGP_WGS, any = 0, most[GB_CGP_TRIES];
+  for (int q = 0; q < GB_CGP_TRIES && W <= cus; ++q, W *= 2) {
     // a row per thread, or fewer rows a workgroup when they are long
-    uint32_t w = gb_div_up(cg->n, GB_CGP_THREADS);
+    uint32_t w = gb_div_up(n, GB_CGP_THREADS);
     const uint32_t we = gb_div_up(m->nnz, GB_CGP_ENTRIES / 8 * 7);
     if (w < we) w = we;
     if (w > W) w = W;
-    const uint32_t rows = gb_div_up(gb_div_up(cg->n, w), GB_WAVE) * GB_WAVE;
-    if (rows > GB_CGP_ROWS * GB_CGP_THREADS) continue;
-    w = gb_div_up(cg->n, rows);
-    uint32_t ptr[GB_CGP_GRID + 1];
-    if (hipMemcpy2DAsync(ptr, 4, m->rowptr, (size_t)rows * 4, 4, w, hipMemcpyDeviceToHost,
-                         gb_stream()) != hipSuccess ||
-        hipStreamSynchronize(gb_stream()) != hipSuccess) {
-      (void)hipGetLastError();
-      return;
-    }
-    ptr[w] = (uint32_t)m->nnz;
-    uint32_t most = 0;
-    for (uint32_t i = 0; i < w; ++i)
-      if (ptr[i + 1] - ptr[i] > most) most = ptr[i + 1] - ptr[i];
-    if (most > GB_CGP_ENTRIES) continue;
-    // GOOSEBERRY_CG_SPINS: the tests' way into the end of a wait
-    const char *e = getenv("GOOSEBERRY_CG_SPINS");
-    cg->spins = e && *e ? (uint32_t)strtoul(e, nullptr, 10) : GB_CGP_SPINS;
-    cg->grid_one = w;
-    cg->rows_one = rows;
-    return;
+    const uint32_t rows = gb_div_up(gb_div_up(n, w), GB_WAVE) * GB_WAVE;
+    if (rows <= GB_CGP_ROWS * GB_CGP_THREADS) any |= t.rows[q] = rows;
   }
+  if (!any) return GOOSEBERRY_SUCCESS;
+  unsigned char *base = nullptr;
+  const int rv = gb_cg_scratch_base(&base);
+  if (rv != GOOSEBERRY_SUCCESS) return rv;
+  gb_cgp_most<<<GB_CGP_TRIES, GB_BLOCK, 0, gb_stream()>>>(m->rowptr, n, t, (uint32_t *)base);
+  GB_LAUNCH_CHECK();
+  GB_HIP(gb_fetch(most, base, sizeof(most)));
+  for (int q = 0; q < GB_CGP_TRIES; ++q) {
+    if (!t.rows[q] || most[q] > GB_CGP_ENTRIES) continue;
+    m->cg_grid = gb_div_up(n, t.rows[q]);
+    m->cg_rows = t.rows[q];
+    break;
+  }
+  return GOOSEBERRY_SUCCESS;
 }
 
 // Launch geometry and partial-array sizes of a solve with m.
-static void gb_cg_geometry(gbd_cg *cg, const gbd_matrix *m) {
+static int gb_cg_geometry(gbd_cg *cg, gbd_matrix *m) {
   cg->m = m;
   cg->n = m->nrows;
   uint32_t ge = gb_div_up(cg->n ? cg->n : 1, GB_BLOCK);
@@ -810,22 +844,35 @@ static void gb_cg_geometry(gbd_cg *cg, const gbd_matrix *m) {
   if (gv > GB_CGV_GRID) gv = GB_CGV_GRID;
   cg->chunk = gb_div_up(gb_div_up(nn, gv), GB_WAVE) * GB_WAVE;
   cg->grid_vec = gb_div_up(nn, cg->chunk);
-  gb_cg_geometry_one(cg);
   uint32_t gs = gb_spmv_npartials(m);
   cg->npartials = gs > cg->grid_elem ? gs : cg->grid_elem;
+  if (!m->cg_known) {
+    const int rv = gb_cg_one_find(m);
+    if (rv != GOOSEBERRY_SUCCESS) return rv;
+    m->cg_known = true;
+  }
+  cg->grid_one = m->cg_grid;
+  cg->rows_one = m->cg_rows;
+  // GOOSEBERRY_CG_SPINS: the tests' way into the end of a wait
+  const char *e = getenv("GOOSEBERRY_CG_SPINS");
+  cg->spins = e && *e ? (uint32_t)strtoul(e, nullptr, 10) : GB_CGP_SPINS;
+  return GOOSEBERRY_SUCCESS;
 }
 
 static uint32_t gb_cg_np2(const gbd_cg *cg) {
   return cg->grid_elem > cg->grid_vec ? cg->grid_elem : cg->grid_vec;
 }
 
-int gbd_cg_create(const gbd_matrix *m, gbd_cg **out) {
+int gbd_cg_create(gbd_matrix *m, gbd_cg **out) {
   int rv = gb_ensure_init();
   if (rv != GOOSEBERRY_SUCCESS) return rv;
   if (m->nrows != m->ncols) return GOOSEBERRY_ERROR_INVALIDINPUT;
   gbd_cg *cg = (gbd_cg *)calloc(1, sizeof(gbd_cg));
   if (!cg) return GOOSEBERRY_ERROR_NOMEMORY;
-  gb_cg_geometry(cg, m);
+  if ((rv = gb_cg_geometry(cg, m)) != GOOSEBERRY_SUCCESS) {
+    free(cg);
+    return rv;
+  }
   size_t nb = (size_t)(cg->n ? cg->n : 1) * sizeof(double);
   hipError_t e = gb_dev_alloc((void **)&cg->r, nb);
   if (e == hipSuccess) e = gb_dev_alloc((void **)&cg->p, nb);
@@ -954,6 +1001,11 @@ int gbd_cg_poll(gbd_cg *cg, gbd_cg_state *st, double *h_trace) {
   return GOOSEBERRY_SUCCESS;
 }
 
+void gbd_matrix_cg_shape(const gbd_matrix *m, uint32_t *workgroups, uint32_t *rows) {
+  *workgroups = m->cg_grid;
+  *rows = m->cg_rows;
+}
+
 int gbd_cg_one_launch(const gbd_cg *cg) { return cg->grid_one != 0; }
 
 void gbd_cg_several_launches(gbd_cg *cg) { cg->grid_one = 0; }
@@ -962,13 +1014,13 @@ const double *gbd_cg_b(const gbd_cg *cg) { return cg->b; }
 
 size_t gbd_cg_scratch_max() { return GB_CG_SCRATCH_BYTES; }
 
-int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out) {
+int gbd_cg_scratch(gbd_matrix *m, gbd_cg **out) {
   int rv = gb_ensure_init();
   if (rv != GOOSEBERRY_SUCCESS) return rv;
   if (m->nrows != m->ncols) return GOOSEBERRY_ERROR_INVALIDINPUT;
   gbd_cg *cg = &g_scratch_cg;
   memset(cg, 0, sizeof(*cg));
-  gb_cg_geometry(cg, m);
+  if ((rv = gb_cg_geometry(cg, m)) != GOOSEBERRY_SUCCESS) return rv;
   auto al = [](uint64_t b) { return (b + 255) & ~(uint64_t)255; };
   const uint64_t nb = al((uint64_t)(cg->n ? cg->n : 1) * sizeof(double));
   const uint64_t o_p = nb, o_ap = 2 * nb, o_p2 = 3 * nb;
@@ -983,19 +1035,8 @@ int gbd_cg_scratch(const gbd_matrix *m, gbd_cg **out) {
                  (unsigned long long)need, m->nrows, (unsigned long long)GB_CG_SCRATCH_BYTES);
     return GOOSEBERRY_ERROR_INVALIDINPUT;
   }
-  int dev = 0;
-  GB_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= GB_CG_SCRATCH_MAXDEV) {
-    gb_set_error("device %d is beyond the %d devices the scratch table covers", dev,
-                 GB_CG_SCRATCH_MAXDEV);
-    return GOOSEBERRY_ERROR_INVALIDINPUT;
-  }
-  if (!g_scratch_addr[dev]) {
-    void *a = nullptr;
-    GB_HIP(hipGetSymbolAddress(&a, HIP_SYMBOL(scratch)));
-    g_scratch_addr[dev] = a;
-  }
-  unsigned char *base = (unsigned char *)g_scratch_addr[dev];
+  unsigned char *base = nullptr;
+  if ((rv = gb_cg_scratch_base(&base)) != GOOSEBERRY_SUCCESS) return rv;
   cg->r = (double *)base;
   cg->p = (double *)(base + o_p);
   cg->ap = (double *)(base + o_ap);

@@ -88,6 +88,10 @@ struct gbd_matrix {
   uint64_t *pbase;    // host, nparts + 1
   uint32_t *prowptr;  // nrows + nparts
   uint64_t *rowptr64; // nrows + 1
+  // CG in one launch (gb_cg.hip): what the plan's first solve found
+  bool cg_known;
+  uint32_t cg_grid;     // workgroups, or 0: several launches an iteration
+  uint32_t cg_rows;     // and rows per workgroup
   uint32_t holders;   // batch slots holding pointers into the plan: while
                       // nonzero the plan must not be rebuilt or freed
 };

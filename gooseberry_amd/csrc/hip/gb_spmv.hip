@@ -1751,6 +1751,8 @@ static int gb_plan_build(gbd_matrix *m) {
   gb_vdict_free(m);
   if (!m->view) gb_xtile_free(m);
   m->pipe_grid = 0;
+  m->cg_known = false;
+  m->cg_grid = m->cg_rows = 0;
   memset(m->hist, 0, sizeof(m->hist));
   m->nstream = m->nwave = m->nblockrows = 0;
   if (m->nparts) return gb_parts_plan(m);

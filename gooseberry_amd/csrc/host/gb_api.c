@@ -395,6 +395,19 @@ int gooseberry_matrix_info(gooseberry_matrix_t mat,
   return GOOSEBERRY_SUCCESS;
 }
 
+int gooseberry_matrix_kernels(gooseberry_matrix_t mat,
+    gooseberry_matrix_kernels_t *kernels)
+{
+  GB_API_GUARD();
+  if (!mat || !kernels) return GOOSEBERRY_ERROR_INVALIDINPUT;
+  memset(kernels, 0, sizeof(*kernels));
+  uint32_t wgs, rows;
+  gbd_matrix_cg_shape(mat->m, &wgs, &rows);
+  kernels->cg_workgroups = wgs;
+  kernels->cg_rows = rows;
+  return GOOSEBERRY_SUCCESS;
+}
+
 int gooseberry_matrix_spmv(gooseberry_matrix_t mat, const real_t *d_x,
     real_t *d_y)
 {

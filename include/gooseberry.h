@@ -499,6 +499,19 @@ int gooseberry_matrix_info(
     gooseberry_matrix_t mat,
     gooseberry_matrix_info_t * info);
 
+/* Which kernels the library takes for a matrix, a test hook with no
+ * counterpart in the reference. */
+typedef struct gooseberry_matrix_kernels_t {
+  dim_t cg_workgroups;    /* gooseberry_matrix_cgd and _noalloc, as of the last
+                             solve: workgroups of a run of iterations in one
+                             launch, or 0: several launches an iteration */
+  dim_t cg_rows;          /* and rows of each workgroup */
+} gooseberry_matrix_kernels_t;
+
+int gooseberry_matrix_kernels(
+    gooseberry_matrix_t mat,
+    gooseberry_matrix_kernels_t * kernels);
+
 /* y = A x, device vectors, enqueued on the library stream. */
 int gooseberry_matrix_spmv(
     gooseberry_matrix_t mat,

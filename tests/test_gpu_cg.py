@@ -143,13 +143,67 @@ def test_one_launch_scattered_columns_and_repeats(gb, oracle):
     assert true_rel(oracle, rp, ri, rv, x, b) <= 1.05e-10
 
 
+# (workgroups, rows each) of the one-launch solve on 256 CUs; (0, 0): rows over
+# 64 entries, entries that fit no choice of workgroups, more than 2048 rows a
+# workgroup
+SHAPES = [
+    (1, 0, 1, 64), (512, 2, 1, 512), (513, 2, 2, 320), (1025, 20, 3, 384), (10000, 15, 20, 512),
+    (20000, 22, 53, 384), (32768, 2, 64, 512), (32769, 2, 57, 576), (40000, 18, 90, 448),
+    (65600, 2, 61, 1088), (80000, 15, 157, 512), (131072, 2, 64, 2048), (131073, 2, 121, 1088),
+    (262145, 2, 241, 1088), (400000, 3, 250, 1600), (524288, 1, 256, 2048),
+    (1025, 40, 0, 0), (40000, 20, 0, 0), (524289, 2, 0, 0)]
+
+
+@pytest.mark.parametrize("n,half,workgroups,rows", SHAPES)
+def test_one_launch_shapes(gb, oracle, n, half, workgroups, rows):
+    print("cg shape", n, half, flush=True)
+    rp, ri, rv = band_spd(n, half, n)
+    M = gb.Matrix(rp, ri, rv)
+    b = gb.uniform(n, n)
+    x, info = M.cgd(b, 1e-10, gb.TOL_RELATIVE)
+    want = {"cg_workgroups": workgroups, "cg_rows": rows}
+    assert {k: M.kernels()[k] for k in want} == want
+    assert info.status == 1 and true_rel(oracle, rp, ri, rv, x, b) <= 1.05e-10
+    # the allocation-free entry point takes the same kernels, also first
+    N = gb.Matrix(rp, ri, rv)
+    db, dx, i2 = gb.DeviceArray.from_host(b), gb.DeviceArray(n), gb.CgdInfo()
+    assert gb.lib().gooseberry_matrix_cgd_noalloc(N.h, db.ptr, dx.ptr, 1e-10, gb.TOL_RELATIVE, 0,
+                                                 ctypes.byref(i2)) == gb.SUCCESS
+    assert {k: N.kernels()[k] for k in want} == want
+    assert i2.niter == info.niter and np.array_equal(dx.numpy(), x)
+
+
+def test_one_launch_choice_follows_the_plan_and_reports_failures(gb):
+    rp, ri, rv = gb.laplacian(2, 100)
+    M = gb.Matrix(rp, ri, rv)
+    b = gb.uniform(1, M.nrows)
+    # the first launch of a plan's first solve counts its entries
+    gb.inject_fault(gb.FAULT_LAUNCH, 0)
+    try:
+        with pytest.raises(gb.GooseberryError) as e:
+            M.cgd(b, 1e-8, gb.TOL_RELATIVE)
+    finally:
+        gb.inject_fault(gb.FAULT_LAUNCH, -1)
+    assert e.value.name == "DEVICE" and M.kernels()["cg_workgroups"] == 0
+    x, _ = M.cgd(b, 1e-8, gb.TOL_RELATIVE)
+    assert M.kernels()["cg_workgroups"] == 20
+    for plan in ({"csplit": 2}, {"xtile": 1024}, {"short_max": 4}):
+        M.replan(plan)
+        y, info = M.cgd(b, 1e-8, gb.TOL_RELATIVE)
+        assert info.status == 1 and M.kernels()["cg_workgroups"] == 0
+        assert np.linalg.norm(x - y) <= 1e-5 * np.linalg.norm(x)
+    M.replan(None)
+    y, _ = M.cgd(b, 1e-8, gb.TOL_RELATIVE)
+    assert M.kernels()["cg_workgroups"] == 20 and np.array_equal(x, y)
+
+
 # A wait given up in one launch, by exchange: the first one (workgroups may
 # still be starting), one amid the run, and the last of the run, after which
 # the other workgroups have the solve's end (iteration cap, convergence) and
 # only the one that gave up lacks its rows of x
 @pytest.mark.parametrize("end", ["cap", "converged"])
 @pytest.mark.parametrize("exchange", ["first", "second", "amid", "last"])
-@pytest.mark.parametrize("n,half", [(1025, 2), (40000, 2), (262144, 2), (20000, 40)])
+@pytest.mark.parametrize("n,half", [(1025, 2), (40000, 2), (262144, 2), (20000, 22)])
 def test_wait_given_up_is_never_a_result(gb, oracle, monkeypatch, n, half, exchange, end):
     print("cg wait given up", n, half, exchange, end, flush=True)
     # waits that do run out afterwards end after some ten milliseconds
