@@ -215,7 +215,8 @@ int gbd_cg_enqueue(gbd_cg *cg, uint32_t k);
  * launch (any number: the launch stops where the solve does).  Such a run whose
  * workgroups did not get to run side by side leaves `waited` set in the state,
  * whatever else it says, and the solve has to start again;
- * gbd_cg_several_launches turns to one launch per step.  gbd_cg_b is the b to
+ * gbd_cg_several_launches turns to one launch per step, for every workspace of
+ * the matrix until its plan is rebuilt.  gbd_cg_b is the b to
  * start again with: the caller's, or a copy of it when x is in its place. */
 int gbd_cg_one_launch(const gbd_cg *cg);
 /* the same of a matrix's plan: workgroups (0: several launches) and rows each */

@@ -393,7 +393,8 @@ gb_cg_update_xp(double *__restrict__ x, const double *__restrict__ r,
 // leaves, without its rows of x; the others then run out of time in a later
 // exchange, or, if this was the last, end the solve.  So `waited` is a word
 // that only the set-up clears and no other end of a run touches, and the host
-// looks at it before all else: the solve starts again on the other kernels.
+// looks at it before all else: the solve starts again on the other kernels,
+// and the matrix stays with them until its plan is built anew.
 // Workgroups may still be starting when it is set, and one thread decides for
 // each of them whether it runs.
 //
@@ -412,7 +413,7 @@ gb_cg_update_xp(double *__restrict__ x, const double *__restrict__ r,
 #define GB_CGP_GRID 256u
 #define GB_CGP_ROWS 4          // rows per thread at most
 #define GB_CGP_WGS 64u         // workgroups, while the rows fit them
-#define GB_CGP_SPINS (1u << 20)
+#define GB_CGP_SPINS (1u << 20)  // 0.16 s, paid once: the matrix takes the others then
 static_assert(GB_CGP_GRID <= GB_CGP_THREADS, "one slot per thread");
 #define GB_CGP_PAD 16          // slots a cache line apart
 #define GB_CGP_SLOT_BYTES (3ull * GB_CGP_GRID * GB_CGP_PAD * 8)
@@ -931,6 +932,7 @@ int gbd_cg_start(gbd_cg *cg, const double *d_b, double *d_x, double tol,
     cg->trace_cap = trace_cap;
   }
   if (cg->x != d_x) gb_cg_drop_graph(cg);
+  if (!cg->m->cg_grid) cg->grid_one = 0;  // another workspace of the matrix gave up
   if (cg->grid_one && d_b == d_x) {
     // a run that gives up a wait starts again from b
     const size_t nb = (size_t)(cg->n ? cg->n : 1) * sizeof(double);
@@ -1008,7 +1010,7 @@ void gbd_matrix_cg_shape(const gbd_matrix *m, uint32_t *workgroups, uint32_t *ro
 
 int gbd_cg_one_launch(const gbd_cg *cg) { return cg->grid_one != 0; }
 
-void gbd_cg_several_launches(gbd_cg *cg) { cg->grid_one = 0; }
+void gbd_cg_several_launches(gbd_cg *cg) { cg->grid_one = cg->m->cg_grid = cg->m->cg_rows = 0; }
 
 const double *gbd_cg_b(const gbd_cg *cg) { return cg->b; }
 

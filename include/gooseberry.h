@@ -542,8 +542,13 @@ typedef struct gooseberry_cgd_info_t {
 /* CG of src/cgd.c:40-129 on a resident matrix: x0 = 0, the reference's
  * update order, stop when sqrt(r.r) <= threshold or after niter SpMVs
  * (niter == 0: no cap).  b == 0 returns x = 0 at once.  d_b, d_x device
- * vectors.  log (a FILE *, may be NULL) receives the reference's
- * "ITER: i RMSE: v" lines. */
+ * vectors (d_x may be d_b).  log (a FILE *, may be NULL) receives the
+ * reference's "ITER: i RMSE: v" lines.  Small systems run whole batches of
+ * iterations in one launch, whose workgroups wait for each other; where other
+ * work keeps them from running side by side (0.2 s at most), the solve starts
+ * again with several launches an iteration, and the matrix stays with those
+ * until its plan is rebuilt.  The two ways differ by the order of the dot
+ * products; on either a solve gives the same bits every time. */
 int gooseberry_matrix_cgd(
     gooseberry_matrix_t mat,
     const real_t * d_b,
@@ -557,12 +562,13 @@ int gooseberry_matrix_cgd(
 /* gooseberry_matrix_cgd without any device allocation, for callers that
  * cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  The
- * work vectors (r, p, Ap: 24 bytes per row), the partial sums and the state
- * live in one file-scope device array of
+ * work vectors (r, p, Ap: 24 bytes per row; 40 for the small systems that run
+ * in one launch), the partial sums and the state live in one file-scope device
+ * array of
  * gooseberry_cgd_noalloc_max_bytes() bytes (128 MiB: about 5.5 million
  * rows) that each GPU holds until the process ends; a larger system returns
- * GOOSEBERRY_ERROR_INVALIDINPUT before any launch.  Kernels are launched one
- * by one (no graphs); no log.  Every call on a GPU shares that array, so
+ * GOOSEBERRY_ERROR_INVALIDINPUT before any launch.  Larger systems' kernels are
+ * launched one by one (no graphs); no log.  Every call on a GPU shares that array, so
  * calls that overlap on one GPU race (the library lock serialises the calls
  * of one process).  Same results, bit for bit, as gooseberry_matrix_cgd. */
 int gooseberry_matrix_cgd_noalloc(

@@ -233,6 +233,43 @@ def test_wait_given_up_is_never_a_result(gb, oracle, monkeypatch, n, half, excha
     assert i3.niter == i2.niter and np.array_equal(x2, x3)
 
 
+@pytest.mark.parametrize("first", ["cgd", "noalloc"])
+def test_a_wait_given_up_is_remembered_by_the_matrix(gb, monkeypatch, first):
+    # after one entry point gave up a wait, neither runs in one launch again (the
+    # armed fault is not taken), and both give the same bits; a new plan may
+    monkeypatch.setenv("GOOSEBERRY_CG_SPINS", "20000")
+    rp, ri, rv = gb.laplacian(2, 150)
+    M = gb.Matrix(rp, ri, rv)
+    b = gb.uniform(9, M.nrows)
+    db, dx = gb.DeviceArray.from_host(b), gb.DeviceArray(b.size)
+
+    def solve(entry):
+        info = gb.CgdInfo()
+        f = getattr(gb.lib(), "gooseberry_matrix_cgd" + ("" if entry == "cgd" else "_noalloc"))
+        log = (None,) if entry == "cgd" else ()
+        assert f(M.h, db.ptr, dx.ptr, 1e-9, gb.TOL_RELATIVE, 0, *log,
+                 ctypes.byref(info)) == gb.SUCCESS
+        return dx.numpy().tobytes(), int(info.niter), info.rnorm
+
+    other = "noalloc" if first == "cgd" else "cgd"
+    one = solve(other)
+    assert solve(first) == one and M.kernels()["cg_workgroups"] == 44
+    try:
+        gb.inject_fault(gb.FAULT_CG_WAIT, 2)
+        several = solve(first)
+        assert M.kernels()["cg_workgroups"] == 0 and several != one
+        gb.inject_fault(gb.FAULT_CG_WAIT, 0)
+        assert solve(other) == several and solve(first) == several
+        M.replan(None)
+        assert M.kernels()["cg_workgroups"] == 0
+        assert solve(other) == several and M.kernels()["cg_workgroups"] == 0  # takes the fault
+        M.replan(None)
+        assert solve(other) == one and solve(first) == one
+        assert M.kernels()["cg_workgroups"] == 44
+    finally:
+        gb.inject_fault(gb.FAULT_CG_WAIT, -1)
+
+
 @pytest.mark.parametrize("noalloc", [False, True])
 @pytest.mark.parametrize("exchange", [None, 0, 5, "last"])
 def test_solve_in_the_place_of_b(gb, monkeypatch, exchange, noalloc):
