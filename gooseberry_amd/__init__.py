@@ -132,7 +132,8 @@ class _MatrixInfo(C.Structure):
 
 
 class _MatrixKernels(C.Structure):
-    _fields_ = [("cg_workgroups", C.c_uint32), ("cg_rows", C.c_uint32)]
+    _fields_ = [("cg_workgroups", C.c_uint32), ("cg_rows", C.c_uint32),
+                ("spmv_lds", C.c_uint32)]
 
 
 class CgdInfo(C.Structure):

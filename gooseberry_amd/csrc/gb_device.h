@@ -168,6 +168,9 @@ int gbd_matrix_make_f32(gbd_matrix *m);
  * (square matrices with a positive, finite diagonal; INVALIDINPUT else). */
 int gbd_matrix_make_f32_jacobi(gbd_matrix *m);
 
+/* bytes of unused LDS that the row-block SpMV asks for (few workgroups per CU) */
+uint32_t gbd_matrix_spmv_lds(const gbd_matrix *m);
+
 /* y = A x (FP64).  bitwise the reference's row-sequential sums for rows in
  * LDS-staged blocks; tree-reduced for longer rows. */
 int gbd_spmv(const gbd_matrix *m, const double *d_x, double *d_y);

@@ -1198,13 +1198,13 @@ int gbd_batch_commit(gbd_batch *B, const uint8_t *active) {
   // matrices in segment 0
   uint32_t nseg = 1;
   uint64_t cnt[GB_SPLIT_MAX] = {0};
-  uint64_t scattered = 0, blocks = 0;  // items of row blocks without 16-bit offsets, all items
+  uint64_t scattered = 0, blocks = 0;  // items of row blocks of scattered columns, all items
   for (uint32_t i = 0; i < B->max_slots; ++i) {
     if (!B->used[i] || (active && !active[i])) continue;
     const gb_bsys &S = B->h_sys[i];
     if (S.xt.ptr) continue;  // launched on its own
     if (!S.nsplit) {
-      scattered += S.pl.dcol ? 0 : S.pl.nstream;
+      scattered += B->slot_mat[i]->scattered && !S.pl.dcol ? S.pl.nstream : 0;
       blocks += S.pl.nwork;
     }
     if (S.nsplit) {

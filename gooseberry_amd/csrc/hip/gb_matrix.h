@@ -88,6 +88,7 @@ struct gbd_matrix {
   uint64_t *pbase;    // host, nparts + 1
   uint32_t *prowptr;  // nrows + nparts
   uint64_t *rowptr64; // nrows + 1
+  bool scattered;       // the short rows' columns jump from row to row
   // CG in one launch (gb_cg.hip): what the plan's first solve found
   bool cg_known;
   uint32_t cg_grid;     // workgroups, or 0: several launches an iteration
@@ -177,15 +178,19 @@ static inline uint32_t gb_spmv_nwork(const gbd_matrix *m) {
 // Row blocks whose columns scatter over x gather best from three workgroups of
 // 256 threads per CU: with more, their gathers queue up in the caches.  These
 // bytes of LDS, unused, on top of a row-block kernel's own (9 or 18 KB) keep
-// it to three.  Taken where the plan has no 16-bit offsets and nine of ten work
-// items are row blocks; wavefront rows (100 entries: 136 us at eight
-// workgroups per CU, 199 us at three) and banded matrices want them all.
-// Random matrices of 29 entries a row, FP32 / FP64 SpMV, at 8 and 3 workgroups:
-// 100,000 rows 19.0 -> 18.0 / 20.4 -> 19.6 us, 300,007 rows 52.2 -> 43.4 /
-// 54.9 -> 48.3 us, 1,048,576 rows 198 -> 173 / 309 -> 305 us.
+// it to three.  Taken where the rows' columns jump (gb_plan_classify: half of
+// the short rows or more), the plan has no 16-bit offsets and nine of ten work
+// items are row blocks.  Random matrices of 29 entries a row, FP32 / FP64 SpMV,
+// at 8 and 3 workgroups: 100,000 rows 19.5 -> 18.5 / 21.1 -> 20.3 us, 300,007
+// rows 52.9 -> 43.8 / 55.8 -> 49.6 us, 1,048,576 rows 200 -> 173 / 309 -> 306 us,
+// in four column slices 216 -> 178 / 212 -> 188.  Wavefront rows (100 entries:
+// 136 us at eight, 199 at three) want them all, and so do stencils whose
+// offsets do not fit 16 bits (200 x 200 x 100 points 55.4 and 77.7 / 74.4 and
+// 90.0 us) or were not asked for (160^3 points 59.2 and 85.1 / 76.5 and 95.6).
 #define GB_SPMV_FEW_LDS 34000u
 static inline uint32_t gb_spmv_few_lds(const gbd_matrix *m) {
-  const bool few = !m->dcol && (uint64_t)m->nstream * 10 >= (uint64_t)gb_spmv_nwork(m) * 9;
+  const bool few = m->scattered && !m->dcol &&
+                   (uint64_t)m->nstream * 10 >= (uint64_t)gb_spmv_nwork(m) * 9;
   return few ? GB_SPMV_FEW_LDS : 0;
 }
 // workgroups of one SpMV launch (the number of p.Ap partials with DOT)

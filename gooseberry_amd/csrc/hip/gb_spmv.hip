@@ -35,14 +35,19 @@ __device__ __forceinline__ uint32_t gb_row_class(uint32_t len,
 #define GB_PLAN_MISFIT 33  // short rows that rule out 16-bit offsets (below)
 #define GB_PLAN_NWAVE 34   // wave rows
 #define GB_PLAN_NBLOCK 35  // block rows
-#define GB_PLAN_NST 36     // row blocks (the scan of the flags, 32 bits)
-#define GB_PLAN_NCOUNT 37
+#define GB_PLAN_NJUMP 36   // short rows far from the row before (below)
+#define GB_PLAN_NST 37     // row blocks (the scan of the flags, 32 bits)
+#define GB_PLAN_NCOUNT 38
+#define GB_PLAN_JUMP 256   // columns: 2 KB of x
 
 // Per row: bin (0 short / 1 wave / 2 block), the "starts a row block" flag
 // and the counts.  GB_PLAN_MISFIT counts the short rows whose first or last
 // column rules out 16-bit offsets from any block they can fall in (column -
 // row above 32767, or below -32768 - (rowcap - 1)), so that the plan skips
-// building offsets that cannot fit.
+// building offsets that cannot fit.  GB_PLAN_NJUMP counts the short rows whose
+// first or last column lies more than GB_PLAN_JUMP from that of the row before
+// (in the same wavefront): nearly all where the columns scatter, one in a grid
+// line or fewer in a stencil, however far apart its planes are.
 //
 // A row in the window of the row before it starts a block at every rowcap-th
 // row from the window's first: the last row at or before it whose window is
@@ -62,7 +67,7 @@ gb_plan_classify(const uint32_t *__restrict__ rowptr,
   const uint32_t lane = threadIdx.x & (GB_WAVE - 1);
   for (uint32_t i = threadIdx.x; i < GB_PLAN_NST; i += GB_BLOCK) h[i] = 0;
   __syncthreads();
-  uint32_t nmis = 0, nw = 0, nb = 0;  // of the wavefront
+  uint32_t nmis = 0, nw = 0, nb = 0, nj = 0;  // of the wavefront
   for (uint64_t base = (uint64_t)blockIdx.x * GB_BLOCK + (threadIdx.x - lane); base < nrows;
        base += (uint64_t)gridDim.x * GB_BLOCK) {
     const uint32_t r0 = (uint32_t)base, r = r0 + lane;
@@ -76,13 +81,21 @@ gb_plan_classify(const uint32_t *__restrict__ rowptr,
     const uint32_t len = b - a, c = gb_row_class(len, p);
     const uint32_t w = a / p.window;
     const bool fresh = r == 0 || pa / p.window != w;  // the window's first row
-    bool misfit = false;
-    if (live && c == 0 && len && !p.wide_index) {
-      const int64_t lo = -32768 - (int64_t)(p.rowcap - 1);
-      const int64_t rr = (int64_t)r + cshift;
-      const int64_t d0 = (int64_t)rowind[a] - rr, d1 = (int64_t)rowind[b - 1] - rr;
-      misfit = d0 > 32767 || d0 < lo || d1 > 32767 || d1 < lo;
+    const bool cols = live && c == 0 && len;
+    uint32_t c0 = 0, c1 = 0;
+    if (cols) {
+      c0 = rowind[a];
+      c1 = rowind[b - 1];
     }
+    const int64_t lo = -32768 - (int64_t)(p.rowcap - 1);
+    const int64_t rr = (int64_t)r + cshift;
+    const int64_t d0 = (int64_t)c0 - rr, d1 = (int64_t)c1 - rr;
+    const bool misfit = cols && (d0 > 32767 || d0 < lo || d1 > 32767 || d1 < lo);
+    const uint32_t p0 = (uint32_t)__shfl_up((int)c0, 1, GB_WAVE);
+    const uint32_t p1 = (uint32_t)__shfl_up((int)c1, 1, GB_WAVE);
+    const bool pair = cols && (__ballot(cols) << 1 >> lane & 1ull);
+    const bool jump = pair && ((c0 > p0 ? c0 - p0 : p0 - c0) > GB_PLAN_JUMP ||
+                               (c1 > p1 ? c1 - p1 : p1 - c1) > GB_PLAN_JUMP);
     bool f = live && c == 0 && (fresh || gb_row_class(a - pa, p) != 0);
     const uint64_t starts = __ballot(live && fresh);
     const uint64_t before = starts & ((2ull << lane) - 1ull);
@@ -120,11 +133,13 @@ gb_plan_classify(const uint32_t *__restrict__ rowptr,
       todo &= ~same;
     }
     nmis += (uint32_t)__popcll(__ballot(misfit));
+    nj += (uint32_t)__popcll(__ballot(jump));
     nw += (uint32_t)__popcll(__ballot(live && c == 1));
     nb += (uint32_t)__popcll(__ballot(live && c == 2));
   }
   if (lane == 0) {
     if (nmis) atomicAdd(&h[GB_PLAN_MISFIT], nmis);
+    if (nj) atomicAdd(&h[GB_PLAN_NJUMP], nj);
     if (nw) atomicAdd(&h[GB_PLAN_NWAVE], nw);
     if (nb) atomicAdd(&h[GB_PLAN_NBLOCK], nb);
   }
@@ -1751,6 +1766,7 @@ static int gb_plan_build(gbd_matrix *m) {
   gb_vdict_free(m);
   if (!m->view) gb_xtile_free(m);
   m->pipe_grid = 0;
+  m->scattered = false;
   m->cg_known = false;
   m->cg_grid = m->cg_rows = 0;
   memset(m->hist, 0, sizeof(m->hist));
@@ -1782,6 +1798,7 @@ static int gb_plan_build(gbd_matrix *m) {
   m->nstream = nst;
   m->nwave = (uint32_t)hc[GB_PLAN_NWAVE];
   m->nblockrows = (uint32_t)hc[GB_PLAN_NBLOCK];
+  m->scattered = 2 * hc[GB_PLAN_NJUMP] >= n - m->nwave - m->nblockrows - hc[0] && hc[GB_PLAN_NJUMP];
   if (m->nwave || m->nblockrows) {  // short rows are reached by their blocks
     GB_HIP(gb_dev_alloc((void **)&m->rowbins, (size_t)n * 4));
     rv = gbd_countingsort_kv_unchecked(cls, nullptr, 0, 2, n, m->rowbins, nullptr);
@@ -1942,7 +1959,6 @@ int gbd_matrix_create_trusted(uint32_t nrows, uint32_t ncols, uint32_t *d_rowptr
 
 // One 64-bit row pointer read back (the part boundaries' binary search).
 static int gb_rowptr64_at(const uint64_t *d_rowptr64, uint32_t i, uint64_t *v) {
-  hipStream_t s = gb_stream();
   GB_HIP(gb_fetch(v, d_rowptr64 + i, 8));
   return GOOSEBERRY_SUCCESS;
 }
@@ -2177,6 +2193,10 @@ int gbd_matrix_info(const gbd_matrix *m, uint32_t *nrows, uint32_t *ncols,
 
 // row parts: 1 when every part reads 16-bit offsets; the largest value
 // table of the parts when every part is value-indexed
+uint32_t gbd_matrix_spmv_lds(const gbd_matrix *m) {
+  return gb_spmv_few_lds(m->nsplit ? m->split[0] : m->nparts ? m->parts[0] : m);
+}
+
 uint32_t gbd_matrix_index16(const gbd_matrix *m) {
   if (!m->nparts) return m->dcol ? 1u : 0u;
   for (uint32_t q = 0; q < m->nparts; ++q)

@@ -405,6 +405,7 @@ int gooseberry_matrix_kernels(gooseberry_matrix_t mat,
   gbd_matrix_cg_shape(mat->m, &wgs, &rows);
   kernels->cg_workgroups = wgs;
   kernels->cg_rows = rows;
+  kernels->spmv_lds = gbd_matrix_spmv_lds(mat->m);
   return GOOSEBERRY_SUCCESS;
 }
 

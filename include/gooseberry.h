@@ -506,6 +506,9 @@ typedef struct gooseberry_matrix_kernels_t {
                              solve: workgroups of a run of iterations in one
                              launch, or 0: several launches an iteration */
   dim_t cg_rows;          /* and rows of each workgroup */
+  dim_t spmv_lds;         /* bytes of LDS that the row-block SpMV leaves unused to
+                             have fewer workgroups per CU (scattered columns),
+                             of the first slice or part where there are some */
 } gooseberry_matrix_kernels_t;
 
 int gooseberry_matrix_kernels(

@@ -581,3 +581,49 @@ def test_plan_row_blocks(gb, oracle, n, shape, plan):
     mag = np.add.reduceat(np.append(np.abs(rv * x[ri]), 0.0), rp[:-1].astype(np.int64))
     mag[deg == 0] = 0.0
     assert np.all(np.abs(M.spmv(x) - ref) <= 2 * np.maximum(deg, 1) * 2.3e-16 * mag)
+
+
+def _far_stencil(n, far):
+    # rows of columns r - far, r, r + far: no 16-bit offsets, but rows side by side
+    r = np.arange(n)
+    cols = np.stack([r - far, r, r + far], 1)
+    keep = (cols >= 0) & (cols < n)
+    rp = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.uint32)
+    return rp, cols[keep].astype(np.uint32)
+
+
+# Few workgroups per CU only where the columns of most rows jump: random
+# matrices and their column slices; not stencils, whatever their offsets, nor
+# random matrices with 16-bit offsets or many long rows
+@pytest.mark.parametrize("kind,plan,few", [
+    ("random", None, True), ("random", {"wide_index": 1}, True), ("random", {"csplit": 4}, True),
+    ("random", {"exact": 1}, True), ("random", {"short_max": 16, "wave_max": 64}, False),
+    ("random_small", None, False), ("unsorted_rows", None, True), ("half", None, False),
+    ("far_stencil", None, False), ("far_stencil", {"csplit": 4}, False),
+    ("stencil", None, False), ("stencil", {"wide_index": 1}, False),
+    ("stencil", {"csplit": 4}, False), ("empty", None, False)])
+def test_few_workgroups_for_scattered_columns_only(gb, oracle, kind, plan, few):
+    rng = np.random.default_rng(17)
+    n = 20000 if kind == "random_small" else 70000
+    if kind == "stencil":
+        rp, ri, _ = gb.laplacian(2, 250, 280)
+    elif kind == "far_stencil":
+        rp, ri = _far_stencil(n, 33000)
+    else:
+        deg = rng.integers(0 if kind == "empty" else 2, 1 if kind == "empty" else 30, n)
+        rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+        row = np.repeat(np.arange(n), deg)
+        ri = rng.integers(0, n, row.size)
+        if kind == "half":  # 7 of 10 rows next to the diagonal, the others anywhere
+            near = (row % 10 < 7)
+            ri = np.where(near, np.minimum(row + np.arange(row.size) - rp[row], n - 1), ri)
+        if kind != "unsorted_rows":
+            ri = ri[np.lexsort((ri, row))]
+        ri = ri.astype(np.uint32)
+    rv, x = rng.uniform(-1, 1, ri.size), rng.uniform(-1, 1, n)
+    print("few workgroups", kind, plan, flush=True)
+    M = gb.Matrix(rp, ri, rv, ncols=n, plan=plan)
+    assert (M.kernels()["spmv_lds"] > 0) == few, (M.info(), M.kernels())
+    ref = oracle.spmult(n, n, 1, rp, ri, rv, x)
+    # sums of at most 30 products of magnitude below 1, in any order
+    assert np.max(np.abs(M.spmv(x) - ref)) <= 30 * 30 * 2.3e-16
