@@ -63,6 +63,7 @@ EXPORTED = [
     "gooseberry_device_alloc", "gooseberry_device_free",
     "gooseberry_memcpy_htod", "gooseberry_memcpy_dtoh", "gooseberry_memcpy_dtod",
     "gooseberry_device_synchronize", "gooseberry_device_memory",
+    "gooseberry_device_cache",
     "gooseberry_event_create", "gooseberry_event_destroy",
     "gooseberry_event_record", "gooseberry_event_elapsed_ms",
     "gooseberry_matrix_create", "gooseberry_matrix_create_device",
@@ -209,6 +210,7 @@ def _sig(lib):
         "gooseberry_memcpy_dtod": (i32, [_P, _P, sz]),
         "gooseberry_device_synchronize": (i32, []),
         "gooseberry_device_memory": (i32, [C.POINTER(sz), C.POINTER(sz)]),
+        "gooseberry_device_cache": (i32, [C.POINTER(u64), C.POINTER(u64)]),
         "gooseberry_event_create": (i32, [C.POINTER(_P)]),
         "gooseberry_event_destroy": (i32, [_P]),
         "gooseberry_event_record": (i32, [_P]),
@@ -390,6 +392,14 @@ def device_memory():
     check(lib().gooseberry_device_memory(C.byref(f), C.byref(t)),
           "gooseberry_device_memory")
     return f.value, t.value
+
+
+def device_cache():
+    """Test hook: ((blocks, bytes), (blocks, bytes)) of the freed buffers kept
+    below 4 MiB and from 4 MiB on."""
+    n, b = (C.c_uint64 * 2)(), (C.c_uint64 * 2)()
+    check(lib().gooseberry_device_cache(n, b), "gooseberry_device_cache")
+    return (n[0], b[0]), (n[1], b[1])
 
 
 class Event:

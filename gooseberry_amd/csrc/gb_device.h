@@ -44,6 +44,8 @@ void *gbd_stream(void); /* the library stream as a hipStream_t */
  * check (kind 1) from now on reports a failure, once; after < 0 disarms. */
 int gbd_inject_fault(int kind, long long after);
 int gbd_device_memory(size_t *free_bytes, size_t *total_bytes);
+/* freed blocks that are kept: [0] below 4 MiB, [1] from 4 MiB on */
+void gbd_device_cache(uint64_t blocks[2], uint64_t bytes[2]);
 const char *gbd_last_error(void);
 /* sets the text gbd_last_error returns (host-side refusals) */
 void gbd_set_error(const char *msg);

@@ -149,13 +149,15 @@ uint32_t gb_num_cus() {
 // that a 1,000-row sparse product with its plan took, 155 with these blocks
 // kept and gb_fetch.  Every library launch and copy runs on
 // g_stream, so a block's reuse is ordered after its last use exactly as a
-// pool block's is.  The cache holds at most g_cache_cap bytes and
-// GB_CACHE_BLOCKS blocks (the oldest go back first), is emptied when an
-// allocation finds the device out of memory, and its bytes count as free in
-// gbd_device_memory.
+// pool block's is.  The cache holds at most g_cache_cap bytes of large blocks,
+// and apart from them GB_CACHE_BLOCKS small ones of GB_CACHE_SMALL bytes in all
+// (the oldest of its kind goes back first: many small arrays do not push the
+// large blocks out), is emptied when an allocation finds the device out of
+// memory, and its bytes count as free in gbd_device_memory.
 #define GB_CACHE_LARGE (4ull << 20)
 #define GB_CACHE_ROUND (2ull << 20)
 #define GB_CACHE_BLOCKS 1024
+#define GB_CACHE_SMALL (1ull << 30)
 
 static size_t gb_cache_round(size_t bytes) {
   if (bytes >= GB_CACHE_LARGE) return (bytes + GB_CACHE_ROUND - 1) & ~(GB_CACHE_ROUND - 1);
@@ -166,31 +168,40 @@ static size_t gb_cache_round(size_t bytes) {
 
 static std::mutex g_cache_mu;
 static std::unordered_map<void *, size_t> g_cache_live;  // handed out: size
-static std::list<std::pair<size_t, void *>> g_cache_fifo;  // free, oldest first
-static std::multimap<size_t, std::list<std::pair<size_t, void *>>::iterator> g_cache_free;
-static size_t g_cache_bytes = 0;
+struct gb_cache {
+  std::list<std::pair<size_t, void *>> fifo;  // free blocks, oldest first
+  std::multimap<size_t, std::list<std::pair<size_t, void *>>::iterator> by_size;
+  size_t bytes = 0;
+};
+static gb_cache g_cache[2];  // small blocks, large blocks
 
-static void gb_cache_evict_oldest() {  // g_cache_mu held
-  auto &front = g_cache_fifo.front();
-  auto range = g_cache_free.equal_range(front.first);
+static gb_cache &gb_cache_of(size_t rounded) { return g_cache[rounded >= GB_CACHE_LARGE]; }
+
+static void gb_cache_evict_oldest(gb_cache &c) {  // g_cache_mu held
+  auto &front = c.fifo.front();
+  auto range = c.by_size.equal_range(front.first);
   for (auto it = range.first; it != range.second; ++it)
-    if (it->second == g_cache_fifo.begin()) {
-      g_cache_free.erase(it);
+    if (it->second == c.fifo.begin()) {
+      c.by_size.erase(it);
       break;
     }
-  g_cache_bytes -= front.first;
+  c.bytes -= front.first;
   (void)hipFreeAsync(front.second, g_stream);
-  g_cache_fifo.pop_front();
+  c.fifo.pop_front();
 }
 
 static void gb_cache_trim() {
   std::lock_guard<std::mutex> lk(g_cache_mu);
-  while (!g_cache_fifo.empty()) gb_cache_evict_oldest();
+  for (gb_cache &c : g_cache)
+    while (!c.fifo.empty()) gb_cache_evict_oldest(c);
 }
 
-size_t gb_cache_cached_bytes() {
+void gbd_device_cache(uint64_t *blocks, uint64_t *bytes) {
   std::lock_guard<std::mutex> lk(g_cache_mu);
-  return g_cache_bytes;
+  for (int i = 0; i < 2; ++i) {
+    blocks[i] = g_cache[i].fifo.size();
+    bytes[i] = g_cache[i].bytes;
+  }
 }
 
 // Injected faults (gbd_inject_fault, a test hook): with a countdown c >= 0
@@ -226,13 +237,14 @@ hipError_t gb_dev_alloc(void **p, size_t bytes) {
     std::lock_guard<std::mutex> lk(g_cache_mu);
     // the block of this size freed last (its lines are the likeliest to
     // be in the caches still)
-    auto range = g_cache_free.equal_range(r);
+    gb_cache &c = gb_cache_of(r);
+    auto range = c.by_size.equal_range(r);
     if (range.first != range.second) {
       auto it = std::prev(range.second);
       *p = it->second->second;
-      g_cache_fifo.erase(it->second);
-      g_cache_free.erase(it);
-      g_cache_bytes -= r;
+      c.fifo.erase(it->second);
+      c.by_size.erase(it);
+      c.bytes -= r;
       g_cache_live[*p] = r;
       return hipSuccess;
     }
@@ -258,12 +270,15 @@ hipError_t gb_dev_free(void *p) {
     if (it != g_cache_live.end()) {
       const size_t r = it->second;
       g_cache_live.erase(it);
-      if (r <= g_cache_cap) {
-        while (g_cache_bytes + r > g_cache_cap || g_cache_fifo.size() >= GB_CACHE_BLOCKS)
-          gb_cache_evict_oldest();
-        g_cache_fifo.emplace_back(r, p);
-        g_cache_free.emplace(r, std::prev(g_cache_fifo.end()));
-        g_cache_bytes += r;
+      const bool large = r >= GB_CACHE_LARGE;
+      gb_cache &c = g_cache[large];
+      const size_t cap = !large && GB_CACHE_SMALL < g_cache_cap ? GB_CACHE_SMALL : g_cache_cap;
+      if (r <= cap) {
+        while (c.bytes + r > cap || (!large && c.fifo.size() >= GB_CACHE_BLOCKS))
+          gb_cache_evict_oldest(c);
+        c.fifo.emplace_back(r, p);
+        c.by_size.emplace(r, std::prev(c.fifo.end()));
+        c.bytes += r;
         return hipSuccess;
       }
     }
@@ -738,7 +753,9 @@ int gbd_device_memory(size_t *free_bytes, size_t *total_bytes) {
   if (rv != GOOSEBERRY_SUCCESS) return rv;
   size_t f = 0, t = 0;
   GB_HIP(hipMemGetInfo(&f, &t));
-  f += gb_cache_cached_bytes();  // cached blocks are given back on demand
+  uint64_t blocks[2], bytes[2];
+  gbd_device_cache(blocks, bytes);
+  f += bytes[0] + bytes[1];  // cached blocks are given back on demand
   if (f > t) f = t;
   if (free_bytes) *free_bytes = f;
   if (total_bytes) *total_bytes = t;

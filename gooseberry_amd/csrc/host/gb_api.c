@@ -114,6 +114,14 @@ int gooseberry_device_memory(size_t *free_bytes, size_t *total_bytes)
   return gbd_device_memory(free_bytes, total_bytes);
 }
 
+int gooseberry_device_cache(uint64_t *blocks, uint64_t *bytes)
+{
+  GB_API_GUARD();
+  if (!blocks || !bytes) return GOOSEBERRY_ERROR_INVALIDINPUT;
+  gbd_device_cache(blocks, bytes);
+  return GOOSEBERRY_SUCCESS;
+}
+
 int gooseberry_event_create(void **ev)
 {
   GB_API_GUARD();

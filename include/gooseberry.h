@@ -387,6 +387,10 @@ int gooseberry_memcpy_dtoh(void * h_dst, const void * d_src, size_t bytes);
 int gooseberry_memcpy_dtod(void * d_dst, const void * d_src, size_t bytes);
 int gooseberry_device_synchronize(void);
 int gooseberry_device_memory(size_t * free_bytes, size_t * total_bytes);
+/* freed buffers that the library keeps for later allocations, a test hook with
+ * no counterpart in the reference: two numbers each, of buffers below 4 MiB and
+ * of larger ones */
+int gooseberry_device_cache(uint64_t * blocks, uint64_t * bytes);
 /* timing events on the library stream */
 int gooseberry_event_create(void ** ev);
 int gooseberry_event_destroy(void * ev);

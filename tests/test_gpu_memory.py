@@ -76,3 +76,26 @@ def test_many_small_blocks_are_given_back(gb):
     assert all(np.array_equal(y.numpy(), np.full(8, -float(i))) for i, y in enumerate(ys))
     for y in ys:
         y.free()
+
+
+def test_kept_blocks_by_kind(gb):
+    # many small arrays neither push the large blocks out nor pass their own
+    # limits (1024 blocks, 1 GiB); a fuller device takes everything back
+    mib = 1 << 20
+    big = [gb.DeviceArray((40 + 2 * i) * mib, np.uint8) for i in range(5)]
+    for x in big:
+        x.free()
+    large = gb.device_cache()[1]
+    assert large[0] >= 5 and large[1] >= sum((40 + 2 * i) * mib for i in range(5))
+    xs = [gb.DeviceArray(100 + i, np.uint8) for i in range(1500)]
+    for x in xs:
+        x.free()
+    (n, size), after = gb.device_cache()
+    assert n == 1024 and size <= 1024 * 2048 and after == large
+    # blocks of 3.5 MiB: 292 fill 1 GiB
+    xs = [gb.DeviceArray(3 * mib + mib // 2, np.uint8) for _ in range(400)]
+    kept = gb.device_cache()[1]
+    for x in xs:
+        x.free()
+    (n, size), after = gb.device_cache()
+    assert size <= 1 << 30 and n <= 1024 and size > (1 << 30) - 4 * mib and after == kept
