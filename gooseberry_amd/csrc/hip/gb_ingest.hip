@@ -24,7 +24,7 @@
 //      column without a value); the reference's loop then makes just these
 //      entries of the line.
 //   4. If any token failed (or the text holds too many for 32-bit row
-//      pointers), the lines are gone through by the reference's loop, one
+//      pointers, or a line of over 8 GiB), the lines are gone through by the reference's loop, one
 //      line per lane: a count pass (entries per row and the column range),
 //      row pointers, a fill pass.
 //   5. A value whose rounding needs more than 19 digits' worth of precision
@@ -316,11 +316,16 @@ gb_in_lines(const char *__restrict__ txt, uint64_t len, const uint64_t *__restri
   }
 }
 
-// plain text: entries per row = half its tokens, and their total
+// plain text: entries per row = half its tokens, and their total.  Token
+// numbers count modulo 2^32, which tells the tokens of a line of up to
+// GB_IN_LINE_MAX bytes apart.  With ls, lines longer than `most` bytes raise
+// the total beyond what the plain pass takes.
+#define GB_IN_LINE_MAX ((1ull << 33) - 2)
 __global__ void __launch_bounds__(GB_BLOCK)
 gb_in_rowcnt(const uint32_t *__restrict__ lt, uint32_t nlines,
              const uint32_t *__restrict__ rowof, uint32_t *__restrict__ cnt,
-             unsigned long long *__restrict__ total) {
+             unsigned long long *__restrict__ total, const uint64_t *__restrict__ ls, uint32_t nl,
+             uint64_t len, uint64_t most) {
   __shared__ unsigned long long lds[GB_WAVES_PER_BLOCK];
   unsigned long long v = 0;
   for (uint32_t k = blockIdx.x * GB_BLOCK + threadIdx.x; k < nlines;
@@ -330,9 +335,18 @@ gb_in_rowcnt(const uint32_t *__restrict__ lt, uint32_t nlines,
     const uint32_t n = (lt[k + 1] - lt[k]) / 2;
     cnt[r] = n;
     v += n;
+    if (ls && (k < nl ? ls[k + 1] : len) - ls[k] > most) v += 1ull << 32;
   }
   v = gb_block_sum(v, lds);
   if (threadIdx.x == 0) atomicAdd(total, v);
+}
+
+// the longest line whose tokens the plain pass can number;
+// GOOSEBERRY_INGEST_LINE_MAX: the tests' way to the lines' passes
+static uint64_t gb_in_line_max() {
+  const char *e = getenv("GOOSEBERRY_INGEST_LINE_MAX");
+  const uint64_t v = e && *e ? strtoull(e, nullptr, 10) : GB_IN_LINE_MAX;
+  return v < GB_IN_LINE_MAX ? v : GB_IN_LINE_MAX;
 }
 
 // An entry in the usual form, "column value" with blanks between, at most 9
@@ -826,8 +840,9 @@ int gbd_parse_csr(const char *d_txt, uint64_t len, uint32_t *r_nrows, uint32_t *
     GB_IN_TRY(hipGetLastError());
     if (nlines && !general) {
       const uint32_t g = gb_in_grid(nlines);
-      gb_in_rowcnt<<<g > 512u ? 512u : g, GB_BLOCK, 0, s>>>(lt, nlines, rowof, cnt,
-                                                            &meta->total);
+      const uint64_t most = gb_in_line_max();
+      gb_in_rowcnt<<<g > 512u ? 512u : g, GB_BLOCK, 0, s>>>(
+          lt, nlines, rowof, cnt, &meta->total, len > most ? ls : nullptr, nl, len, most);
       GB_IN_TRY(hipGetLastError());
     } else if (nlines) {
       auto *k = gb_in_wide(len, nlines) ? gb_in_lines<false, 16384> : gb_in_lines<false, 8192>;

@@ -292,3 +292,14 @@ def test_matrixmarket_files(gb, oracle, tmp_path):
     # a resident matrix from a MatrixMarket file
     M = gb.Matrix.read(os.path.join(str(tmp_path), "sym.mtx"), gb.FORMAT_MATRIXMARKET)
     assert (M.nrows, M.ncols, M.nnz) == (600, 600, int(ref[2][-1]))
+
+
+@pytest.mark.parametrize("most", [0, 11, 12, 100, 10 ** 12])
+def test_lines_too_long_for_the_plain_pass(gb, oracle, tmp_path, monkeypatch, most):
+    # tokens are numbered in 32 bits, so a text with a longer line (over 8 GiB;
+    # here `most` bytes) is gone through line by line; the newline counts
+    monkeypatch.setenv("GOOSEBERRY_INGEST_LINE_MAX", str(most))
+    rng = np.random.default_rng(3)
+    for tail in (b"", b"\n", b"\n5 1 6 2 7 33"):
+        lines = [b"1 2.5 3 4.5", b"", b"# 1 2 3 4 5 6 7 8 9"] + [line_of(n, rng) for n in (12, 60)]
+        check_text(gb, oracle, tmp_path, b"\n".join(lines * 30) + tail)
