@@ -363,11 +363,19 @@ static int gb_countingsort(const uint32_t *d_keys, const uint32_t *d_vals,
   const size_t ncounts = (size_t)CS_RADIX * ntiles;
   uint32_t *counts = nullptr, *tk[2] = {nullptr, nullptr},
            *tv[2] = {nullptr, nullptr};
-  GB_HIP(gb_dev_alloc((void **)&counts, ncounts * sizeof(uint32_t)));
-  GB_HIP(gb_dev_alloc((void **)&tk[0], n * sizeof(uint32_t)));
-  GB_HIP(gb_dev_alloc((void **)&tk[1], n * sizeof(uint32_t)));
-  GB_HIP(gb_dev_alloc((void **)&tv[0], n * sizeof(uint32_t)));
-  if (npass > 1) GB_HIP(gb_dev_alloc((void **)&tv[1], n * sizeof(uint32_t)));
+  hipError_t e = gb_dev_alloc((void **)&counts, ncounts * sizeof(uint32_t));
+  if (e == hipSuccess) e = gb_dev_alloc((void **)&tk[0], n * sizeof(uint32_t));
+  if (e == hipSuccess) e = gb_dev_alloc((void **)&tk[1], n * sizeof(uint32_t));
+  if (e == hipSuccess) e = gb_dev_alloc((void **)&tv[0], n * sizeof(uint32_t));
+  if (e == hipSuccess && npass > 1) e = gb_dev_alloc((void **)&tv[1], n * sizeof(uint32_t));
+  if (e != hipSuccess) {
+    // a caller that can do without the sort goes on with the memory back
+    (void)gb_dev_free(counts);
+    (void)gb_dev_free(tk[0]);
+    (void)gb_dev_free(tk[1]);
+    (void)gb_dev_free(tv[0]);
+    return gb_hip_fail(e, "gb_countingsort", __FILE__, __LINE__);
+  }
   const uint32_t *ck = d_keys, *cv = d_vals;
   for (int p = 0; p < npass; ++p) {
     const int shift = 8 * p;

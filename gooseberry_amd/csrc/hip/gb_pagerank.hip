@@ -420,6 +420,15 @@ static uint32_t gb_pr_grid(uint64_t n) {
   return g ? (uint32_t)g : 1u;
 }
 
+// the entries' positions in column order, and where each column starts
+static int gb_pr_sort(const uint32_t *rowind, uint32_t n, uint64_t nnz, uint32_t **perm,
+                      uint32_t **dist) {
+  hipError_t e = gb_dev_alloc((void **)perm, (size_t)(nnz ? nnz : 1) * 4);
+  if (e == hipSuccess) e = gb_dev_alloc((void **)dist, ((size_t)n + 1) * 4);
+  if (e != hipSuccess) return gb_hip_fail(e, "gb_pr_sort", __FILE__, __LINE__);
+  return gbd_countingsort_kv_unchecked(rowind, nullptr, 0, n - 1, nnz, *perm, *dist);
+}
+
 extern "C" {
 
 int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
@@ -458,11 +467,13 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
   // it has the column tiles to fill the GPU with a workgroup each;
   // GOOSEBERRY_PAGERANK_SORTED_SUMS set to "0" takes the layout wherever its
   // tiles fit, set to anything else the sort (the same bits: a check of one
-  // path against the other).
+  // path against the other).  Where memory lacks for the sort, the walk needs
+  // none.
   const char *sorted_env = getenv("GOOSEBERRY_PAGERANK_SORTED_SUMS");
-  bool tile_sums = m->xt.ptr && nnz && (1u << m->xt.lc) <= GB_XT_CMAX;
-  if (sorted_env && *sorted_env) tile_sums = tile_sums && strcmp(sorted_env, "0") == 0;
-  else tile_sums = tile_sums && m->xt.T >= GB_PRX_TILES;
+  const bool walks = m->xt.ptr && nnz && (1u << m->xt.lc) <= GB_XT_CMAX;
+  bool tile_sums = walks;
+  if (sorted_env && *sorted_env) tile_sums = walks && strcmp(sorted_env, "0") == 0;
+  else tile_sums = walks && m->xt.T >= GB_PRX_TILES;
 #define GB_PR_TRY(call)                                         \
   do {                                                          \
     he = (call);                                                \
@@ -479,10 +490,6 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
 
   GB_PR_TRY(gb_dev_alloc((void **)&indeg, (size_t)n * 8));
   if (!own_copy) GB_PR_TRY(gb_dev_alloc((void **)&nval, (size_t)(nnz ? nnz : 1) * 8));
-  if (!tile_sums) {
-    GB_PR_TRY(gb_dev_alloc((void **)&perm, (size_t)(nnz ? nnz : 1) * 4));
-    GB_PR_TRY(gb_dev_alloc((void **)&dist, ((size_t)n + 1) * 4));
-  }
   GB_PR_TRY(gb_dev_alloc((void **)&flag, (size_t)n * 4));
   GB_PR_TRY(gb_dev_alloc((void **)&idx, ((size_t)n + 1) * 4));
   GB_PR_TRY(gb_dev_alloc((void **)&sinks, (size_t)n * 4));
@@ -492,6 +499,17 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
   GB_PR_TRY(gb_dev_alloc((void **)&part, GB_PR_ERR_GRID * 8));
   GB_PR_TRY(gb_dev_alloc((void **)&err, 8));
 
+  if (!tile_sums) {
+    rv = gb_pr_sort(m->rowind, n, nnz, &perm, &dist);
+    if (rv == GOOSEBERRY_ERROR_NOMEMORY && walks) {
+      (void)gb_dev_free(perm);
+      (void)gb_dev_free(dist);
+      perm = dist = nullptr;
+      tile_sums = true;
+    } else if (rv != GOOSEBERRY_SUCCESS) {
+      goto done;
+    }
+  }
   if (tile_sums) {
     // column sums and the layout's quotients, one workgroup per column tile
     GB_PR_TRY(gb_dev_alloc((void **)&snval, ((size_t)nnz + GB_XT_PAD) * 8));
@@ -501,7 +519,6 @@ int gbd_pagerank(const gbd_matrix *m, double damping, uint64_t niter,
     GB_PR_TRY(hipGetLastError());
   } else {
     // column sums in row order (column indices were validated with the matrix)
-    GB_PR_RV(gbd_countingsort_kv_unchecked(m->rowind, nullptr, 0, n - 1, nnz, perm, dist));
     gb_pr_colsum<<<gb_div_up(n, GB_BLOCK), GB_BLOCK, 0, s>>>(n, dist, perm, m->val, indeg);
     GB_PR_TRY(hipGetLastError());
     gb_pr_colsum_long<<<gb_div_up(n, GB_WAVES_PER_BLOCK), GB_BLOCK, 0, s>>>(n, dist, perm,

@@ -263,3 +263,27 @@ def test_pagerank_sums_by_number_of_tiles(gb, n, xtile, monkeypatch):
         x, it, err, ns = M.pagerank(0.85, 8, 0.0)
         got.append((x.tobytes(), it, err, ns))
     assert got[0] == got[1] == got[2]
+
+
+def test_pagerank_without_memory_for_the_sort(gb):
+    # on an x-tile plan the column sums need no sort: where an allocation of it
+    # fails, the walk over the layout takes its place (the same bits); any other
+    # failing allocation is reported, and the library stays usable
+    rp, ri, rv = _hub_graph(20000, 11)
+    M = gb.Matrix(rp, ri, rv, plan={"xtile": 4096})  # 5 tiles: sorted sums
+    want = M.pagerank(0.85, 8, 0.0)
+    done = []
+    for after in range(60):
+        gb.inject_fault(gb.FAULT_ALLOC, after)
+        try:
+            x, it, err, ns = M.pagerank(0.85, 8, 0.0)
+            assert np.array_equal(x, want[0]) and (it, err, ns) == want[1:]
+            done.append(True)
+        except gb.GooseberryError as e:
+            assert e.name == "NOMEMORY"
+            done.append(False)
+        finally:
+            gb.inject_fault(gb.FAULT_ALLOC, -1)
+    last = max(i for i, ok in enumerate(done) if not ok)
+    assert sum(done[:last]) >= 3, done  # the permutation, the starts, the sort's own
+    assert np.array_equal(M.pagerank(0.85, 8, 0.0)[0], want[0])
