@@ -133,7 +133,7 @@ struct gbd_batch {
 
 __device__ __forceinline__ double gb_b_sum_chunks(const double *part, uint32_t n,
                                                   double *red) {
-  // same code and order in every workgroup of K4 and in the init reduction
+  // same code and order in every workgroup of K2 and K3 and in the init reduction
   double s = 0.0;
 #pragma unroll 1
   for (uint32_t base = 0; base < n; base += GB_BLOCK * 4) {

@@ -995,7 +995,7 @@ int gbd_cg_poll(gbd_cg *cg, gbd_cg_state *st, double *h_trace) {
                           hipMemcpyDeviceToHost, s));
   GB_HIP(hipStreamSynchronize(s));
   *st = *cg->h_st;
-  // the last K4 of a stopped solve records its status before any K2 has
+  // the last K3 of a stopped solve records its status before any K2 has
   // turned it into `done`
   if (st->status) st->done = 1;
   if (h_trace && cg->trace_cap)

@@ -94,19 +94,24 @@ def band_spd(n, half, seed):
 def solve_both(gb, monkeypatch, rp, ri, rv, b, tol, niter=0):
     """One launch for the run of iterations, and (its waits given up at once)
     one launch per step."""
-    x1, i1 = gb.Matrix(rp, ri, rv).cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
+    N = gb.Matrix(rp, ri, rv)
+    x1, i1 = N.cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
+    workgroups = N.kernels()["cg_workgroups"]
     monkeypatch.setenv("GOOSEBERRY_CG_SPINS", "0")
     M = gb.Matrix(rp, ri, rv)
     x2, i2 = M.cgd(b, tol, gb.TOL_RELATIVE, niter=niter)
     x3, i3 = M.cgd(b, tol, gb.TOL_RELATIVE, niter=niter)  # stays with that
     monkeypatch.delenv("GOOSEBERRY_CG_SPINS")
     assert i3.niter == i2.niter and np.array_equal(x2, x3)
+    # (a workgroup alone waits for nobody)
+    assert M.kernels()["cg_workgroups"] == (1 if workgroups == 1 else 0)
     return (x1, i1), (x2, i2)
 
 
 # rows around the sizes of the one-launch solve: one workgroup (512 rows), 64
-# workgroups of 512 to 2048 rows, 128 and 256 workgroups, and past them; and
-# the entries its LDS holds (rows of about 3, 28 and 60 entries)
+# workgroups of 512 to 2048 rows, 128 and 256 workgroups, and past them; and, on
+# both sides with several launches, rows of over 64 entries and more entries than
+# LDS holds (SHAPES below says which is which)
 @pytest.mark.parametrize("n,half", [
     (1, 0), (2, 1), (64, 3), (511, 2), (512, 2), (513, 2), (1025, 40), (5000, 44), (32768, 2),
     (32769, 2), (40000, 20), (65600, 2), (131072, 2), (131073, 2), (262145, 2), (524289, 2)])
