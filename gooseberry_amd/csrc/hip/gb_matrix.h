@@ -58,7 +58,7 @@ struct gbd_matrix {
   // x tiles (params.xtile = C): xt is what FP64 products read.  FP32 products
   // and the FP64 residuals of mixed solves read xt32, made with the FP32
   // values: tiles of C columns and blocks of equal rows always (its arrays
-  // are xt's own where that has them too).  See gb_xtile_build.
+  // are xt's own where that has them too).  See gb_xtile_layout.
   gb_xt xt, xt32;
   float *xt_val32;      // nnz, with val32: its values in xt32's order
   float *xt_val32j;     // nnz, with val32j: its values in xt32's order

@@ -432,7 +432,8 @@ typedef struct gooseberry_plan_t {
                        tile's products at a time (matrices with scattered
                        columns; a row's sum is regrouped by tile, as with a
                        column split, and the layout costs 12 bytes an entry
-                       more); 0: off.  Not with csplit or exact. */
+                       more, and 12 again for FP32 products and mixed
+                       solves); 0: off.  Not with csplit or exact. */
 } gooseberry_plan_t;
 
 /* Upload a host CSR matrix to HBM and build its SpMV plan on the GPU. */
