@@ -354,3 +354,26 @@ def test_xtile_mixed_solves_beside_fp64(gb, jacobi):
     assert np.array_equal(x, x2) and info2.niter == info.niter
     assert np.array_equal(xf, xf2) and np.array_equal(B.spmv(b), y)
     assert np.array_equal(A.spmv(b), y)
+
+
+# 256 blocks of 8192 rows are full: no block can take a row more, the FP64
+# layout is the one of equal rows, and FP32 reads the same arrays; a row less
+# than 2^21 leaves that, and 512 rows more a layout of mostly equal blocks again
+@pytest.mark.parametrize("n", [1 << 21, (1 << 21) - 1, (1 << 21) + 512])
+def test_xtile_layout_shared_by_both_types(gb, oracle, n):
+    rng = np.random.default_rng(n)
+    print("x tiles, both types", n, flush=True)
+    deg = np.zeros(n, np.int64)
+    deg[::97] = 9
+    deg[5] = 40000
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+    m = 30011
+    ri = rng.integers(0, m, int(rp[-1])).astype(np.uint32)
+    x = rng.integers(0, 8, m).astype(np.float64)
+    want = oracle.spmult(n, m, 1, rp, ri, np.ones(ri.size), x)
+    M = gb.Matrix(rp, ri, np.ones(ri.size), ncols=m, plan={"xtile": 8192})
+    for plan in ({"xtile": 4096}, None):  # integers below 2^24: exact in any order
+        assert np.array_equal(M.spmv(x), want)
+        assert np.array_equal(M.spmv_f32(x).astype(np.float64), want)
+        assert np.array_equal(M.spmv(x), want)
+        M.replan(plan)
